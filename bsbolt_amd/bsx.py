@@ -41,9 +41,9 @@ EXPORTS = ("bsx_create", "bsx_destroy", "bsx_last_error", "bsx_set_stream", "bsx
            "bsx_extend_batch_device_noalloc", "bsx_ksw_global2", "bsx_reg2aln_cigar_device",
            "bsx_set_tuning", "bsx_get_tuning")
 TIMED_SLOTS = 16
-# lanes per task and columns per lane of the plain form's bins (bsx_internal.h kExtShape);
-# one lane per task is the lane-per-task kernel
-EXT_SHAPES = ((4, 4), (1, 32), (1, 48), (1, 64), (16, 6), (16, 8), (32, 6), (32, 8), (64, 8), (64, 16), (64, 32))
+# lanes per task and columns per lane of the plain form's query-length bins (bsx_internal.h
+# kExtShape); one lane per task is the two-tasks-per-lane kernel
+EXT_SHAPES = ((1, 32), (1, 64), (1, 96), (16, 8), (32, 6), (32, 8), (64, 8), (64, 16), (64, 32))
 
 # learned-band form (include/bsx.h)
 BAND_PLAIN, BAND_LEARNED, BAND_FIXED = 0, 1, 2

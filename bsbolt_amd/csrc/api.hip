@@ -18,11 +18,7 @@
 
 using namespace bsx;
 
-// counts[kCountSlots], cursor[kCountSlots], err[4], fetch[kFetchSlots], split[2 * kLaneFrameClasses],
-// bcount[kExtBins * kRowBuckets], bcursor[kExtBins * kRowBuckets],
-// fcount[kLaneFrameClasses * kRowBuckets], fcursor[kLaneFrameClasses * kRowBuckets]
-static constexpr size_t kSmallBytes = 4 * (2 * kCountSlots + 4 + kFetchSlots + 2 * kLaneFrameClasses +
-                                           2 * kExtBins * kRowBuckets + 2 * kLaneFrameClasses * kRowBuckets);
+static constexpr size_t kSmallBytes = 4 * (size_t)kExtCounterWords;
 
 // band model buffer: params, adam_m, adam_v (FP32), then the BF16 operand copies
 static constexpr size_t kAlign = 256;
@@ -352,15 +348,7 @@ static ExtWork ext_work(bsx_ctx* c) {
   wk.bin_of = (uint8_t*)c->ws->bin_of.p;
   wk.desc = (ExtDesc*)c->ws->desc.p;
   wk.rec = (int32_t*)c->ws->rec.p;
-  wk.counts = (uint32_t*)c->ws->small.p;
-  wk.cursor = wk.counts + kCountSlots;
-  wk.err = (int32_t*)(wk.cursor + kCountSlots);
-  wk.fetch = (uint32_t*)(wk.err + 4);
-  wk.split = wk.fetch + kFetchSlots;
-  wk.bcount = wk.split + 2 * kLaneFrameClasses;
-  wk.bcursor = wk.bcount + kExtBins * kRowBuckets;
-  wk.fcount = wk.bcursor + kExtBins * kRowBuckets;
-  wk.fcursor = wk.fcount + kLaneFrameClasses * kRowBuckets;
+  ext_counters(wk, (uint32_t*)c->ws->small.p);
   wk.nbin_of = (uint8_t*)c->ws->nbin_of.p;
   wk.need_plain = (uint8_t*)c->ws->need_plain.p;
   wk.ss = c->ss_on ? &c->ss : nullptr;
@@ -443,7 +431,7 @@ static int extend_queue(bsx_ctx* c, const ExtArgs& a, ExtWork wk, uint8_t* cls) 
   } else if (c->band_policy == BSX_BAND_FIXED) {
     plan = BandPlan{kBandFixed, c->band_class, nullptr, true, false};
   }
-  HIPCHK(c, launch_extend(a, wk, c->num_cu, c->stream, nullptr, &plan), "extension launch");
+  HIPCHK(c, launch_extend(a, wk, c->num_cu, c->stream, &plan), "extension launch");
   HIPCHK(c, hipMemcpyAsync(c->err_host, wk.err, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream),
          "hipMemcpyAsync(err)");
   c->last_n = plan.mode == kBandPlain ? 0 : (int64_t)n;
@@ -491,15 +479,7 @@ int bsx_extend_batch_device_noalloc(bsx_ctx* c, const bsx_scoring* sc, const bsx
   uint8_t* cls = (uint8_t*)b; b += align_up(kNoallocN);
   wk.desc = (ExtDesc*)b; b += align_up(sizeof(ExtDesc) * kNoallocN);
   wk.rec = (int32_t*)b; b += align_up(32 * kNoallocN);
-  wk.counts = (uint32_t*)b;
-  wk.cursor = wk.counts + kCountSlots;
-  wk.err = (int32_t*)(wk.cursor + kCountSlots);
-  wk.fetch = (uint32_t*)(wk.err + 4);
-  wk.split = wk.fetch + kFetchSlots;
-  wk.bcount = wk.split + 2 * kLaneFrameClasses;
-  wk.bcursor = wk.bcount + kExtBins * kRowBuckets;
-  wk.fcount = wk.bcursor + kExtBins * kRowBuckets;
-  wk.fcursor = wk.fcount + kLaneFrameClasses * kRowBuckets;
+  ext_counters(wk, (uint32_t*)b);
   return extend_queue(c, a, wk, cls);
 }
 
@@ -544,9 +524,9 @@ int bsx_kernel_times(bsx_ctx* c, float* ms, int n_slots, int* calls) {
 }
 
 int bsx_ext_bin_limits(int32_t* limits, int n) {
-  if (!limits) return kExtBins;
-  for (int b = 0; b < kExtBins && b < n; ++b) limits[b] = bin_limit(b);
-  return kExtBins;
+  if (!limits) return kQueryBins;
+  for (int b = 0; b < kQueryBins && b < n; ++b) limits[b] = bin_limit(b);
+  return kQueryBins;
 }
 
 int bsx_set_band_policy(bsx_ctx* c, int policy, int band_class) {
@@ -629,7 +609,7 @@ int bsx_band_labels_device(bsx_ctx* c, const bsx_scoring* sc, const bsx_ext_task
   ExtWork wk = ext_work(c);
   for (int cl = kBandClasses - 2; cl >= 0; --cl) {
     BandPlan plan{kBandFixed, cl, nullptr, true, true};
-    HIPCHK(c, launch_extend(a, wk, c->num_cu, c->stream, nullptr, &plan), "narrow launch");
+    HIPCHK(c, launch_extend(a, wk, c->num_cu, c->stream, &plan), "narrow launch");
     HIPCHK(c, launch_band_label_merge(a, wk, cl, labels, cl == kBandClasses - 2, c->num_cu, c->stream), "label merge");
   }
   HIPCHK(c, hipMemcpyAsync(c->err_host, wk.err, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream),

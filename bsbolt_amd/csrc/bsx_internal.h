@@ -6,16 +6,18 @@
 namespace bsx {
 
 // Extension work is split into bins by query length; each bin runs a kernel
-// instantiation with L lanes per task and C query columns per lane
-// (qlen <= L*C).  Index = bin id.  L = 1 is the lane-per-task kernel (one task
-// per lane, its whole query in registers, ~22 VALU instructions per column);
-// L >= 16 are the group kernels, whose row cost per task ~ (fixed + per-column
-// work * C) * L / 64 wave instructions carries a fixed part (prefix scans,
-// group reductions) that the lane kernel does not have.
-constexpr int kExtBins = 11;
+// instantiation.  Index = bin id.  Shape (1, Q) is the two-tasks-per-lane
+// kernel (pair.hip, queries of at most Q bases); shape (L, C) a group kernel
+// with L lanes per task and C query columns per lane (qlen <= L*C).  The last
+// bin takes the queries of the pair bins where the pair kernel does not run
+// them: batches below kPairMinTasks and tasks outside its range (pair_takes).
+constexpr int kExtBins = 10;
+constexpr int kPairBins = 3;
+constexpr int kQueryBins = 9;  // bins told apart by query length alone
+constexpr int kShortBin = 9;
 struct BinShape { int lanes, cols; };
 constexpr BinShape kExtShape[kExtBins] = {
-    {4, 4}, {1, 32}, {1, 48}, {1, 64}, {16, 6}, {16, 8}, {32, 6}, {32, 8}, {64, 8}, {64, 16}, {64, 32}};
+    {1, 32}, {1, 64}, {1, 96}, {16, 8}, {32, 6}, {32, 8}, {64, 8}, {64, 16}, {64, 32}, {16, 6}};
 constexpr int kExtBlock = 64;             // threads per extension block: one wave, so a block
                                           // never holds wave slots idle while a sibling finishes
 constexpr int kExtTasksPerBlock = 32;     // task descriptors owned by one plain-kernel block
@@ -26,7 +28,7 @@ constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; 
 constexpr int kGlbBins = 9;
 constexpr BinShape kGlbShape[kGlbBins] = {
     {8, 2}, {8, 3}, {8, 4}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
-constexpr int kExtSlices = 8;  // fetch-counter slots per bin (CIGAR bins, lane-kernel bins and classes)
+constexpr int kExtSlices = 8;  // fetch-counter slots per bin (CIGAR bins, lane frame classes)
 constexpr int glb_bin_limit(int b) { return kGlbShape[b].lanes * kGlbShape[b].cols; }
 // First entry of fetch slice s of a list of n entries: a balanced partition,
 // the first n % kExtSlices slices hold one entry more.
@@ -36,25 +38,22 @@ __host__ __device__ inline uint32_t slice_begin(uint32_t n, int s) {
 }
 
 // Plain bins list their tasks longest run first, so that a kernel's last
-// tasks are short ones and its waves drain together.  The rows a run takes
-// follow min(tlen, 2*h0) closely (the run ends when the target does, or once
-// the score built on h0 is spent or the z-drop fires); the key is bucketed in
-// kRowBuckets steps of 32 rows, bucket 0 = longest.  Lane-kernel bins place
-// rank r of that order at slot r / kExtSlices of fetch slice r % kExtSlices,
-// so that every slice is itself longest first.  The order changes no result.
-constexpr int kRowBuckets = 8;
+// tasks are short ones and its waves drain together, and so that the tasks of
+// one pair-kernel wave, which start together, also end together.  The rows a
+// run takes follow min(tlen, 2*h0) closely (the run ends when the target does,
+// or once the score built on h0 is spent or the z-drop fires); the key is
+// bucketed in steps of 8 rows up to 192 and of 32 beyond, bucket 0 = longest.
+// Steps of 32 throughout cost the pair kernels a quarter to a third more rows
+// (the waves of a bucket all run as long as its longest run); steps of 4
+// changed nothing.  The lane frame kernel's lists place rank r of that order at
+// slot r / kExtSlices of fetch slice r % kExtSlices, so that every slice is
+// itself longest first.  The order changes no result.
+constexpr int kRowBuckets = 32;
 __host__ __device__ inline int row_bucket(int tlen, int h0) {
   const int est = tlen < 2 * h0 ? tlen : 2 * h0;
-  const int k = est >> 5;
-  return kRowBuckets - 1 - (k < kRowBuckets - 1 ? (k > 0 ? k : 0) : kRowBuckets - 1);
+  const int k = est < 192 ? (est > 0 ? est >> 3 : 0) : 24 + ((est - 192) >> 5);
+  return kRowBuckets - 1 - (k < kRowBuckets - 1 ? k : kRowBuckets - 1);
 }
-constexpr uint32_t lane_bin_mask() {
-  uint32_t m = 0;
-  for (int b = 0; b < kExtBins; ++b)
-    if (kExtShape[b].lanes == 1) m |= 1u << b;
-  return m;
-}
-constexpr uint32_t kLaneBinMask = lane_bin_mask();
 
 // Learned-band form: classes 0..3 run the band-following frame kernel with
 // frames of 24, 40, 80, 144 columns; class 4 is the plain kernel.  Count slots: plain bins
@@ -80,10 +79,23 @@ struct BandPlan {
 
 // Scores are tracked as (h << 11 | column) keys in 32-bit lanes.
 constexpr int kScoreLimit = 1 << 20;
+// Largest score of a run of the two-tasks-per-lane kernel: (h << 7 | position)
+// keys and the per-column F caps fill 16 bits.
+constexpr int kPairScoreMax = 511;
+constexpr int kPairMaxTlen = 640;        // cell counts of a run (tlen * 96) fit 16 bits
+constexpr int kPairMaxGapExt = 25;       // gap-extension cost of a z-drop test fits 16 bits
+// Smallest batch whose short queries run the pair kernel.  A lane runs its two
+// tasks serially, so a batch takes at least its longest run (0.4 ms for 100 bp
+// reads, 0.8 ms for 150 bp); below this the group kernels, which spread a task
+// over 16 lanes, finish sooner.  us per call, pair / group kernels: 100 bp
+// 32,000 tasks 429 / 276, 64,000 451 / 431, 128,000 529 / 763; 150 bp 32,000
+// 810 / 555, 64,000 874 / 968, 128,000 1406 / 1869.
+constexpr int64_t kPairMinTasks = 65536;
 
 // Kernel-side view of an extension batch (all pointers are device memory).
 struct ExtArgs {
   int o_del, e_del, o_ins, e_ins, zdrop, mat_max;
+  bool pair;  // the batch's short queries may run the pair kernel
   // Query profile by query code qc (0..4): bytes k=0..3 of prof_lo[qc] hold
   // mat[k*5+qc] (target code k), prof_hi[qc] holds mat[20+qc] (target N).
   uint32_t prof_lo[5];
@@ -120,7 +132,7 @@ struct StreamSet {
   hipEvent_t fork = nullptr, join[kSide] = {};
 };
 // launches of the plain bins: stream 0 = the call's stream, k > 0 = side[k-1]
-constexpr int kBinStream[11] = {2, 1, 3, 1, 0, 2, 3, 0, 0, 0, 0};
+constexpr int kBinStream[kExtBins] = {1, 2, 0, 3, 1, 2, 3, 3, 3, 1};
 inline hipStream_t pick_stream(const StreamSet* ss, hipStream_t main, int k) {
   return (ss && k > 0 && ss->side[k - 1]) ? ss->side[k - 1] : main;
 }
@@ -164,18 +176,37 @@ struct ExtWork {
   int tpb_plain = kExtTasksPerBlock, tpb_narrow = kNarrowTasksPerBlock;
   int shape_var[2] = {0, 0};
 };
+// The counters of a workspace lie in one array: counts, cursor, err[4], fetch,
+// split, bcount, bcursor, fcount, fcursor.
+constexpr int kExtCounterWords = 2 * kCountSlots + 4 + kFetchSlots + 2 * kLaneFrameClasses +
+                                 2 * kExtBins * kRowBuckets + 2 * kLaneFrameClasses * kRowBuckets;
+inline void ext_counters(ExtWork& wk, uint32_t* p) {
+  wk.counts = p;
+  wk.cursor = wk.counts + kCountSlots;
+  wk.err = (int32_t*)(wk.cursor + kCountSlots);
+  wk.fetch = (uint32_t*)(wk.err + 4);
+  wk.split = wk.fetch + kFetchSlots;
+  wk.bcount = wk.split + 2 * kLaneFrameClasses;
+  wk.bcursor = wk.bcount + kExtBins * kRowBuckets;
+  wk.fcount = wk.bcursor + kExtBins * kRowBuckets;
+  wk.fcursor = wk.fcount + kLaneFrameClasses * kRowBuckets;
+}
 // Bins with alternative group shapes (same columns per task, so the binning is
-// unchanged; the tuner picks one per device): index 0 = bin 4 (queries of
-// 65-96 bases), 1 = bin 5 (97-128).  Variant 0 is kExtShape's shape.
-constexpr int kTunedBin0 = 4;
+// unchanged; the tuner picks one per device): index 0 = the short bin (queries
+// of at most 96 bases), 1 = queries of 97-128.  Variant 0 is kExtShape's shape.
+constexpr int kTunedBin[2] = {kShortBin, kPairBins};
 constexpr BinShape kAltShape[2][2] = {{{16, 6}, {32, 3}}, {{16, 8}, {32, 4}}};
-static_assert(kExtShape[kTunedBin0].lanes == kAltShape[0][0].lanes &&
-              kExtShape[kTunedBin0].cols == kAltShape[0][0].cols &&
-              kExtShape[kTunedBin0 + 1].lanes == kAltShape[1][0].lanes &&
-              kExtShape[kTunedBin0 + 1].cols == kAltShape[1][0].cols &&
-              kAltShape[0][1].lanes * kAltShape[0][1].cols == bin_limit(kTunedBin0) &&
-              kAltShape[1][1].lanes * kAltShape[1][1].cols == bin_limit(kTunedBin0 + 1), "alternative shapes");
-constexpr int kTimedSlots = 16;  // kExtBins + 4 narrow classes + predictor
+static_assert(kExtShape[kTunedBin[0]].lanes == kAltShape[0][0].lanes &&
+              kExtShape[kTunedBin[0]].cols == kAltShape[0][0].cols &&
+              kExtShape[kTunedBin[1]].lanes == kAltShape[1][0].lanes &&
+              kExtShape[kTunedBin[1]].cols == kAltShape[1][0].cols &&
+              kAltShape[0][1].lanes * kAltShape[0][1].cols == bin_limit(kTunedBin[0]) &&
+              kAltShape[1][1].lanes * kAltShape[1][1].cols == bin_limit(kTunedBin[1]), "alternative shapes");
+// timing slots: the query-length bins, the narrow classes, the short bin, and
+// the predictor last
+constexpr int kTimedSlots = 16;
+constexpr int time_slot_bin(int b) { return b == kShortBin ? kQueryBins + kBandClasses - 1 : b; }
+constexpr int time_slot_class(int c) { return kQueryBins + c; }
 static_assert(kExtBins + kBandClasses <= kTimedSlots, "timing slots");
 inline void time_begin(const ExtWork& wk, int slot, hipStream_t st) {
   if (wk.tev) (void)hipEventRecord(wk.tev[2 * slot], st);
@@ -188,15 +219,13 @@ inline void time_end(const ExtWork& wk, int slot, hipStream_t st) {
 }
 
 struct ExtKArgs;
-// lane-per-task kernel of bin `bin` (query width Q); grid = resident waves, or
-// fewer when the host knows the bin's task count (hint >= 0)
-template <int Q, bool E1>
-void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int num_cu, hipStream_t st, int64_t hint);
+// two-tasks-per-lane kernel of bin `bin` (query width Q), n tasks in the batch
+template <int Q>
+void launch_pair_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, hipStream_t st);
 // lane-per-task frame kernel (frame of WF columns) of lane-frame class `cls`
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st);
-hipError_t launch_extend(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st,
-                         const int64_t* host_bin_counts, const BandPlan* plan);
+hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan);
 hipError_t launch_narrow(const ExtArgs& a, const ExtKArgs& k, const ExtWork& wk, int num_cu, hipStream_t st,
                          const BandPlan& plan);
 

@@ -72,6 +72,7 @@ struct ExtKArgs {
   uint32_t trow_lo[5];  // by target code t: bytes q = 0..3 hold mat[t*5+q]
   uint32_t trow_hi[5];  // by target code t: byte 0 holds mat[t*5+4]
   int tpb;              // task descriptors owned by one block
+  int mat_max;          // largest substitution score, at least 0
 };
 
 // The eight result words of a task (ksw.c:473-478 plus the cell count), one

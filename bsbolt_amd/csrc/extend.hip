@@ -35,6 +35,8 @@
 // without a memory round trip.  Groups run a flattened loop (start-task-or-row
 // per iteration) so the groups of a wave never wait for one another between
 // tasks.
+#include <algorithm>
+
 #include "bsx_internal.h"
 #include "ext_common.h"
 
@@ -338,9 +340,19 @@ ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_
 
 __device__ __forceinline__ int ext_bin_of(int qlen) {
 #pragma unroll
-  for (int b = 0; b < kExtBins; ++b)
+  for (int b = 0; b < kQueryBins; ++b)
     if (qlen <= bin_limit(b)) return b;
   return -1;
+}
+
+// Whether the pair kernel computes this task: every score of the run, its cell
+// count and its z-drop test fit 16 bits, and its first row reaches no column
+// past the band (a band of qlen or more holds every column; else the
+// first-row value at column w+1, h0 - oe_ins - w*e_ins, must not be positive).
+__device__ __forceinline__ bool pair_takes(const ExtArgs& A, int64_t t, int qlen, int tlen, int h0) {
+  if (!A.pair || tlen > kPairMaxTlen || h0 + qlen * A.mat_max > kPairScoreMax) return false;
+  const int w = ext_clamped_w(A, t);
+  return w >= qlen || (int64_t)h0 - A.o_ins - A.e_ins - (int64_t)w * A.e_ins <= 0;
 }
 
 // mode 0: validate every task, write bin_of and count per bin and row bucket
@@ -351,7 +363,7 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
   constexpr int NB = kExtBins * kRowBuckets;
   __shared__ uint32_t hist[kExtBins], bhist[NB];
   if (threadIdx.x < kExtBins) hist[threadIdx.x] = 0;
-  if (threadIdx.x < NB) bhist[threadIdx.x] = 0;
+  for (int k = threadIdx.x; k < NB; k += blockDim.x) bhist[k] = 0;
   __syncthreads();
   int bad = 0, first_bad = 0x7fffffff;
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < A.n;
@@ -372,9 +384,12 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
       b = 0xff;
       ++bad;
       first_bad = min(first_bad, (int)t);
-    } else if (mode == 0) {
-      atomicAdd(&hist[b], 1u);
-      atomicAdd(&bhist[b * kRowBuckets + row_bucket(tl, h0)], 1u);
+    } else {
+      if (b < kPairBins && !pair_takes(A, t, ql, tl, h0)) b = kShortBin;
+      if (mode == 0) {
+        atomicAdd(&hist[b], 1u);
+        atomicAdd(&bhist[b * kRowBuckets + row_bucket(tl, h0)], 1u);
+      }
     }
     W.bin_of[t] = (uint8_t)b;
   }
@@ -384,39 +399,40 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
   }
   __syncthreads();
   if (threadIdx.x < kExtBins && hist[threadIdx.x]) atomicAdd(&W.counts[threadIdx.x], hist[threadIdx.x]);
-  if (threadIdx.x < NB && bhist[threadIdx.x]) atomicAdd(&W.bcount[threadIdx.x], bhist[threadIdx.x]);
+  for (int k = threadIdx.x; k < NB; k += blockDim.x)
+    if (bhist[k]) atomicAdd(&W.bcount[k], bhist[k]);
 }
 
 // Each block handles a contiguous range of tasks: it counts them per bin and
 // row bucket in LDS, reserves one range per (bin, bucket) with a single global
 // atomic, and writes the descriptors of its tasks into those ranges.  A task's
 // rank in its bin's longest-first order is its bucket's base plus its place in
-// the bucket; lane-kernel bins spread the ranks over the fetch slices.
+// the bucket.
 __global__ void __launch_bounds__(256)
 ext_bin_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block, const uint8_t* __restrict__ need) {
   constexpr int NB = kExtBins * kRowBuckets;
-  __shared__ uint32_t off[NB], hist[NB], cur[NB], lbase[kExtBins], lsize[kExtBins];
+  __shared__ uint32_t off[NB], hist[NB], cur[NB], lbase[kExtBins];
   const int64_t t0 = (int64_t)blockIdx.x * per_block;
   const int64_t t1 = min(A.n, t0 + per_block);
-  if (threadIdx.x < NB) { hist[threadIdx.x] = 0; cur[threadIdx.x] = 0; }
+  for (int k = threadIdx.x; k < NB; k += blockDim.x) { hist[k] = 0; cur[k] = 0; }
   __syncthreads();
   for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
     const int b = W.bin_of[t];
     if (b != 0xff && (!need || need[t])) atomicAdd(&hist[b * kRowBuckets + row_bucket(A.tlen[t], A.h0[t])], 1u);
   }
   __syncthreads();
-  if (threadIdx.x < NB) {
-    const int b = threadIdx.x / kRowBuckets, k = threadIdx.x % kRowBuckets;
+  for (int x = threadIdx.x; x < NB; x += blockDim.x) {
+    const uint32_t hcount = hist[x];
+    if (!hcount) continue;
+    const int b = x / kRowBuckets, k = x % kRowBuckets;
     uint32_t s = 0;
     for (int j = 0; j < k; ++j) s += W.bcount[b * kRowBuckets + j];
-    const uint32_t hcount = hist[threadIdx.x];
-    off[threadIdx.x] = s + (hcount ? atomicAdd(&W.bcursor[threadIdx.x], hcount) : 0u);
+    off[x] = s + atomicAdd(&W.bcursor[x], hcount);
   }
   if (threadIdx.x < kExtBins) {
     uint32_t s = 0;
     for (int b = 0; b < (int)threadIdx.x; ++b) s += W.counts[b];
     lbase[threadIdx.x] = s;
-    lsize[threadIdx.x] = W.counts[threadIdx.x];
   }
   __syncthreads();
   for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
@@ -424,20 +440,15 @@ ext_bin_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block, const uint8_t* _
     if (b == 0xff || (need && !need[t])) continue;
     const int kb = b * kRowBuckets + row_bucket(A.tlen[t], A.h0[t]);
     const uint32_t r = off[kb] + atomicAdd(&cur[kb], 1u);
-    const uint32_t p = (kLaneBinMask >> b) & 1u ? slice_begin(lsize[b], (int)(r % kExtSlices)) + r / kExtSlices : r;
-    write_desc(A, t, W.desc + lbase[b] + p);
+    write_desc(A, t, W.desc + lbase[b] + r);
   }
 }
 
-static_assert(kExtBins * kRowBuckets <= kFetchSlots && kExtBins * kRowBuckets <= 256, "bucket counters");
-__global__ void ext_reset_kernel(ExtWork W) {
-  const int k = threadIdx.x;
-  if (k < kCountSlots) { W.counts[k] = 0; W.cursor[k] = 0; }
-  if (k < kFetchSlots) W.fetch[k] = 0;
-  if (k < 2 * kLaneFrameClasses) W.split[k] = 0;
-  if (k < kExtBins * kRowBuckets) { W.bcount[k] = 0; W.bcursor[k] = 0; }
-  if (k < kLaneFrameClasses * kRowBuckets) { W.fcount[k] = 0; W.fcursor[k] = 0; }
-  if (k == 0) { W.err[0] = 0; W.err[1] = 0x7fffffff; }
+// clears every counter of the workspace (ExtWork's, `words` dwords from counts on)
+__global__ void __launch_bounds__(256) ext_reset_kernel(ExtWork W, int words) {
+  for (int k = threadIdx.x; k < words; k += blockDim.x) W.counts[k] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) W.err[1] = 0x7fffffff;
 }
 
 // Copies the packed per-task records into the caller's (nullable) arrays.
@@ -458,27 +469,25 @@ ext_unpack_kernel(ExtArgs A, ExtWork W, const int32_t* __restrict__ rec) {
   }
 }
 
-// one block per k.tpb descriptors of bin B; without a host-side count the
-// grid covers the whole batch and surplus blocks exit at once
+// one block per k.tpb descriptors of bin B; the grid covers the whole batch and
+// surplus blocks exit at once (the host does not know the bin's count)
 template <int L, int C, bool E1>
 static void launch_group(const ExtKArgs& k, const ExtWork& wk, int B, int64_t n, hipStream_t st) {
   const int64_t blocks = (n + k.tpb - 1) / k.tpb;
   if (blocks < 1) return;
-  time_begin(wk, B, st);
+  time_begin(wk, time_slot_bin(B), st);
   hipLaunchKernelGGL((ext_plain_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, st, k,
                      (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B);
-  time_end(wk, B, st);
+  time_end(wk, time_slot_bin(B), st);
 }
 
 template <int B, bool E1>
-static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n_all, int num_cu, hipStream_t st,
-                       int64_t hint) {
+static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st, bool pair) {
   constexpr int L = kExtShape[B].lanes, C = kExtShape[B].cols;
-  const int64_t n = hint >= 0 ? hint : n_all;
-  if constexpr (L == 1) {
-    launch_lane_bin<C, E1>(k, wk, B, num_cu, st, hint);
-  } else if constexpr (B == kTunedBin0 || B == kTunedBin0 + 1) {
-    constexpr int V = B - kTunedBin0;
+  if constexpr (B < kPairBins) {
+    if (pair) launch_pair_bin<C>(k, wk, B, n, st);
+  } else if constexpr (B == kTunedBin[0] || B == kTunedBin[1]) {
+    constexpr int V = B == kTunedBin[0] ? 0 : 1;
     if (wk.shape_var[V] == 1)
       launch_group<kAltShape[V][1].lanes, kAltShape[V][1].cols, E1>(k, wk, B, n, st);
     else
@@ -489,22 +498,14 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n_all, int 
 }
 
 template <int B, bool E1>
-static void launch_bins_from(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st,
-                             const int64_t* hc) {
-  launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[B]), hc ? hc[B] : -1);
-  if constexpr (B > 0) launch_bins_from<B - 1, E1>(k, wk, n, num_cu, st, hc);
+static void launch_bins_from(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st, bool pair) {
+  launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[B]), pair);
+  if constexpr (B > 0) launch_bins_from<B - 1, E1>(k, wk, n, num_cu, st, pair);
 }
 
-template <bool E1>
-static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st,
-                        const int64_t* hc) {
-  // longest queries first so the long tasks do not form the tail
-  launch_bins_from<kExtBins - 1, E1>(k, wk, n, num_cu, st, hc);
-}
-
-hipError_t launch_extend(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st,
-                         const int64_t* host_bin_counts, const BandPlan* plan) {
-  hipLaunchKernelGGL(ext_reset_kernel, dim3(1), dim3(kFetchSlots), 0, st, wk);
+hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan) {
+  a.pair = a.n >= kPairMinTasks && a.e_del <= kPairMaxGapExt && a.e_ins <= kPairMaxGapExt;
+  hipLaunchKernelGGL(ext_reset_kernel, dim3(1), dim3(256), 0, st, wk, kExtCounterWords);
   if (a.n <= 0) return hipGetLastError();
   int64_t blocks = (a.n + 255) / 256;  // unpack pass
   if (blocks > (int64_t)num_cu * 16) blocks = (int64_t)num_cu * 16;
@@ -516,6 +517,7 @@ hipError_t launch_extend(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStr
   k.query = a.query; k.target = a.target; k.rec = wk.rec;
   k.o_del = a.o_del; k.e_del = a.e_del; k.o_ins = a.o_ins; k.e_ins = a.e_ins; k.zdrop = a.zdrop;
   k.tpb = wk.tpb_plain;
+  k.mat_max = a.mat_max;
   for (int q = 0; q < 5; ++q) { k.prof_lo[q] = a.prof_lo[q]; k.prof_hi[q] = a.prof_hi[q]; }
   for (int t = 0; t < 5; ++t) {  // the same matrix by target code
     uint32_t lo = 0;
@@ -533,14 +535,14 @@ hipError_t launch_extend(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStr
     hipError_t e = launch_narrow(a, kn, wk, num_cu, st, *plan);
     if (e != hipSuccess || plan->skip_plain) return e;
     hipLaunchKernelGGL(ext_bin_count_kernel, dim3((unsigned)sblocks), dim3(256), 0, st, a, wk, 2);
-    host_bin_counts = nullptr;
   }
   const int64_t per_block = (a.n + sblocks - 1) / sblocks;
   hipLaunchKernelGGL(ext_bin_scatter_kernel, dim3((unsigned)sblocks), dim3(256), 0, st, a, wk, per_block,
                      band ? (const uint8_t*)wk.need_plain : nullptr);
   ss_fork(wk.ss, st);
-  if (a.e_del == 1 && a.e_ins == 1) launch_bins<true>(k, wk, a.n, num_cu, st, host_bin_counts);
-  else launch_bins<false>(k, wk, a.n, num_cu, st, host_bin_counts);
+  // longest queries first so the long tasks do not form the tail
+  if (a.e_del == 1 && a.e_ins == 1) launch_bins_from<kExtBins - 1, true>(k, wk, a.n, num_cu, st, a.pair);
+  else launch_bins_from<kExtBins - 1, false>(k, wk, a.n, num_cu, st, a.pair);
   ss_join(wk.ss, st);
   hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
   return hipGetLastError();

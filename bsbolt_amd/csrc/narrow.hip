@@ -44,9 +44,9 @@ __host__ __device__ constexpr int frame_of_class(int c) { return frame_lanes(c) 
 // and group frames of 80 and 144 columns).  A task goes to its predicted frame
 // class only where that class is at least 20% cheaper per row than the plain
 // bin of its query length.
-constexpr int kPlainRowPs[kExtBins] = {42, 43, 57, 59, 109, 158, 600, 700, 1000, 2000, 4000};
+constexpr int kPlainRowPs[kExtBins] = {43, 59, 109, 158, 600, 700, 1000, 2000, 4000, 109};
 constexpr int kFrameRowPs[kBandClasses - 1] = {29, 75, 152, 239};
-static_assert(kExtBins == 11 && kBandClasses == 5, "row cost tables");
+static_assert(kExtBins == 10 && kBandClasses == 5, "row cost tables");
 __host__ __device__ constexpr bool narrow_pays(int c, int b) {
   return 10 * kFrameRowPs[c] < 8 * kPlainRowPs[b];
 }
@@ -406,6 +406,7 @@ ext_narrow_count_kernel(ExtArgs A, ExtWork W, BandPlan plan) {
   __shared__ uint32_t hist[kBandClasses], front[kLaneFrameClasses], fhist[NF];
   if (threadIdx.x < kBandClasses) hist[threadIdx.x] = 0;
   if (threadIdx.x < kLaneFrameClasses) front[threadIdx.x] = 0;
+  static_assert(NF <= 256, "one thread per counter");
   if (threadIdx.x < NF) fhist[threadIdx.x] = 0;
   __syncthreads();
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < A.n;
@@ -511,12 +512,12 @@ static void launch_narrow_class(const ExtKArgs& k, const ExtWork& wk, int64_t n,
   if (blocks < 1) return;
   // classes on separate streams; a lane-frame class's lane kernel beside its group kernel
   const hipStream_t sg = pick_stream(wk.ss, st, CL == 3 ? 0 : CL + 1);
-  time_begin(wk, kExtBins + CL, sg);
+  time_begin(wk, time_slot_class(CL), sg);
   if constexpr (CL < kLaneFrameClasses) launch_lane_frame<frame_of_class(CL), E1>(k, wk, CL, num_cu, sg);
   hipLaunchKernelGGL((ext_narrow_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, sg, k,
                      (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, (const uint32_t*)wk.split, CL,
                      wk.need_plain);
-  time_end(wk, kExtBins + CL, sg);
+  time_end(wk, time_slot_class(CL), sg);
 }
 
 template <bool E1>
