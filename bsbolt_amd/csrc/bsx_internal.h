@@ -8,16 +8,16 @@ namespace bsx {
 // Extension work is split into bins by query length; each bin runs a kernel
 // instantiation.  Index = bin id.  Shape (1, Q) is the two-tasks-per-lane
 // kernel (pair.hip, queries of at most Q bases); shape (L, C) a group kernel
-// with L lanes per task and C query columns per lane (qlen <= L*C).  The last
-// bin takes the queries of the pair bins where the pair kernel does not run
-// them: batches below kPairMinTasks and tasks outside its range (pair_takes).
-constexpr int kExtBins = 10;
-constexpr int kPairBins = 3;
+// with L lanes per task and C query columns per lane (qlen <= L*C).  The bins
+// from kQueryBins on take the queries of the pair bins where the pair kernel
+// does not run them: batches below kPairMinTasks and tasks outside its range
+// (pair_takes).
+constexpr int kExtBins = 12;
+constexpr int kPairBins = 5;
 constexpr int kQueryBins = 9;  // bins told apart by query length alone
-constexpr int kShortBin = 9;
 struct BinShape { int lanes, cols; };
-constexpr BinShape kExtShape[kExtBins] = {
-    {1, 32}, {1, 64}, {1, 96}, {16, 8}, {32, 6}, {32, 8}, {64, 8}, {64, 16}, {64, 32}, {16, 6}};
+constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}, {1, 224}, {32, 8},
+                                          {64, 8}, {64, 16}, {64, 32}, {16, 6},  {16, 8},  {32, 6}};
 constexpr int kExtBlock = 64;             // threads per extension block: one wave, so a block
                                           // never holds wave slots idle while a sibling finishes
 constexpr int kExtTasksPerBlock = 32;     // task descriptors owned by one plain-kernel block
@@ -79,11 +79,11 @@ struct BandPlan {
 
 // Scores are tracked as (h << 11 | column) keys in 32-bit lanes.
 constexpr int kScoreLimit = 1 << 20;
-// Largest score of a run of the two-tasks-per-lane kernel: (h << 7 | position)
-// keys and the per-column F caps fill 16 bits.
-constexpr int kPairScoreMax = 511;
-constexpr int kPairMaxTlen = 640;        // cell counts of a run (tlen * 96) fit 16 bits
-constexpr int kPairMaxGapExt = 25;       // gap-extension cost of a z-drop test fits 16 bits
+// Largest score of a run of the two-tasks-per-lane kernel of width Q: its
+// (score, position) keys and per-column F caps fill 16 bits.
+constexpr int pair_score_max(int Q) { return Q <= 128 ? 511 : 255; }
+constexpr int kPairMaxTlen = 640;   // with kPairMaxGapExt: the gap cost of a z-drop test,
+constexpr int kPairMaxGapExt = 25;  // e * (tlen + Q), and the z-drop itself fit 15 bits
 // Smallest batch whose short queries run the pair kernel.  A lane runs its two
 // tasks serially, so a batch takes at least its longest run (0.4 ms for 100 bp
 // reads, 0.8 ms for 150 bp); below this the group kernels, which spread a task
@@ -132,7 +132,7 @@ struct StreamSet {
   hipEvent_t fork = nullptr, join[kSide] = {};
 };
 // launches of the plain bins: stream 0 = the call's stream, k > 0 = side[k-1]
-constexpr int kBinStream[kExtBins] = {1, 2, 0, 3, 1, 2, 3, 3, 3, 1};
+constexpr int kBinStream[kExtBins] = {2, 0, 1, 2, 3, 3, 2, 1, 0, 3, 2, 1};
 inline hipStream_t pick_stream(const StreamSet* ss, hipStream_t main, int k) {
   return (ss && k > 0 && ss->side[k - 1]) ? ss->side[k - 1] : main;
 }
@@ -192,9 +192,9 @@ inline void ext_counters(ExtWork& wk, uint32_t* p) {
   wk.fcursor = wk.fcount + kLaneFrameClasses * kRowBuckets;
 }
 // Bins with alternative group shapes (same columns per task, so the binning is
-// unchanged; the tuner picks one per device): index 0 = the short bin (queries
-// of at most 96 bases), 1 = queries of 97-128.  Variant 0 is kExtShape's shape.
-constexpr int kTunedBin[2] = {kShortBin, kPairBins};
+// unchanged; the tuner picks one per device): index 0 = queries of at most 96
+// bases, 1 = queries of 97-128.  Variant 0 is kExtShape's shape.
+constexpr int kTunedBin[2] = {9, 10};
 constexpr BinShape kAltShape[2][2] = {{{16, 6}, {32, 3}}, {{16, 8}, {32, 4}}};
 static_assert(kExtShape[kTunedBin[0]].lanes == kAltShape[0][0].lanes &&
               kExtShape[kTunedBin[0]].cols == kAltShape[0][0].cols &&
@@ -202,17 +202,17 @@ static_assert(kExtShape[kTunedBin[0]].lanes == kAltShape[0][0].lanes &&
               kExtShape[kTunedBin[1]].cols == kAltShape[1][0].cols &&
               kAltShape[0][1].lanes * kAltShape[0][1].cols == bin_limit(kTunedBin[0]) &&
               kAltShape[1][1].lanes * kAltShape[1][1].cols == bin_limit(kTunedBin[1]), "alternative shapes");
-// timing slots: the query-length bins, the narrow classes, the short bin, and
-// the predictor last
+// timing slots: the plain bins (the last one is not timed), the narrow classes,
+// and the predictor last
 constexpr int kTimedSlots = 16;
-constexpr int time_slot_bin(int b) { return b == kShortBin ? kQueryBins + kBandClasses - 1 : b; }
-constexpr int time_slot_class(int c) { return kQueryBins + c; }
-static_assert(kExtBins + kBandClasses <= kTimedSlots, "timing slots");
+constexpr int time_slot_bin(int b) { return b < 11 ? b : -1; }
+constexpr int time_slot_class(int c) { return 11 + c; }
+static_assert(11 + kBandClasses <= kTimedSlots, "timing slots");
 inline void time_begin(const ExtWork& wk, int slot, hipStream_t st) {
-  if (wk.tev) (void)hipEventRecord(wk.tev[2 * slot], st);
+  if (wk.tev && slot >= 0) (void)hipEventRecord(wk.tev[2 * slot], st);
 }
 inline void time_end(const ExtWork& wk, int slot, hipStream_t st) {
-  if (wk.tev) {
+  if (wk.tev && slot >= 0) {
     (void)hipEventRecord(wk.tev[2 * slot + 1], st);
     *wk.tmask |= 1u << slot;
   }

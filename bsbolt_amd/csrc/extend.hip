@@ -36,6 +36,7 @@
 // per iteration) so the groups of a wave never wait for one another between
 // tasks.
 #include <algorithm>
+#include <utility>
 
 #include "bsx_internal.h"
 #include "ext_common.h"
@@ -58,9 +59,13 @@ ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_
   uint32_t lbase = 0;
   for (int b = 0; b < bin; ++b) lbase += counts[b];
   const uint32_t nlist = counts[bin];
-  const uint32_t blk0 = blockIdx.x * (uint32_t)A.tpb;
+  // The grid is capped (most bins of a large batch are small, and a launch's
+  // surplus blocks are not free: 122,000 empty ones took 27-54 us a bin), so a
+  // block owns more than one chunk of tpb descriptors where the bin is large.
+  const uint32_t tpb = max((uint32_t)A.tpb, (nlist + gridDim.x - 1) / gridDim.x);
+  const uint32_t blk0 = blockIdx.x * tpb;
   if (blk0 >= nlist) return;  // uniform over the block
-  const uint32_t blk1 = min(blk0 + (uint32_t)A.tpb, nlist);
+  const uint32_t blk1 = min(blk0 + tpb, nlist);
   if (threadIdx.x == 0) lds_next = blk0;
   __syncthreads();
   const ExtDesc* __restrict__ desc = desc_all + lbase;
@@ -345,15 +350,22 @@ __device__ __forceinline__ int ext_bin_of(int qlen) {
   return -1;
 }
 
-// Whether the pair kernel computes this task: every score of the run, its cell
-// count and its z-drop test fit 16 bits, and its first row reaches no column
-// past the band (a band of qlen or more holds every column; else the
-// first-row value at column w+1, h0 - oe_ins - w*e_ins, must not be positive).
-__device__ __forceinline__ bool pair_takes(const ExtArgs& A, int64_t t, int qlen, int tlen, int h0) {
-  if (!A.pair || tlen > kPairMaxTlen || h0 + qlen * A.mat_max > kPairScoreMax) return false;
-  const int w = ext_clamped_w(A, t);
-  return w >= qlen || (int64_t)h0 - A.o_ins - A.e_ins - (int64_t)w * A.e_ins <= 0;
+// Bin of a task the pair kernel does not take.
+__device__ __forceinline__ int ext_group_bin_of(int qlen) {
+#pragma unroll
+  for (int b = kQueryBins; b < kExtBins; ++b)
+    if (qlen <= bin_limit(b)) return b;
+  return kPairBins;
 }
+static_assert(bin_limit(kPairBins - 1) <= bin_limit(kPairBins), "every pair-bin query fits a group bin");
+
+// Whether the pair kernel of bin b computes this task: every score of the run
+// and its z-drop test fit 16 bits.
+__device__ __forceinline__ bool pair_takes(const ExtArgs& A, int b, int qlen, int tlen, int h0) {
+  const int most = b == 4 ? pair_score_max(kExtShape[4].cols) : pair_score_max(kExtShape[3].cols);
+  return A.pair && tlen <= kPairMaxTlen && h0 + qlen * A.mat_max <= most;
+}
+static_assert(pair_score_max(kExtShape[0].cols) == pair_score_max(kExtShape[3].cols) && kPairBins == 5, "score limits");
 
 // mode 0: validate every task, write bin_of and count per bin and row bucket
 // mode 1: validate only (the learned-band form counts after its narrow pass)
@@ -385,7 +397,7 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
       ++bad;
       first_bad = min(first_bad, (int)t);
     } else {
-      if (b < kPairBins && !pair_takes(A, t, ql, tl, h0)) b = kShortBin;
+      if (b < kPairBins && !pair_takes(A, b, ql, tl, h0)) b = ext_group_bin_of(ql);
       if (mode == 0) {
         atomicAdd(&hist[b], 1u);
         atomicAdd(&bhist[b * kRowBuckets + row_bucket(tl, h0)], 1u);
@@ -477,10 +489,10 @@ ext_unpack_kernel(ExtArgs A, ExtWork W, const int32_t* __restrict__ rec) {
 // 10.6) and 500 flanks of 150 bp reads in 16 (1.11 ms, now 0.24).
 template <int L, int C, bool E1>
 static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st) {
-  constexpr int64_t kBlocksPerSimd = 4;
+  constexpr int64_t kBlocksPerSimd = 4, kMaxBlocksPerCu = 128;
   const int64_t fill = n / (num_cu * 4 * kBlocksPerSimd);
   k.tpb = (int)std::min<int64_t>(k.tpb, std::max<int64_t>(64 / L, fill));
-  const int64_t blocks = (n + k.tpb - 1) / k.tpb;
+  const int64_t blocks = std::min<int64_t>((n + k.tpb - 1) / k.tpb, (int64_t)num_cu * kMaxBlocksPerCu);
   if (blocks < 1) return;
   time_begin(wk, time_slot_bin(B), st);
   hipLaunchKernelGGL((ext_plain_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, st, k,
@@ -504,11 +516,14 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
   }
 }
 
-template <int B, bool E1>
-static void launch_bins_from(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st, bool pair) {
-  launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[B]), pair);
-  if constexpr (B > 0) launch_bins_from<B - 1, E1>(k, wk, n, num_cu, st, pair);
+// The pair bins of a large batch hold nearly all of its work: they start first.
+template <bool E1, int... B>
+static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st, bool pair,
+                        std::integer_sequence<int, B...>) {
+  (launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[B]), pair), ...);
 }
+using BinOrder = std::integer_sequence<int, 4, 3, 2, 1, 0, 8, 7, 6, 5, 11, 10, 9>;
+static_assert(kExtBins == 12, "launch order");
 
 hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan) {
   a.pair = a.n >= kPairMinTasks && a.e_del <= kPairMaxGapExt && a.e_ins <= kPairMaxGapExt;
@@ -547,9 +562,8 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   hipLaunchKernelGGL(ext_bin_scatter_kernel, dim3((unsigned)sblocks), dim3(256), 0, st, a, wk, per_block,
                      band ? (const uint8_t*)wk.need_plain : nullptr);
   ss_fork(wk.ss, st);
-  // longest queries first so the long tasks do not form the tail
-  if (a.e_del == 1 && a.e_ins == 1) launch_bins_from<kExtBins - 1, true>(k, wk, a.n, num_cu, st, a.pair);
-  else launch_bins_from<kExtBins - 1, false>(k, wk, a.n, num_cu, st, a.pair);
+  if (a.e_del == 1 && a.e_ins == 1) launch_bins<true>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
+  else launch_bins<false>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
   ss_join(wk.ss, st);
   hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
   return hipGetLastError();

@@ -1,11 +1,11 @@
 // Two-tasks-per-lane form of the bit-exact ksw_extend2
-// (bsbolt/External/BWA/ksw.c:380-479) for queries of up to 96 bases.
+// (bsbolt/External/BWA/ksw.c:380-479) for queries of up to 224 bases.
 //
 // Each lane of a wave owns two whole tasks, one in each 16-bit half of its
 // registers, so one packed instruction advances two DP cells.  Per query
 // column a lane keeps G1 = eh[j].h (plus the match score a where non-zero) and
 // E = eh[j].e.  A row is the reference's column loop run inside the lane.
-// Every value is an integer in [0, kPairScoreMax]: h0 + qlen * max(mat) bounds
+// Every value is an integer in [0, pair_score_max]: h0 + qlen * max(mat) bounds
 // all scores of a run and is checked per task, so unsigned 16-bit arithmetic
 // with subtraction saturating at 0 gives exactly the reference's values (its
 // own recurrences clamp at 0 wherever a value could go below).
@@ -21,9 +21,11 @@
 // G successors 0 as well, so no per-column mask is needed except one: F is set
 // to 0 at column `end` (the reference stops there).  That holds because beg
 // never decreases, the columns the cap i-w cuts off are zeroed here, the
-// reference's own end scan leaves only zero columns past `end`, and the
-// per-task test excludes the runs whose first row reaches past the band
-// (w < qlen and a positive first-row value at column w+1).
+// reference's own end scan leaves only zero columns past `end`, and a column
+// that no row has reached yet is given its first-row value (ksw.c:395-397) only
+// when the band first includes it: the band grows by at most two columns a row,
+// the first of them overwritten by the row before, so that is the one column
+// past the largest `end` so far.
 //
 // Position p of a task is its column j + off, off = -qlen mod 8, so that the
 // query ends on a multiple of 8: H(i, qlen-1) is then the value carried out of
@@ -34,12 +36,21 @@
 // together and the list is ordered longest run first, so the bands of a wave
 // drift through the columns together and most blocks of a row are skipped.
 //
-// VALU-bound: 21 packed instructions per column (168 per block) and 175 per
-// row, for 128 tasks at once; the lane-per-task and 16-lane kernels it replaced
-// took 31 per column for 64 tasks and ~300 per row for 4.  3.9M flanks of
-// 2x150 bp reads, queries of <= 32 / 33-64 / 65-96 bases, kernel alone: 0.43 /
-// 1.46 / 1.44 ms (was 1.16 / 3.5 / 5.0); the whole call 6.2 ms (was 11.9).
+// VALU-bound: 20 packed instructions per column (162 per block) and ~175 per
+// row, for 128 tasks at once; the kernels it replaced took 31 per column for 64
+// tasks (lane per task) and ~300 per row for 2-4 tasks (16-64 lanes per task).
+// Widths 32 to 96 hold the state in the 256 VGPRs of two (three) waves per SIMD
+// and issue VALU on 79-90% of the cycles.  Widths 128 and 224 take all 512
+// registers of a SIMD for one wave: the compiler keeps the columns past ~96 in
+// accumulation registers, two to four moves per eight columns, and a lone wave
+// issues on half the cycles; that still is 3 (128) to 6 (224) times the group
+// kernels' rate.  Kernel alone, queries of <= 32 / 33-64 / 65-96 / 97-128 /
+// 129-224 bases: 3.9M flanks of 2x150 bp reads 0.42 / 1.42 / 1.47 / 0.85 / 0.14
+// ms (was 1.16 / 3.5 / 5.0 / 2.5 / 0.33); 351,491 flanks of 250 bp reads 0.18 /
+// 0.49 / 0.86 / 1.19 / 2.39 ms (97 and longer: was 2.3 / 9.2).  Whole calls: 4.2
+// ms (was 11.9) and 3.6 ms (was 10.2).
 #include <type_traits>
+#include <utility>
 
 #include "bsx_internal.h"
 #include "ext_common.h"
@@ -67,36 +78,26 @@ __device__ __forceinline__ u16x2 smin(u16x2 a, u16x2 b) {
   return __builtin_bit_cast(u16x2, __builtin_elementwise_min(pks(a), pks(b)));
 }
 
-// The next three are written as instructions: the compiler turns min(x, 1) into
-// a compare and a select per half, and a multiply by a power of two into shifts.
-__device__ __forceinline__ u16x2 one_if(u16x2 x) {  // 1 in every non-zero half
-  u16x2 r;
-  asm("v_pk_min_u16 %0, %1, 1 op_sel_hi:[1,0]" : "=v"(r) : "v"(x));
-  return r;
-}
-__device__ __forceinline__ u16x2 mad(u16x2 x, u16x2 s, u16x2 y) {  // x * s + y, s uniform
-  u16x2 r;
-  asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(s), "v"(y));
-  return r;
-}
-template <int K>
-__device__ __forceinline__ u16x2 mad_add(u16x2 x, u16x2 s, std::integral_constant<int, K>) {  // x * s + K, 0 <= K <= 64
-  u16x2 r;
-  asm("v_pk_mad_u16 %0, %1, %2, %3 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(x), "s"(s), "n"(K));
-  return r;
-}
-template <int K>
-__device__ __forceinline__ u16x2 mad_mul(u16x2 x, std::integral_constant<int, K>, u16x2 y) {  // x * K + y, 0 <= K <= 64
-  u16x2 r;
-  asm("v_pk_mad_u16 %0, %1, %2, %3 op_sel_hi:[1,0,1]" : "=v"(r) : "v"(x), "n"(K), "v"(y));
-  return r;
+// A uniform constant in both halves whose value the compiler does not see: it
+// would turn min(x, 1) into a compare and a select per half, a multiply by a
+// power of two into shifts, and a chain of subtractions into one constant each.
+__device__ __forceinline__ u16x2 hidden(uint32_t x) {
+  uint32_t v = x | x << 16;
+  asm("" : "+s"(v));
+  return pk(v);
 }
 
-// In-place forms: the result takes its operand's register, so the column state
-// keeps its registers through the conditional blocks (no copies at the joins).
-__device__ __forceinline__ void in_and(u16x2& x, uint32_t m) { asm("v_and_b32 %0, %0, %1" : "+v"(x) : "v"(m)); }
-__device__ __forceinline__ void in_sat(u16x2& x, u16x2 s) { asm("v_pk_sub_u16 %0, %0, %1 clamp" : "+v"(x) : "s"(s)); }
-__device__ __forceinline__ void in_max(u16x2& x, u16x2 y) { asm("v_pk_max_u16 %0, %0, %1" : "+v"(x) : "v"(y)); }
+// x * e, at most 0xffff (x a column number below 2^14, e below 2^16)
+__device__ __forceinline__ u16x2 emul(u16x2 x, u16x2 e) {
+  const uint32_t lo = (pku(x) & 0xffffu) * (pku(e) & 0xffffu), hi = (pku(x) >> 16) * (pku(e) >> 16);
+  return pk(min(lo, 0xffffu) | min(hi, 0xffffu) << 16);
+}
+
+// f(0), f(1), ... with compile-time arguments (a loop this long is not unrolled)
+template <class F, int... I>
+__device__ __forceinline__ void for_each_index(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
 
 // bitwise OR over the wave, as a scalar
 __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
@@ -126,15 +127,17 @@ struct PairSeq {
 };
 
 // waves per SIMD the register budget leaves room for
-constexpr int pair_min_waves(int Q) { return Q <= 32 ? 3 : 2; }
+constexpr int pair_min_waves(int Q) { return Q <= 32 ? 3 : Q <= 96 ? 2 : 1; }
 
-template <int Q>
+template <int Q, bool SAME>
 __global__ void __launch_bounds__(64, pair_min_waves(Q))
 ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t* __restrict__ counts, int bin) {
   constexpr int NB = Q / 8;
-  static_assert(Q % 8 == 0 && Q <= 128, "pair kernel width");
-  constexpr uint32_t kStep = kPairScoreMax;  // F cap per column left before `end`: above any score
-  static_assert(kStep * Q <= 65535, "cap fits 16 bits");
+  static_assert(Q % 8 == 0 && NB < 31, "pair kernel width");
+  constexpr int KB = Q <= 128 ? 7 : 8;                   // position bits of a (score, position) key
+  constexpr uint32_t kStep = pair_score_max(Q);          // F cap per column left before `end`: no score above it
+  constexpr uint32_t kEndStep = Q <= 120 ? 4096 : 2048;  // query-end test, per block left: above any score
+  static_assert(kStep * Q <= 65535 && (kStep << KB) + Q <= 65536 && kEndStep * NB <= 65535, "16-bit ranges");
   __shared__ uint2 trow[8];         // penalties of a target code: query codes 0..3, and N
   __shared__ uint4 s_q[NB][64];     // query codes of a block: task 0 (.x .z), task 1 (.y .w)
   const int lane = threadIdx.x;
@@ -152,7 +155,9 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
   }
   const ExtDesc* __restrict__ desc = desc_all + lbase;
 
-  const u16x2 s128 = splat(128u);
+  const u16x2 one = hidden(1), step = hidden(kStep), skey = hidden(1u << KB);
+  const u16x2 bit[8] = {one, hidden(2), hidden(4), hidden(8), hidden(16), hidden(32), hidden(64), hidden(128)};
+  auto one_if = [&](u16x2 x) { return pkmin(x, one); };  // 1 in every non-zero half
   const u16x2 a_ = splat((uint32_t)A.mat_max);
   const u16x2 oe_del = splat((uint32_t)min(A.o_del + A.e_del, 0xffff));
   const u16x2 oe_ins = splat((uint32_t)min(A.o_ins + A.e_ins, 0xffff));
@@ -194,13 +199,15 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
   const u16x2 off = pk2((8 - qlen[0]) & 7, (8 - qlen[1]) & 7), qpos = ql + off;
   const u16x2 offbit = pk2(1 << ((8 - qlen[0]) & 7), 1 << ((8 - qlen[1]) & 7));
   const u16x2 wv = pk2(w[0], w[1]);
-  const u16x2 qcap = qpos * splat(512u);  // (qpos / 8) * 4096: block test of the query end
+  const u16x2 qcap = qpos * splat(kEndStep / 8);  // kEndStep per block of the query
+
+  const u16x2 hh0 = pk2(h0[0], h0[1]);
 
   // ---- state ----
   u16x2 G[Q], E[Q];
   {  // first row (ksw.c:395-397): eh[0].h = h0, eh[j].h = max(h0 - oe_ins - (j-1)*e_ins, 0)
-    const u16x2 hh = pk2(h0[0], h0[1]);
-    u16x2 ramp = pksat(hh, oe_ins), cap = qpos * splat(kStep);  // nothing past the query's end
+    const u16x2 hh = hh0;
+    u16x2 ramp = pksat(hh, oe_ins), cap = smin(qpos, wv + off + splat(1u)) * splat(kStep);  // nothing past the first row's band
 #pragma unroll
     for (int p = 0; p < Q; ++p) {
       u16x2 g;
@@ -216,16 +223,21 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
       }
       g = pkmin(g, cap);
       cap = pksat(cap, splat(kStep));
-      G[p] = mad(one_if(g), a_, g);
+      G[p] = one_if(g) * a_ + g;
       E[p] = splat(0u);
     }
   }
   u16x2 beg = splat(0u), end = ql;  // columns, not positions
-  u16x2 fcol = pksat(pk2(h0[0], h0[1]), splat((uint32_t)min(A.o_del, 0xffff)));  // first-column value before row 0
-  u16x2 best = pk2(h0[0], h0[1]), best_i = splat(0xffffu), best_j = splat(0xffffu);
-  u16x2 gbest = splat(0xffffu), gbest_i = splat(0xffffu), moff = splat(0u), ncell = splat(0u);
+  u16x2 emax = smin(ql, wv + splat(1u));  // largest end so far
+  // first-row values past the first row's band, of any task of the wave
+  const bool ramped = __any(pku(pksat(pksat(hh0, oe_ins), emul(emax - splat(1u), e_ins)) &
+                                pk(negmask(emax - ql))) != 0);
+  u16x2 fcol = pksat(hh0, splat((uint32_t)min(A.o_del, 0xffff)));  // first-column value before row 0
+  u16x2 best = hh0, best_i = splat(0xffffu), best_j = splat(0xffffu);
+  u16x2 gbest = splat(0xffffu), gbest_i = splat(0xffffu), moff = splat(0u);
+  uint32_t ncell[2] = {0, 0};
   uint32_t act = ~negmask(tl - splat(1u));  // halves whose task runs
-  const u16x2 zd = splat((uint32_t)(A.zdrop > 0 && A.zdrop < 0x3fff ? A.zdrop : 0x3fff));
+  const u16x2 zd = splat((uint32_t)(A.zdrop > 0 && A.zdrop < 1023 ? A.zdrop : 1023));
   beg = beg & pk(act);
   end = end & pk(act);
 
@@ -262,6 +274,16 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
     const u16x2 fc1 = fcol + one_if(fcol) * a_;
     const u16x2 endp = end + off;
     // blocks with a column in [beg, end] of a running task
+    u16x2 newcol = splat(0u), newg = splat(0u);
+    bool grown = false;
+    if (ramped) {
+      const u16x2 nc = emax + splat(1u);
+      const u16x2 r = pksat(pksat(hh0, oe_ins), emul(emax, e_ins)) & pk(negmask(nc - end));
+      newg = r + one_if(r) * a_;
+      newcol = nc + off;
+      grown = __any(pku(newg) != 0);
+      emax = smax(emax, end);
+    }
     uint32_t live;
     {
       const uint32_t ep = pku(smin(endp, qpos - splat(1u))), bp = pku(beg0 + off);
@@ -274,8 +296,8 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
     const u16x2 x0 = endp * splat(kStep);
 
     u16x2 F = splat(0u), carry = splat(0u), mk = splat(0u), hk = splat(0u), lk = splat(0u), hl = splat(0u);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
+    auto block = [&](auto bb) {
+      constexpr int b = decltype(bb)::value;
       if (live >> b & 1u) {
         const uint4 q = s_q[b][lane];
         u16x2 X = pksat(x0, splat(kStep * 8u * b));
@@ -285,9 +307,17 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
             const uint32_t keep = ~negmask(d);
-            in_and(G[8 * b + c], keep);
-            in_and(E[8 * b + c], keep);
+            G[8 * b + c] = G[8 * b + c] & pk(keep);
+            E[8 * b + c] = E[8 * b + c] & pk(keep);
             d = d + splat(1u);
+          }
+        }
+        if (grown) {  // a column the band reaches for the first time
+          u16x2 d = newcol - splat(8u * b);
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            G[8 * b + c] = G[8 * b + c] | (newg & pk(negmask(one_if(d) - splat(1u))));
+            d = d - splat(1u);
           }
         }
         u16x2 M[8];
@@ -306,45 +336,33 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
           if (b == 0) G[p] = ((offbit >> (uint16_t)c) & splat(1u)) * fc1 + carry;  // carry is 0 up to column 0
           else G[p] = carry;
           const u16x2 t = one_if(h);
-          carry = mad(t, a_, h);
-          in_sat(E[p], e_del);
-          in_max(E[p], pksat(M[c], oe_del));
-          X = pksat(X, splat(kStep));
-          F = pkmin(pkmax(pksat(M[c], oe_ins), pksat(F, e_ins)), X);
-          kb = pkmax(kb, mad_add(h, s128, cc));
-          const u16x2 te = one_if(E[p]);
-          if constexpr (c < 7) {
-            hb = mad_mul(t, std::integral_constant<int, 1 << c>{}, hb);
-            eb = mad_mul(te, std::integral_constant<int, 1 << c>{}, eb);
-          } else {
-            hb = mad(t, s128, hb);
-            eb = mad(te, s128, eb);
-          }
+          carry = t * a_ + h;
+          const u16x2 open = pksat(M[c], oe_del);
+          E[p] = pkmax(pksat(E[p], e_del), open);
+          X = pksat(X, step);
+          F = pkmin(pkmax(SAME ? open : pksat(M[c], oe_ins), pksat(F, e_ins)), X);
+          kb = pkmax(kb, h * skey + splat((uint32_t)c));
+          hb = t * bit[c] + hb;
+          eb = one_if(E[p]) * bit[c] + eb;
         };
-        column(std::integral_constant<int, 0>{});
-        column(std::integral_constant<int, 1>{});
-        column(std::integral_constant<int, 2>{});
-        column(std::integral_constant<int, 3>{});
-        column(std::integral_constant<int, 4>{});
-        column(std::integral_constant<int, 5>{});
-        column(std::integral_constant<int, 6>{});
-        column(std::integral_constant<int, 7>{});
+        for_each_index(column, std::make_integer_sequence<int, 8>{});
         mk = pkmax(mk, kb + splat(8u * b));
         // last block with a non-zero H: its bits below its number
         hk = pkmax(hk, one_if(hb) * splat(256u * b) + hb);
         // first block with a non-zero E(j) or G(j): bits of E | H shifted to G's column
         const u16x2 cb = pk(pku(hb) << 1 | pku(eb));
-        lk = pkmax(lk, one_if(cb) * splat(512u * (15u - b)) + cb);
+        lk = pkmax(lk, one_if(cb) * splat(512u * (31u - b)) + cb);
         // the value carried out of the block that ends the query is H(i, qlen-1);
         // nothing is carried past it
-        const u16x2 z = pksat(qcap, splat(4096u * (b + 1)));
+        const u16x2 z = pksat(qcap, splat(kEndStep * (b + 1)));
         hl = pkmax(hl, pksat(carry, z));
         carry = pkmin(carry, z);
       } else {
         carry = splat(0u);
         F = splat(0u);
       }
-    }
+    };
+    for_each_index(block, std::make_integer_sequence<int, NB>{});
 
     // ---- end of row (ksw.c:449-470) ----
     const uint32_t some = negmask(beg - end);  // end > beg
@@ -356,9 +374,13 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
       gbest_i = sel(up, iv, gbest_i);
       gbest = sel(up, h1, gbest);
     }
-    ncell = ncell + ((end - beg) & pk(some & act));
-    const u16x2 m = (mk >> (uint16_t)7);
-    const u16x2 mj = (mk & splat(127u)) - off;
+    {
+      const uint32_t w2 = pku(end - beg) & some & act;
+      ncell[0] += w2 & 0xffffu;
+      ncell[1] += w2 >> 16;
+    }
+    const u16x2 m = mk >> (uint16_t)KB;
+    const u16x2 mj = (mk & splat((1u << KB) - 1)) - off;
     const uint32_t better = negmask(best - m) & act;
     const u16x2 di = iv - best_i, dj = mj - best_j;
     const u16x2 dd = di - dj;
@@ -378,7 +400,7 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
       for (int k = 0; k < 2; ++k) {
         const uint32_t hv = k ? hk32 >> 16 : hk32 & 0xffffu, lv = k ? lk32 >> 16 : lk32 & 0xffffu;
         ne[k] = (int)((hv >> 8) * 8) + 31 - (int)__builtin_clz((hv & 255u) | 1u);
-        nb[k] = (int)((15u - (lv >> 9)) * 8) + (int)__builtin_ctz(lv | 0x10000u);
+        nb[k] = (int)((31u - (lv >> 9)) * 8) + (int)__builtin_ctz(lv | 0x10000u);
       }
       const u16x2 npos = pk2(ne[0], ne[1]) - off + splat(3u);
       end = smin(npos, ql) & pk(act);
@@ -392,7 +414,7 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
     auto h16 = [&](u16x2 v) { return k ? (int)((int32_t)pku(v) >> 16) : (int)(int16_t)(pku(v) & 0xffffu); };
     int4* rp = (int4*)(A.rec + (int64_t)task[k] * 8);
     rp[0] = make_int4(h16(best), h16(best_j) + 1, h16(best_i) + 1, h16(gbest_i) + 1);
-    rp[1] = make_int4(h16(gbest), h16(moff), k ? (int)(pku(ncell) >> 16) : (int)(pku(ncell) & 0xffffu), 0);
+    rp[1] = make_int4(h16(gbest), h16(moff), (int)ncell[k], 0);
   }
 }
 
@@ -401,12 +423,15 @@ void launch_pair_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, h
   const int64_t blocks = (n + 127) / 128;  // surplus blocks exit at once
   if (blocks < 1) return;
   time_begin(wk, time_slot_bin(bin), st);
-  hipLaunchKernelGGL((ext_pair_kernel<Q>), dim3((unsigned)blocks), dim3(64), 0, st, k, (const ExtDesc*)wk.desc,
-                     (const uint32_t*)wk.counts, bin);
+  const bool same = k.o_del + k.e_del == k.o_ins + k.e_ins;  // one gap-open value serves E and F
+  hipLaunchKernelGGL((same ? ext_pair_kernel<Q, true> : ext_pair_kernel<Q, false>), dim3((unsigned)blocks), dim3(64),
+                     0, st, k, (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, bin);
   time_end(wk, time_slot_bin(bin), st);
 }
 template void launch_pair_bin<32>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
 template void launch_pair_bin<64>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
 template void launch_pair_bin<96>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
+template void launch_pair_bin<128>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
+template void launch_pair_bin<224>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
 
 }  // namespace bsx

@@ -48,25 +48,35 @@ def repeat(t, n):
 
 
 CASES = {
-    # every query length of the three bins, h0 as seeds give it
-    "lengths": dict(qlens=range(1, 98), n=1940, h0=lambda r, q: r.integers(1, 140), w=(100,)),
+    # every query length of the bins up to 128 bases, h0 as seeds give it
+    "lengths": dict(qlens=range(1, 130), n=1935, h0=lambda r, q: r.integers(1, 140), w=(100,)),
+    "long_lengths": dict(qlens=(127, 128, 129, 135, 136, 137, 160, 191, 200, 222, 223, 224, 225, 230), n=700,
+                         h0=lambda r, q: r.integers(1, max(2, 256 - q)), w=(100, 300)),
     # bands narrower than the query: the cap cuts columns, the first row may reach past the band
     "bands": dict(qlens=(1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 95, 96), n=1200, h0=lambda r, q: r.integers(1, 60),
                   w=(0, 1, 2, 7, 16, 40)),
+    # the first row's values reach far past the band, and the band comes back to them
+    "first_row": dict(qlens=(40, 64, 96, 100, 128), n=1500, h0=lambda r, q: r.integers(60, 380), w=(1, 3, 10, 30, 60),
+                      sub=0.15),
+    "first_row_long": dict(qlens=(129, 150, 180, 224), n=600, h0=lambda r, q: r.integers(20, 256 - q + 1),
+                           w=(1, 3, 10, 30, 60, 100), sub=0.1),
     # N bases in query and target
     "n_bases": dict(qlens=(5, 24, 40, 64, 90, 96), n=600, h0=lambda r, q: r.integers(1, 80), w=(100,), n_frac=0.03),
     # scores at and past the kernel's limit (h0 + qlen = 511 runs in it, 512 does not)
     "scores": dict(qlens=(1, 16, 32, 64, 96), n=600, h0=lambda r, q: 511 - q + r.integers(-1, 2), w=(100, 500),
                    sub=0.0),
+    "scores_long": dict(qlens=(128, 129, 200, 224), n=400, h0=lambda r, q: (511 if q <= 128 else 255) - q + r.integers(-1, 2),
+                        w=(100, 500), sub=0.0),
     # target lengths at and past its limit, and empty targets
-    "targets": dict(qlens=(1, 32, 64, 96), n=300, h0=lambda r, q: 511 - q, w=(700,), tail=(0,), tlen=640),
+    "targets": dict(qlens=(1, 32, 64, 96, 128), n=300, h0=lambda r, q: 511 - q, w=(700,), tail=(0,), tlen=640),
     "long_targets": dict(qlens=(1, 32, 64, 96), n=300, h0=lambda r, q: 511 - q, w=(700,), tail=(0,), tlen=641),
-    "no_target": dict(qlens=(1, 32, 96), n=60, h0=lambda r, q: r.integers(1, 60), w=(100,), tlen=0),
+    "no_target": dict(qlens=(1, 32, 96, 128, 200), n=60, h0=lambda r, q: r.integers(1, 60), w=(100,), tlen=0),
 }
 SCORINGS = {
     "bsbolt": dict(),
     "asym": dict(o_del=4, e_del=2, o_ins=7, e_ins=1, zdrop=30, a=2, b=5),
     "gap25": dict(o_del=0, e_del=25, o_ins=3, e_ins=25, zdrop=0),
+    "no_zdrop_25": dict(o_del=5, e_del=25, o_ins=2, e_ins=24, zdrop=30000),
     "gap26": dict(o_del=0, e_del=26, o_ins=3, e_ins=2, zdrop=20000),
 }
 
