@@ -131,8 +131,9 @@ struct StreamSet {
   hipStream_t side[kSide] = {};
   hipEvent_t fork = nullptr, join[kSide] = {};
 };
-// launches of the plain bins: stream 0 = the call's stream, k > 0 = side[k-1]
-constexpr int kBinStream[kExtBins] = {2, 0, 1, 2, 3, 3, 2, 1, 0, 3, 2, 1};
+// streams of the plain bins' launches, without and with the pair kernels: 0 =
+// the call's stream, k > 0 = side[k-1]
+constexpr int kBinStream[2][kExtBins] = {{0, 0, 0, 0, 0, 3, 2, 1, 0, 0, 1, 2}, {0, 3, 2, 1, 0, 3, 2, 1, 3, 3, 1, 2}};
 inline hipStream_t pick_stream(const StreamSet* ss, hipStream_t main, int k) {
   return (ss && k > 0 && ss->side[k - 1]) ? ss->side[k - 1] : main;
 }

@@ -516,13 +516,17 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
   }
 }
 
-// The pair bins of a large batch hold nearly all of its work: they start first.
 template <bool E1, int... B>
 static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_cu, hipStream_t st, bool pair,
                         std::integer_sequence<int, B...>) {
-  (launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[B]), pair), ...);
+  (launch_bin<B, E1>(k, wk, n, num_cu, pick_stream(wk.ss, st, kBinStream[pair ? 1 : 0][B]), pair), ...);
 }
-using BinOrder = std::integer_sequence<int, 4, 3, 2, 1, 0, 8, 7, 6, 5, 11, 10, 9>;
+// The 224-column kernel first, on the call's own stream: its waves need a SIMD
+// to themselves and wait for long once smaller ones are spread over all of them.
+// Then the group bins, nearly empty in a batch with pair bins: behind a pair
+// kernel even an empty launch waits until the chip has room for its blocks (0.5
+// ms for one of 250 bp reads).
+using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 11, 10, 9, 3, 2, 1, 0>;
 static_assert(kExtBins == 12, "launch order");
 
 hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan) {
