@@ -18,7 +18,8 @@
 
 using namespace bsx;
 
-static constexpr size_t kSmallBytes = 4 * (size_t)kExtCounterWords;
+static constexpr size_t kSmallBytes =
+    4 * (size_t)(kExtCounterWords > kGlbCounterWords ? kExtCounterWords : kGlbCounterWords);
 
 // band model buffer: params, adam_m, adam_v (FP32), then the BF16 operand copies
 static constexpr size_t kAlign = 256;
@@ -59,8 +60,9 @@ struct Work {
   DevBuf bin_of, list, desc, rec, small;  // small: counts/cursor/err/fetch
   DevBuf nbin_of, need_plain, cls;        // learned-band form
   DevBuf zbuf;                            // direction-byte slots of the global kernel
+  DevBuf zpair;                           // direction scratch of its two-tasks-per-lane form
   void release() {
-    for (DevBuf* b : {&bin_of, &list, &desc, &rec, &small, &nbin_of, &need_plain, &cls, &zbuf}) b->release();
+    for (DevBuf* b : {&bin_of, &list, &desc, &rec, &small, &nbin_of, &need_plain, &cls, &zbuf, &zpair}) b->release();
   }
 };
 
@@ -854,6 +856,17 @@ int bsx_reg2aln_cigar_device(bsx_ctx* c, const bsx_reg2aln_tasks* t, bsx_reg2aln
   return BSX_OK;
 }
 
+static int glb_buffers(bsx_ctx* c, size_t n, bool cigar) {
+  HIPCHK(c, c->ws->bin_of.ensure(n + 1), "hipMalloc(bin_of)");
+  HIPCHK(c, c->ws->list.ensure(4 * n + 4), "hipMalloc(list)");
+  HIPCHK(c, c->ws->small.ensure(kSmallBytes), "hipMalloc(work)");
+  if (cigar) {
+    HIPCHK(c, c->ws->zbuf.ensure((size_t)glb_groups(c->num_cu, c->ss_on) * (size_t)c->zslot), "hipMalloc(z)");
+    if (n >= (size_t)kGlbPairMinTasks) HIPCHK(c, c->ws->zpair.ensure((size_t)glb_pair_bytes(c->num_cu)), "hipMalloc(zpair)");
+  }
+  return BSX_OK;
+}
+
 int bsx_global_batch_device(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tasks* t,
                             bsx_glb_results* r) {
   if (!c || !t || !r) return fail(c, BSX_EINVAL, "NULL argument");
@@ -868,14 +881,15 @@ int bsx_global_batch_device(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tas
   GlbArgs a{};
   a.o_del = sc->o_del; a.e_del = sc->e_del; a.o_ins = sc->o_ins; a.e_ins = sc->e_ins;
   fill_profile(a, sc);
+  a.mat_max = mat_max(sc);
+  for (int k = 0; k < 25; ++k) a.pen_max = a.mat_max - sc->mat[k] > a.pen_max ? a.mat_max - sc->mat[k] : a.pen_max;
   a.n = t->n;
   a.query = t->query; a.q_off = t->q_off; a.qlen = t->qlen;
   a.target = t->target; a.t_off = t->t_off; a.tlen = t->tlen; a.w = t->w;
   a.score = r->score; a.n_cigar = r->n_cigar; a.cigar = r->cigar; a.cigar_slot = r->cigar_slot;
   const size_t n = (size_t)t->n;
-  HIPCHK(c, c->ws->bin_of.ensure(n + 1), "hipMalloc(bin_of)");
-  HIPCHK(c, c->ws->list.ensure(4 * n + 4), "hipMalloc(list)");
-  HIPCHK(c, c->ws->small.ensure(kSmallBytes), "hipMalloc(work)");
+  rc = glb_buffers(c, n, r->cigar != nullptr);
+  if (rc) return rc;
   GlbWork wk;
   wk.bin_of = (uint8_t*)c->ws->bin_of.p;
   wk.list = (int32_t*)c->ws->list.p;
@@ -883,13 +897,13 @@ int bsx_global_batch_device(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tas
   wk.cursor = wk.counts + kCountSlots;
   wk.err = (int32_t*)(wk.cursor + kCountSlots);
   wk.fetch = (uint32_t*)(wk.err + 4);
+  wk.kcount = wk.fetch + kFetchSlots;
+  wk.kcursor = wk.kcount + kGlbKeys;
   wk.zslot = c->zslot;
   wk.ss = c->ss_on ? &c->ss : nullptr;
-  wk.z = nullptr;
-  if (r->cigar) {
-    HIPCHK(c, c->ws->zbuf.ensure((size_t)glb_groups(c->num_cu, c->ss_on) * (size_t)c->zslot), "hipMalloc(z)");
-    wk.z = (uint8_t*)c->ws->zbuf.p;
-  }
+  wk.z = r->cigar ? (uint8_t*)c->ws->zbuf.p : nullptr;
+  wk.zpair = r->cigar ? (uint8_t*)c->ws->zpair.p : nullptr;
+  wk.pair_bytes = 0;
   HIPCHK(c, launch_global_impl(a, wk, c->num_cu, c->stream), "global launch");
   HIPCHK(c, hipMemcpyAsync(c->err_host, wk.err, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream),
          "hipMemcpyAsync(err)");
@@ -1049,12 +1063,7 @@ int bsx_graph_capture_global(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_ta
                              bsx_graph** out) {
   if (!c || !t || !r) return fail(c, BSX_EINVAL, "NULL argument");
   auto sized = [&]() -> int {
-    const size_t n = t->n > 0 ? (size_t)t->n : 0;
-    HIPCHK(c, c->ws->bin_of.ensure(n + 1), "hipMalloc(bin_of)");
-    HIPCHK(c, c->ws->list.ensure(4 * n + 4), "hipMalloc(list)");
-    HIPCHK(c, c->ws->small.ensure(kSmallBytes), "hipMalloc(work)");
-    if (r->cigar) HIPCHK(c, c->ws->zbuf.ensure((size_t)glb_groups(c->num_cu, c->ss_on) * (size_t)c->zslot), "hipMalloc(z)");
-    return BSX_OK;
+    return glb_buffers(c, t->n > 0 ? (size_t)t->n : 0, r->cigar != nullptr);
   };
   return capture(c, 2, sized, [&]() { return bsx_global_batch_device(c, sc, t, r); }, out);
 }

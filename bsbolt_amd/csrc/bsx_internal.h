@@ -29,6 +29,39 @@ constexpr int kGlbBins = 9;
 constexpr BinShape kGlbShape[kGlbBins] = {
     {8, 2}, {8, 3}, {8, 4}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
 constexpr int kExtSlices = 8;  // fetch-counter slots per bin (CIGAR bins, lane frame classes)
+// Bins of the two-tasks-per-lane CIGAR kernel (gpair.hip), after the others:
+// band widths 2w+1 up to kGlbPairCols, each from glb_pair_top + 1 on.
+constexpr int kGlbPairBins = 5;
+constexpr int kGlbPairCols[kGlbPairBins] = {15, 23, 31, 47, 63};
+__host__ __device__ constexpr int glb_pair_top(int NC) { return NC == 15 ? 0 : NC <= 31 ? NC - 7 : NC - 15; }
+constexpr int kGlbAllBins = kGlbBins + kGlbPairBins;
+constexpr int kGlbPairTlen = 320;        // longest target of a task of these bins
+constexpr int kGlbPairRange = 28000;     // largest size of its scores (16-bit values, -inf = -30000)
+// Direction scratch of these bins, a nibble per cell: the share of every bin
+// (in 1/64 of the total, kGlbPairScratch bytes per CU) is divided among as many
+// waves as have room for 128 tasks of the bin's longest target.  2.5 GB on 256
+// CUs; 150 bp reads run 2,000-4,000 waves a bin.
+constexpr int64_t kGlbPairScratch = 10 << 20;
+constexpr int kGlbPairShare[kGlbPairBins] = {9, 17, 8, 16, 14};
+__host__ __device__ constexpr int64_t glb_pair_region(int NC, int rows) { return (int64_t)128 * rows * 4 * ((NC + 7) / 8); }
+constexpr int64_t glb_pair_bytes(int num_cu) { return kGlbPairScratch * num_cu; }
+// Lists of these bins are ordered by target length, longest first, one bucket
+// per length: the tasks of a wave then take equally many rows, and its lanes walk
+// back through the same row at the same time (one 768-byte piece of scratch per
+// load; with steps of 10 rows the walk fetched a line per lane and took half of
+// the kernel's time).  The other bins have one bucket.
+constexpr int kGlbKeys = kGlbBins + kGlbPairBins * kGlbPairTlen;
+__host__ __device__ constexpr int glb_key(int bin, int tlen) {
+  return bin < kGlbBins ? bin : kGlbBins + (bin - kGlbBins) * kGlbPairTlen + (kGlbPairTlen - tlen);
+}
+// rows of a region for targets of up to tlen bases (whole turns of four rows)
+__host__ __device__ constexpr int glb_pair_rows(int tlen) { return (tlen + 3) / 4 * 4; }
+// Smallest batch whose narrow bands run the pair kernel: below it the batch
+// takes the latency of its waves, and the group kernels finish sooner.  us per
+// call, pair / group kernels: 100 bp reads 64,000 tasks 911 / 684, 128,000 1029 /
+// 967, 300,000 1125 / 1711; 150 bp 64,000 1247 / 1133, 128,000 1333 / 1556; 250
+// bp 64,000 2691 / 2171, 128,000 2670 / 3078.
+constexpr int64_t kGlbPairMinTasks = 98304;
 constexpr int glb_bin_limit(int b) { return kGlbShape[b].lanes * kGlbShape[b].cols; }
 // First entry of fetch slice s of a list of n entries: a balanced partition,
 // the first n % kExtSlices slices hold one entry more.
@@ -231,7 +264,9 @@ hipError_t launch_narrow(const ExtArgs& a, const ExtKArgs& k, const ExtWork& wk,
                          const BandPlan& plan);
 
 struct GlbArgs {
-  int o_del, e_del, o_ins, e_ins;
+  int o_del, e_del, o_ins, e_ins, mat_max;
+  int pen_max;  // largest mat_max - s
+  bool pair;    // the batch's narrow bands may run the two-tasks-per-lane kernel
   uint32_t prof_lo[5];
   int32_t prof_hi[5];
   int64_t n;
@@ -255,8 +290,12 @@ struct GlbWork {
   uint32_t* cursor;
   uint32_t* fetch;
   int32_t* err;  // [0] rejected, [1] first rejected, [2] CIGAR overflows
+  uint32_t* kcount;   // [kGlbKeys] tasks per bin and bucket (glb_key)
+  uint32_t* kcursor;  // [kGlbKeys] scatter cursors of the same
   uint8_t* z;    // per-group direction-byte slots
   int64_t zslot; // bytes per slot
+  uint8_t* zpair;      // direction scratch of the pair kernel (glb_pair_bytes), nullptr without CIGARs
+  int64_t pair_bytes;  // this bin's share of it
   const StreamSet* ss;  // side streams for the bins with few tasks per group (nullptr: one stream)
 };
 
@@ -302,6 +341,9 @@ hipError_t launch_reg2aln_cigar(const Reg2alnArgs& a, int num_cu, hipStream_t st
 // size); the scratch holds one slot per group.
 constexpr int glb_blocks_per_cu(int lanes) { return lanes < 16 ? 4 : 7; }
 int64_t glb_groups(int num_cu, bool side);  // scratch slots, with or without the side-stream region
-hipError_t launch_global_impl(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st);
+void launch_glb_pair(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st);
+hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st);
+// counters of a CIGAR call: counts, cursor, err[4], fetch, kcount, kcursor
+constexpr int kGlbCounterWords = 2 * kCountSlots + 4 + kFetchSlots + 2 * kGlbKeys;
 
 }  // namespace bsx

@@ -18,6 +18,8 @@
 // caller-sized slot.  The walk reads the slot through an LDS window of whole
 // rows: the group loads the next rows with all its lanes at once (one HBM
 // latency per window, not one per step) and every step then reads LDS.
+#include <algorithm>
+
 #include "bsx_internal.h"
 
 namespace bsx {
@@ -388,10 +390,24 @@ __device__ __forceinline__ int glb_bin_of(int ncol) {
   return -1;
 }
 
+// Bin of the two-tasks-per-lane kernel for a valid task, or -1: the whole band
+// (not clipped to the query) fits, and every score fits its 16 bits.
+__device__ __forceinline__ int glb_pair_bin_of(const GlbArgs& A, int ql, int tl, int w) {
+  if (!A.pair || tl > kGlbPairTlen) return -1;
+  const int width = 2 * min(w, max(ql, tl)) + 1;
+  const int64_t range = (int64_t)(ql + tl) * (A.pen_max + max(A.e_del, A.e_ins) + A.mat_max) + A.o_del + A.o_ins;
+  if (range > kGlbPairRange) return -1;
+#pragma unroll
+  for (int b = 0; b < kGlbPairBins; ++b)
+    if (width <= kGlbPairCols[b]) return kGlbBins + b;
+  return -1;
+}
+
 __global__ void __launch_bounds__(256)
 glb_bin_count_kernel(GlbArgs A, GlbWork W) {
-  __shared__ uint32_t hist[kGlbBins];
-  if (threadIdx.x < kGlbBins) hist[threadIdx.x] = 0;
+  __shared__ uint32_t hist[kGlbAllBins], khist[kGlbKeys];
+  if (threadIdx.x < kGlbAllBins) hist[threadIdx.x] = 0;
+  for (int k = threadIdx.x; k < kGlbKeys; k += blockDim.x) khist[k] = 0;
   __syncthreads();
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < A.n;
        t += (int64_t)gridDim.x * blockDim.x) {
@@ -406,44 +422,69 @@ glb_bin_count_kernel(GlbArgs A, GlbWork W) {
       atomicAdd(&W.err[0], 1);
       atomicMin(&W.err[1], (int)t);
     } else {
+      const int pb = glb_pair_bin_of(A, ql, tl, w);
+      b = pb >= 0 ? pb : b;
       atomicAdd(&hist[b], 1u);
+      atomicAdd(&khist[glb_key(b, tl)], 1u);
     }
     W.bin_of[t] = (uint8_t)b;
   }
   __syncthreads();
-  if (threadIdx.x < kGlbBins && hist[threadIdx.x]) atomicAdd(&W.counts[threadIdx.x], hist[threadIdx.x]);
+  if (threadIdx.x < kGlbAllBins && hist[threadIdx.x]) atomicAdd(&W.counts[threadIdx.x], hist[threadIdx.x]);
+  for (int k = threadIdx.x; k < kGlbKeys; k += blockDim.x)
+    if (khist[k]) atomicAdd(&W.kcount[k], khist[k]);
 }
 
-// Ranks within a bin are taken in LDS per 256 tasks and the block reserves
-// each bin's run with one device atomic (a same-address device atomic per
-// task serialises the whole batch on kGlbBins addresses).
+// One block: the start of every bucket's run in the lists.
+__global__ void __launch_bounds__(1024) glb_bin_offset_kernel(GlbWork W) {
+  __shared__ uint32_t part[1024];
+  constexpr int PER = (kGlbKeys + 1023) / 1024;
+  const int k0 = threadIdx.x * PER;
+  uint32_t s = 0;
+  for (int k = k0; k < k0 + PER && k < kGlbKeys; ++k) s += W.kcount[k];
+  part[threadIdx.x] = s;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {
+    const uint32_t x = (int)threadIdx.x >= d ? part[threadIdx.x - d] : 0u;
+    __syncthreads();
+    part[threadIdx.x] += x;
+    __syncthreads();
+  }
+  uint32_t at = part[threadIdx.x] - s;
+  for (int k = k0; k < k0 + PER && k < kGlbKeys; ++k) {
+    W.kcursor[k] = at;
+    at += W.kcount[k];
+  }
+}
+
+// Each block counts its contiguous range of tasks per bin and bucket in LDS and
+// reserves each run with one device atomic (a same-address device atomic per
+// task serialises the whole batch on a few addresses).
 __global__ void __launch_bounds__(256)
-glb_bin_scatter_kernel(int64_t n, GlbWork W) {
-  __shared__ uint32_t off[kGlbBins], cnt[kGlbBins], run[kGlbBins];
-  if (threadIdx.x == 0) {
-    uint32_t s = 0;
-    for (int b = 0; b < kGlbBins; ++b) { off[b] = s; s += W.counts[b]; }
+glb_bin_scatter_kernel(GlbArgs A, GlbWork W, int64_t per_block) {
+  __shared__ uint32_t cur[kGlbKeys];
+  const int64_t t0 = (int64_t)blockIdx.x * per_block, t1 = min(A.n, t0 + per_block);
+  for (int k = threadIdx.x; k < kGlbKeys; k += blockDim.x) cur[k] = 0;
+  __syncthreads();
+  for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
+    const int b = W.bin_of[t];
+    if (b != 0xff) atomicAdd(&cur[glb_key(b, A.tlen[t])], 1u);
   }
-  for (int64_t t0 = (int64_t)blockIdx.x * blockDim.x; t0 < n; t0 += (int64_t)gridDim.x * blockDim.x) {
-    if (threadIdx.x < kGlbBins) cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t t = t0 + threadIdx.x;
-    const int b = t < n ? W.bin_of[t] : 0xff;
-    uint32_t r = 0;
-    if (b != 0xff) r = atomicAdd(&cnt[b], 1u);
-    __syncthreads();
-    if (threadIdx.x < kGlbBins)
-      run[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(&W.cursor[threadIdx.x], cnt[threadIdx.x]) : 0u;
-    __syncthreads();
-    if (b != 0xff) W.list[off[b] + run[b] + r] = (int32_t)t;
+  __syncthreads();
+  for (int x = threadIdx.x; x < kGlbKeys; x += blockDim.x)
+    if (cur[x]) cur[x] = atomicAdd(&W.kcursor[x], cur[x]);
+  __syncthreads();
+  for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
+    const int b = W.bin_of[t];
+    if (b != 0xff) W.list[atomicAdd(&cur[glb_key(b, A.tlen[t])], 1u)] = (int32_t)t;
   }
 }
 
-static_assert(kGlbBins <= kCountSlots && kGlbBins <= 64, "CIGAR bin counters");
-__global__ void glb_reset_kernel(GlbWork W) {
-  const int k = threadIdx.x;
-  if (k < kGlbBins) { W.counts[k] = 0; W.cursor[k] = 0; W.fetch[k] = 0; }
-  if (k == 0) { W.err[0] = 0; W.err[1] = 0x7fffffff; W.err[2] = 0; }
+static_assert(kGlbAllBins <= kCountSlots && kGlbAllBins <= 64, "CIGAR bin counters");
+__global__ void __launch_bounds__(1024) glb_reset_kernel(GlbWork W) {
+  for (int k = threadIdx.x; k < kGlbCounterWords; k += blockDim.x) W.counts[k] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) W.err[1] = 0x7fffffff;
 }
 
 
@@ -485,32 +526,54 @@ int64_t glb_groups(int num_cu, bool side) {
 }
 
 template <int B>
-static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t main) {
+static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t main, hipStream_t beside) {
   constexpr int L = kGlbShape[B].lanes, C = kGlbShape[B].cols;
   const bool side = glb_on_side(B) && w.ss != nullptr;
-  const hipStream_t st = side ? pick_stream(w.ss, main, 1) : main;
+  const hipStream_t st = side ? beside : main;
   const int bpc = side ? kGlbSideBlocksPerCU : glb_blocks_per_cu(L);
   const int64_t zbase = side ? (int64_t)num_cu * glb_groups_per_cu(false) : 0;
   hipLaunchKernelGGL((glb_kernel<L, C>), dim3((unsigned)(num_cu * bpc)), dim3(256), 0, st, a, w, B, zbase);
 }
 
-hipError_t launch_global_impl(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st) {
-  hipLaunchKernelGGL(glb_reset_kernel, dim3(1), dim3(64), 0, st, w);
+hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) {
+  w.pair_bytes = glb_pair_bytes(num_cu);
+  a.pair = a.n >= kGlbPairMinTasks;
+  hipLaunchKernelGGL(glb_reset_kernel, dim3(1), dim3(1024), 0, st, w);
   if (a.n <= 0) return hipGetLastError();
-  int64_t blocks = (a.n + 255) / 256;
-  if (blocks > (int64_t)num_cu * 16) blocks = (int64_t)num_cu * 16;
+  // each block ends with a global atomic per non-empty bucket
+  const int64_t blocks = std::min<int64_t>((a.n + 255) / 256, (int64_t)num_cu * 4);
   hipLaunchKernelGGL(glb_bin_count_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, w);
-  hipLaunchKernelGGL(glb_bin_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a.n, w);
-  ss_fork(w.ss, st);  // side streams start after the scatter
-  glb_launch_bin<3>(a, w, num_cu, st);
-  glb_launch_bin<2>(a, w, num_cu, st);
-  glb_launch_bin<8>(a, w, num_cu, st);
-  glb_launch_bin<7>(a, w, num_cu, st);
-  glb_launch_bin<6>(a, w, num_cu, st);
-  glb_launch_bin<5>(a, w, num_cu, st);
-  glb_launch_bin<4>(a, w, num_cu, st);
-  glb_launch_bin<1>(a, w, num_cu, st);
-  glb_launch_bin<0>(a, w, num_cu, st);
+  hipLaunchKernelGGL(glb_bin_offset_kernel, dim3(1), dim3(1024), 0, st, w);
+  hipLaunchKernelGGL(glb_bin_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, w, (a.n + blocks - 1) / blocks);
+  if (a.pair) {
+    // Only bin 4 (bands of 65-128) is likely to hold tasks beside the pair
+    // bins.  The others go ahead of everything, 5 us each while the chip is
+    // empty: behind a pair kernel, or beside one, even an empty launch waits
+    // until there is room for its blocks (0.5-1.3 ms measured).
+    glb_launch_bin<8>(a, w, num_cu, st, st);
+    glb_launch_bin<7>(a, w, num_cu, st, st);
+    glb_launch_bin<6>(a, w, num_cu, st, st);
+    glb_launch_bin<5>(a, w, num_cu, st, st);
+    glb_launch_bin<3>(a, w, num_cu, st, st);
+    glb_launch_bin<2>(a, w, num_cu, st, st);
+    glb_launch_bin<1>(a, w, num_cu, st, st);
+    glb_launch_bin<0>(a, w, num_cu, st, st);
+    ss_fork(w.ss, st);
+    glb_launch_bin<4>(a, w, num_cu, pick_stream(w.ss, st, 3), pick_stream(w.ss, st, 3));
+    launch_glb_pair(a, w, num_cu, st);
+  } else {
+    ss_fork(w.ss, st);  // side streams start after the scatter
+    const hipStream_t side = pick_stream(w.ss, st, 1);
+    glb_launch_bin<3>(a, w, num_cu, st, side);
+    glb_launch_bin<2>(a, w, num_cu, st, side);
+    glb_launch_bin<8>(a, w, num_cu, st, side);
+    glb_launch_bin<7>(a, w, num_cu, st, side);
+    glb_launch_bin<6>(a, w, num_cu, st, side);
+    glb_launch_bin<5>(a, w, num_cu, st, side);
+    glb_launch_bin<4>(a, w, num_cu, st, side);
+    glb_launch_bin<1>(a, w, num_cu, st, side);
+    glb_launch_bin<0>(a, w, num_cu, st, side);
+  }
   ss_join(w.ss, st);  // the call's stream waits for the side streams
   return hipGetLastError();
 }

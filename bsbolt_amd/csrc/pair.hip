@@ -48,55 +48,17 @@
 // 129-224 bases: 3.9M flanks of 2x150 bp reads 0.42 / 1.42 / 1.47 / 0.85 / 0.14
 // ms (was 1.16 / 3.5 / 5.0 / 2.5 / 0.33); 351,491 flanks of 250 bp reads 0.18 /
 // 0.49 / 0.86 / 1.19 / 2.39 ms (97 and longer: was 2.3 / 9.2).  Whole calls: 4.2
-// ms (was 11.9) and 3.6 ms (was 10.2).
-#include <type_traits>
-#include <utility>
-
+// ms (was 11.9) and 2.9 ms (was 10.2).
 #include "bsx_internal.h"
 #include "ext_common.h"
+#include "packed.h"
 
 namespace bsx {
-
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ u16x2 pk(uint32_t x) { return __builtin_bit_cast(u16x2, x); }
-__device__ __forceinline__ uint32_t pku(u16x2 x) { return __builtin_bit_cast(uint32_t, x); }
-__device__ __forceinline__ i16x2 pks(u16x2 x) { return __builtin_bit_cast(i16x2, x); }
-__device__ __forceinline__ u16x2 pkmax(u16x2 a, u16x2 b) { return __builtin_elementwise_max(a, b); }
-__device__ __forceinline__ u16x2 pkmin(u16x2 a, u16x2 b) { return __builtin_elementwise_min(a, b); }
-__device__ __forceinline__ u16x2 pksat(u16x2 a, u16x2 b) { return __builtin_elementwise_sub_sat(a, b); }
-__device__ __forceinline__ u16x2 pk2(int lo, int hi) { return pk((uint32_t)(lo & 0xffff) | (uint32_t)hi << 16); }
-__device__ __forceinline__ u16x2 splat(uint32_t x) { return pk(x | x << 16); }
-// 0xffff in every half whose signed value is negative
-__device__ __forceinline__ uint32_t negmask(u16x2 x) { return __builtin_bit_cast(uint32_t, pks(x) >> (int16_t)15); }
-__device__ __forceinline__ u16x2 sel(uint32_t m, u16x2 a, u16x2 b) { return pk((pku(a) & m) | (pku(b) & ~m)); }
-__device__ __forceinline__ u16x2 smax(u16x2 a, u16x2 b) {
-  return __builtin_bit_cast(u16x2, __builtin_elementwise_max(pks(a), pks(b)));
-}
-__device__ __forceinline__ u16x2 smin(u16x2 a, u16x2 b) {
-  return __builtin_bit_cast(u16x2, __builtin_elementwise_min(pks(a), pks(b)));
-}
-
-// A uniform constant in both halves whose value the compiler does not see: it
-// would turn min(x, 1) into a compare and a select per half, a multiply by a
-// power of two into shifts, and a chain of subtractions into one constant each.
-__device__ __forceinline__ u16x2 hidden(uint32_t x) {
-  uint32_t v = x | x << 16;
-  asm("" : "+s"(v));
-  return pk(v);
-}
 
 // x * e, at most 0xffff (x a column number below 2^14, e below 2^16)
 __device__ __forceinline__ u16x2 emul(u16x2 x, u16x2 e) {
   const uint32_t lo = (pku(x) & 0xffffu) * (pku(e) & 0xffffu), hi = (pku(x) >> 16) * (pku(e) >> 16);
   return pk(min(lo, 0xffffu) | min(hi, 0xffffu) << 16);
-}
-
-// f(0), f(1), ... with compile-time arguments (a loop this long is not unrolled)
-template <class F, int... I>
-__device__ __forceinline__ void for_each_index(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
 }
 
 // bitwise OR over the wave, as a scalar
@@ -110,21 +72,6 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   x |= __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return (uint32_t)__builtin_amdgcn_readlane(x, 63);
 }
-
-// One task of a lane while it is set up: aligned dword addresses of its
-// sequences (indices are clamped to the dwords that hold its bases).
-typedef const uint32_t __attribute__((address_space(1))) * gdword;
-struct PairSeq {
-  gdword p;
-  int sh, last;
-  __device__ __forceinline__ void set(const uint8_t* base, int len) {
-    const uintptr_t a = (uintptr_t)base;
-    p = (gdword)(a & ~(uintptr_t)3);
-    sh = (int)(a & 3);
-    last = (sh + (len > 0 ? len : 1) - 1) >> 2;
-  }
-  __device__ __forceinline__ uint32_t at(int d) const { return p[d < 0 ? 0 : d < last ? d : last]; }
-};
 
 // waves per SIMD the register budget leaves room for
 constexpr int pair_min_waves(int Q) { return Q <= 32 ? 3 : Q <= 96 ? 2 : 1; }
@@ -166,7 +113,7 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
   // ---- the lane's two tasks ----
   int task[2];
   int qlen[2], tlen[2], h0[2], w[2];
-  PairSeq ts[2];
+  DwordSeq ts[2];
   bool have[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -178,7 +125,7 @@ ext_pair_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
     const uint64_t qoff = (uint64_t)(uint32_t)y.z | (uint64_t)(uint32_t)y.w << 32;
     const uint64_t toff = (uint64_t)(uint32_t)z.x | (uint64_t)(uint32_t)z.y << 32;
     ts[k].set(tlen[k] > 0 ? A.target + toff : A.query + qoff, tlen[k]);
-    PairSeq qs;
+    DwordSeq qs;
     qs.set(A.query + qoff, qlen[k]);
     const int sh = qs.sh - ((8 - qlen[k]) & 7);  // byte of position 0 relative to the first dword
     const int d0 = sh >> 2, bs = sh & 3;
