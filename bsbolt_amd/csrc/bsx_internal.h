@@ -25,9 +25,12 @@ constexpr int kNarrowTasksPerBlock = 16;  // ... by one narrow-kernel block
 constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; }
 
 // The CIGAR (ksw_global2) kernel bins tasks the same way with its own shapes.
-constexpr int kGlbBins = 9;
+// A bin of its own for bands of 25-32 ((8,4)) lost: it is one launch more in a
+// chain of two on its stream (9,319 tasks of 150 bp reads: 417 us of kernels with
+// it, 307 without), and only 7% of the tasks have such a band.
+constexpr int kGlbBins = 8;
 constexpr BinShape kGlbShape[kGlbBins] = {
-    {8, 2}, {8, 3}, {8, 4}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
+    {8, 2}, {8, 3}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
 constexpr int kExtSlices = 8;  // fetch-counter slots per bin (CIGAR bins, lane frame classes)
 // Bins of the two-tasks-per-lane CIGAR kernel (gpair.hip), after the others:
 // band widths 2w+1 up to kGlbPairCols, each from glb_pair_top + 1 on.
@@ -58,10 +61,10 @@ __host__ __device__ constexpr int glb_key(int bin, int tlen) {
 __host__ __device__ constexpr int glb_pair_rows(int tlen) { return (tlen + 3) / 4 * 4; }
 // Smallest batch whose narrow bands run the pair kernel: below it the batch
 // takes the latency of its waves, and the group kernels finish sooner.  us per
-// call, pair / group kernels: 100 bp reads 64,000 tasks 911 / 684, 128,000 1029 /
-// 967, 300,000 1125 / 1711; 150 bp 64,000 1247 / 1133, 128,000 1333 / 1556; 250
-// bp 64,000 2691 / 2171, 128,000 2670 / 3078.
-constexpr int64_t kGlbPairMinTasks = 98304;
+// call, pair / group kernels: 100 bp reads 128,000 tasks 1026 / 721, 192,000 1068 /
+// 1030, 256,000 1088 / 1326; 150 bp 128,000 1329 / 1141, 192,000 1346 / 1621; 250
+// bp 128,000 2526 / 2757, 192,000 2553 / 3858.
+constexpr int64_t kGlbPairMinTasks = 131072;
 constexpr int glb_bin_limit(int b) { return kGlbShape[b].lanes * kGlbShape[b].cols; }
 // First entry of fetch slice s of a list of n entries: a balanced partition,
 // the first n % kExtSlices slices hold one entry more.
@@ -336,10 +339,6 @@ struct Reg2alnArgs {
 };
 hipError_t launch_reg2aln_cigar(const Reg2alnArgs& a, int num_cu, hipStream_t st);
 
-// Blocks per CU of the global kernel by lanes per task (8-lane shapes hold
-// twice the groups per block, so fewer blocks keep the scratch the same
-// size); the scratch holds one slot per group.
-constexpr int glb_blocks_per_cu(int lanes) { return lanes < 16 ? 4 : 7; }
 int64_t glb_groups(int num_cu, bool side);  // scratch slots, with or without the side-stream region
 void launch_glb_pair(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st);
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st);

@@ -19,6 +19,7 @@
 // rows: the group loads the next rows with all its lanes at once (one HBM
 // latency per window, not one per step) and every step then reads LDS.
 #include <algorithm>
+#include <type_traits>
 
 #include "bsx_internal.h"
 
@@ -112,18 +113,12 @@ glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase) {
   __shared__ uint2 s_prof[5];
   if (threadIdx.x < 5) s_prof[threadIdx.x] = make_uint2(A.prof_lo[threadIdx.x], (uint32_t)A.prof_hi[threadIdx.x]);
   __syncthreads();
-  // An empty bin returns before its first fetch (uniform over the grid): each
-  // wave's fetch is a device atomic on one address, ~10 ns apiece serialised.
-  if (nlist == 0) return;
-  for (;;) {
-    // Branch-free fetch: every lane issues the atomic (only lane 0 of the group
-    // adds 1; the compiler folds it into one atomic per wave).  No lane-divergent
-    // region may precede the broadcast: with `if (lig == 0)` around the atomic
-    // the compiler can give the other lanes a loop of their own that reaches
-    // the broadcast without lane 0's new value, and they never leave it.
-    const uint32_t mine = atomicAdd(W.fetch + bin, lig == 0 ? 1u : 0u);
-    const uint32_t idx = __shfl(mine, 0, L);
-    if (idx >= nlist) break;
+  // Every group's first task is its own number; only when the list is longer
+  // than the grid do groups fetch more (each wave's fetch is a device atomic on
+  // one address, ~10 ns apiece serialised, so an empty or short list has none).
+  const uint32_t groups = gridDim.x * (256 / L);
+  uint32_t idx = (uint32_t)group;
+  while (idx < nlist) {
     const int task = list[idx];
     const int qlen = A.qlen[task], tlen = A.tlen[task];
     // a band wider than both sequences is the same band (beg = 0, end = qlen
@@ -331,12 +326,20 @@ glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase) {
         const uint32_t zi = (uint32_t)i * (uint32_t)ncol + (uint32_t)kc;
         int zb;
         if (wrows >= 1) {
-          if (i < wlo || i > whi) {  // refill: rows [i - wrows + 1, i], every lane loading
+          // refill: rows [i - wrows + 1, i], every lane loading; all groups of the
+          // wave at once when one needs it, as the whole wave waits for each round
+          // trip to memory (8 groups on their own and a dword at a time: 200 us
+          // instead of 116 for the 8x2 bin of 9,319 tasks of 150 bp reads)
+          if (__any(i < wlo || i > whi)) {
             const int r0 = i - wrows + 1 > 0 ? i - wrows + 1 : 0;
             const uint32_t d0 = ((uint32_t)r0 * (uint32_t)ncol) >> 2;
             const uint32_t d1 = ((uint32_t)(i + 1) * (uint32_t)ncol - 1u) >> 2;
             __builtin_amdgcn_wave_barrier();
-            for (int q = lig; q <= (int)(d1 - d0); q += L) zwin[q] = zw[d0 + q];
+            uint32_t v[ZW / L];  // every load in flight before the first is stored
+#pragma unroll
+            for (int u = 0; u < ZW / L; ++u) v[u] = zw[min(d0 + lig + u * L, d1)];
+#pragma unroll
+            for (int u = 0; u < ZW / L; ++u) zwin[lig + u * L] = v[u];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -380,6 +383,14 @@ glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase) {
     } else if (A.n_cigar && lig == 0) {
       A.n_cigar[task] = 0;
     }
+    if (groups >= nlist) break;  // uniform over the grid
+    // Branch-free fetch: every lane issues the atomic (only lane 0 of the group
+    // adds 1; the compiler folds it into one atomic per wave).  No lane-divergent
+    // region may precede the broadcast: with `if (lig == 0)` around the atomic
+    // the compiler can give the other lanes a loop of their own that reaches
+    // the broadcast without lane 0's new value, and they never leave it.
+    const uint32_t mine = atomicAdd(W.fetch + bin, lig == 0 ? 1u : 0u);
+    idx = groups + __shfl(mine, 0, L);
   }
 }
 
@@ -487,52 +498,31 @@ __global__ void __launch_bounds__(1024) glb_reset_kernel(GlbWork W) {
   if (threadIdx.x == 0) W.err[1] = 0x7fffffff;
 }
 
+// Direction-byte slots per CU, one slot a group.  A launch uses the part given
+// to its stream; launches that run one after another share kGlbSlotsOne.
+struct GlbPart { int first, slots; };
+constexpr int kGlbSlotsOne = 128, kGlbSlots = 192;
+constexpr GlbPart kGlbAlone = {0, kGlbSlotsOne};
+constexpr GlbPart kGlbStreamPart[1 + StreamSet::kSide] = {{0, 64}, {64, 64}, {128, 32}, {160, 32}};
+static_assert(StreamSet::kSide == 3, "slot parts");
+// Streams of the bins in a batch without pair kernels.  Such a batch takes the
+// latency of its rows, 115-145 us a bin whatever its share of the tasks, so the
+// four bins that are seldom empty run beside each other, and the wide ones follow
+// where they wait for nobody.  With all of them on one stream but (16,4) the
+// call took 2-3 times as long (us, before / now): 100 bp reads 4,000 tasks 480 /
+// 179, 64,000 685 / 426; 150 bp 4,000 815 / 245, 64,000 1143 / 646; 250 bp 4,000
+// 1187 / 392, 64,000 2156 / 1598.
+constexpr int kGlbStream[kGlbBins] = {1, 0, 2, 3, 3, 3, 3, 3};
 
-// The 8x4 and 16x4 bins (bands 25-64 wide) hold about 1.5 tasks per group in
-// a CIGAR pass, so their kernels are mostly tail.  With side streams they run
-// beside the 8x2/8x3 bins on a side stream, with fewer blocks and a slot
-// region of their own after the main one.
-constexpr int kGlbSideBlocksPerCU = 2;
-constexpr bool glb_on_side(int b) { return b == 2 || b == 3; }
-
-constexpr int64_t glb_groups_per_cu(bool side) {
-  int64_t most = 0;
-  for (int b = 0; b < kGlbBins; ++b) {
-    if (glb_on_side(b) != side) continue;
-    const int bpc = side ? kGlbSideBlocksPerCU : glb_blocks_per_cu(kGlbShape[b].lanes);
-    const int64_t g = (int64_t)bpc * (256 / kGlbShape[b].lanes);
-    most = g > most ? g : most;
-  }
-  return most;
-}
-
-// with side streams off every bin runs on the call's stream at its own block
-// count, inside the main region
-constexpr int64_t glb_groups_per_cu_one_stream() {
-  int64_t most = 0;
-  for (int b = 0; b < kGlbBins; ++b) {
-    const int64_t g = (int64_t)glb_blocks_per_cu(kGlbShape[b].lanes) * (256 / kGlbShape[b].lanes);
-    most = g > most ? g : most;
-  }
-  return most;
-}
-static_assert(glb_groups_per_cu(false) >= glb_groups_per_cu_one_stream(), "main slot region covers every bin");
-
-int64_t glb_groups(int num_cu, bool side) {
-  // one direction-byte slot per group: the main region covers the largest grid
-  // of the call's stream (and every bin when side streams are off), the side
-  // region the side-stream grids
-  return (int64_t)num_cu * (glb_groups_per_cu(false) + (side ? glb_groups_per_cu(true) : 0));
-}
+int64_t glb_groups(int num_cu, bool side) { return (int64_t)num_cu * (side ? kGlbSlots : kGlbSlotsOne); }
 
 template <int B>
-static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t main, hipStream_t beside) {
+static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st, GlbPart part) {
   constexpr int L = kGlbShape[B].lanes, C = kGlbShape[B].cols;
-  const bool side = glb_on_side(B) && w.ss != nullptr;
-  const hipStream_t st = side ? beside : main;
-  const int bpc = side ? kGlbSideBlocksPerCU : glb_blocks_per_cu(L);
-  const int64_t zbase = side ? (int64_t)num_cu * glb_groups_per_cu(false) : 0;
-  hipLaunchKernelGGL((glb_kernel<L, C>), dim3((unsigned)(num_cu * bpc)), dim3(256), 0, st, a, w, B, zbase);
+  const int64_t room = std::min<int64_t>(part.slots / (256 / L), 7) * num_cu;
+  const int64_t blocks = std::min<int64_t>(room, (a.n * L + 255) / 256);
+  hipLaunchKernelGGL((glb_kernel<L, C>), dim3((unsigned)blocks), dim3(256), 0, st, a, w, B,
+                     (int64_t)part.first * num_cu);
 }
 
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) {
@@ -546,33 +536,34 @@ hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) 
   hipLaunchKernelGGL(glb_bin_offset_kernel, dim3(1), dim3(1024), 0, st, w);
   hipLaunchKernelGGL(glb_bin_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, w, (a.n + blocks - 1) / blocks);
   if (a.pair) {
-    // Only bin 4 (bands of 65-128) is likely to hold tasks beside the pair
+    // Only bin 3 (bands of 65-128) is likely to hold tasks beside the pair
     // bins.  The others go ahead of everything, 5 us each while the chip is
     // empty: behind a pair kernel, or beside one, even an empty launch waits
     // until there is room for its blocks (0.5-1.3 ms measured).
-    glb_launch_bin<8>(a, w, num_cu, st, st);
-    glb_launch_bin<7>(a, w, num_cu, st, st);
-    glb_launch_bin<6>(a, w, num_cu, st, st);
-    glb_launch_bin<5>(a, w, num_cu, st, st);
-    glb_launch_bin<3>(a, w, num_cu, st, st);
-    glb_launch_bin<2>(a, w, num_cu, st, st);
-    glb_launch_bin<1>(a, w, num_cu, st, st);
-    glb_launch_bin<0>(a, w, num_cu, st, st);
+    glb_launch_bin<7>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<6>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<5>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<4>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<2>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<1>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<0>(a, w, num_cu, st, kGlbAlone);
     ss_fork(w.ss, st);
-    glb_launch_bin<4>(a, w, num_cu, pick_stream(w.ss, st, 3), pick_stream(w.ss, st, 3));
+    glb_launch_bin<3>(a, w, num_cu, pick_stream(w.ss, st, 3), kGlbAlone);
     launch_glb_pair(a, w, num_cu, st);
   } else {
     ss_fork(w.ss, st);  // side streams start after the scatter
-    const hipStream_t side = pick_stream(w.ss, st, 1);
-    glb_launch_bin<3>(a, w, num_cu, st, side);
-    glb_launch_bin<2>(a, w, num_cu, st, side);
-    glb_launch_bin<8>(a, w, num_cu, st, side);
-    glb_launch_bin<7>(a, w, num_cu, st, side);
-    glb_launch_bin<6>(a, w, num_cu, st, side);
-    glb_launch_bin<5>(a, w, num_cu, st, side);
-    glb_launch_bin<4>(a, w, num_cu, st, side);
-    glb_launch_bin<1>(a, w, num_cu, st, side);
-    glb_launch_bin<0>(a, w, num_cu, st, side);
+    const auto beside = [&](auto bin) {
+      constexpr int B = decltype(bin)::value, k = kGlbStream[B];
+      glb_launch_bin<B>(a, w, num_cu, pick_stream(w.ss, st, k), w.ss ? kGlbStreamPart[k] : kGlbAlone);
+    };
+    beside(std::integral_constant<int, 1>());
+    beside(std::integral_constant<int, 2>());
+    beside(std::integral_constant<int, 0>());
+    beside(std::integral_constant<int, 3>());
+    beside(std::integral_constant<int, 7>());
+    beside(std::integral_constant<int, 6>());
+    beside(std::integral_constant<int, 5>());
+    beside(std::integral_constant<int, 4>());
   }
   ss_join(w.ss, st);  // the call's stream waits for the side streams
   return hipGetLastError();

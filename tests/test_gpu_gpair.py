@@ -8,7 +8,7 @@ from bsbolt_amd.tasks import GlbTasks
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
-PAIR_MIN = 98304
+PAIR_MIN = 131072
 
 
 def make_tasks(seed, n, qlens, bands, sub=0.05, gap=0.5, n_frac=0.0):
