@@ -43,7 +43,7 @@ EXPORTS = ("bsx_create", "bsx_destroy", "bsx_last_error", "bsx_set_stream", "bsx
 TIMED_SLOTS = 16
 # lanes per task and columns per lane of the plain form's query-length bins (bsx_internal.h
 # kExtShape); one lane per task is the two-tasks-per-lane kernel
-EXT_SHAPES = ((1, 32), (1, 64), (1, 96), (1, 128), (1, 224), (32, 8), (64, 8), (64, 16), (64, 32))
+EXT_SHAPES = ((1, 32), (1, 64), (1, 96), (1, 128), (1, 224), (64, 4), (64, 8), (64, 16), (64, 32))
 
 # learned-band form (include/bsx.h)
 BAND_PLAIN, BAND_LEARNED, BAND_FIXED = 0, 1, 2

@@ -399,6 +399,7 @@ static int ext_args(bsx_ctx* c, const bsx_scoring* sc, const bsx_ext_tasks* t, E
   a.query = t->query; a.q_off = t->q_off; a.qlen = t->qlen;
   a.target = t->target; a.t_off = t->t_off; a.tlen = t->tlen;
   a.h0 = t->h0; a.w = t->w; a.end_bonus = t->end_bonus;
+  a.qmax = INT_MAX;
   return BSX_OK;
 }
 

@@ -7,8 +7,9 @@ namespace bsx {
 
 // Extension work is split into bins by query length; each bin runs a kernel
 // instantiation.  Index = bin id.  Shape (1, Q) is the two-tasks-per-lane
-// kernel (pair.hip, queries of at most Q bases); shape (L, C) a group kernel
-// with L lanes per task and C query columns per lane (qlen <= L*C).  The bins
+// kernel (pair.hip, queries of at most Q bases); shape (64, C) the wave kernel
+// (wave.hip, queries or bands of at most 64*C columns); other shapes (L, C) a group
+// kernel with L lanes per task and C query columns per lane (qlen <= L*C).  The bins
 // from kQueryBins on take the queries of the pair bins where the pair kernel
 // does not run them: batches below kPairMinTasks and tasks outside its range
 // (pair_takes).
@@ -16,7 +17,7 @@ constexpr int kExtBins = 12;
 constexpr int kPairBins = 5;
 constexpr int kQueryBins = 9;  // bins told apart by query length alone
 struct BinShape { int lanes, cols; };
-constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}, {1, 224}, {32, 8},
+constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}, {1, 224}, {64, 4},
                                           {64, 8}, {64, 16}, {64, 32}, {16, 6},  {16, 8},  {32, 6}};
 constexpr int kExtBlock = 64;             // threads per extension block: one wave, so a block
                                           // never holds wave slots idle while a sibling finishes
@@ -125,13 +126,15 @@ constexpr int kPairMaxGapExt = 25;  // e * (tlen + Q), and the z-drop itself fit
 // reads, 0.8 ms for 150 bp); below this the group kernels, which spread a task
 // over 16 lanes, finish sooner.  us per call, pair / group kernels: 100 bp
 // 32,000 tasks 429 / 276, 64,000 451 / 431, 128,000 529 / 763; 150 bp 32,000
-// 810 / 555, 64,000 874 / 968, 128,000 1406 / 1869.
+// 810 / 555, 64,000 874 / 968, 128,000 1406 / 1869.  (Only the learned-band form
+// bins a batch of fewer than kDirectMaxTasks.)
 constexpr int64_t kPairMinTasks = 65536;
 
 // Kernel-side view of an extension batch (all pointers are device memory).
 struct ExtArgs {
   int o_del, e_del, o_ins, e_ins, zdrop, mat_max;
   bool pair;  // the batch's short queries may run the pair kernel
+  int qmax;   // no query is longer
   // Query profile by query code qc (0..4): bytes k=0..3 of prof_lo[qc] hold
   // mat[k*5+qc] (target code k), prof_hi[qc] holds mat[20+qc] (target N).
   uint32_t prof_lo[5];
@@ -259,6 +262,16 @@ struct ExtKArgs;
 // two-tasks-per-lane kernel of bin `bin` (query width Q), n tasks in the batch
 template <int Q>
 void launch_pair_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, hipStream_t st);
+// wave-per-task kernel of bin `bin`, 64 * C columns
+template <int C>
+void launch_wave_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st);
+// Largest batch that runs a wave per task without binning (wave.hip).  us per
+// call, so / binned, with pair kernels from 65,536 tasks on: 100 bp reads 500
+// tasks 60 / 154, 8,000 97 / 168, 32,000 182 / 278, 80,000 411 / 526, 128,000 703 /
+// 565; 150 bp 500 89 / 192, 32,000 278 / 573, 128,000 1044 / 1045; 250 bp 500 192 /
+// 330, 80,000 1521 / 2693, 128,000 2925 / 2741.
+constexpr int64_t kDirectMaxTasks = 98304;
+void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st);
 // lane-per-task frame kernel (frame of WF columns) of lane-frame class `cls`
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st);

@@ -110,6 +110,14 @@ __device__ __forceinline__ int ext_clamped_w(const ExtArgs& A, int64_t t) {
   return w < lim ? w : lim;
 }
 
+// Whether task t may run: the reference's preconditions and the score range of
+// the kernels.
+__device__ __forceinline__ bool ext_task_ok(const ExtArgs& A, int64_t t) {
+  const int ql = A.qlen[t], h0 = A.h0[t], eb = A.end_bonus[t];
+  return ql >= 1 && ql <= bin_limit(kQueryBins - 1) && A.tlen[t] >= 0 && h0 >= 1 && A.w[t] >= 0 && eb > -kScoreLimit &&
+         eb < kScoreLimit && (int64_t)h0 + (int64_t)ql * A.mat_max < kScoreLimit;
+}
+
 // 48-byte work-list descriptor of task t (clamped band included).
 __device__ __forceinline__ void write_desc(const ExtArgs& A, int64_t t, ExtDesc* dst) {
   const uint64_t qo = A.q_off[t], to = A.t_off[t];

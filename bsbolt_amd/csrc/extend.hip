@@ -1,6 +1,10 @@
 // Bit-exact batched ksw_extend2 (bsbolt/External/BWA/ksw.c:380-479) for gfx950.
 //
-// Layout.  A task is owned by a group of L lanes (L = 16, 32 or 64; 64/L tasks
+// This file holds the group kernel, for queries of up to 192 bases in batches or
+// tasks that the pair kernel (pair.hip) does not take; the wave kernel (wave.hip)
+// takes longer ones and small batches.
+//
+// Layout.  A task is owned by a group of L lanes (L = 16 or 32; 64/L tasks
 // per wave64); lane g holds query columns [g*C, g*C+C) of the DP state in VGPRs:
 //   G[c] = eh[j].h = H(i-1, j-1)   (diagonal predecessor)
 //   E[c] = eh[j].e = E(i, j)
@@ -25,7 +29,7 @@
 // columns >= end, and G(j) = H(i, j-1) holds for every j <= end with
 // H(i, -1) = the first-column value of ksw.c:421-424.
 //
-// Work distribution.  Tasks are binned by query length (bin b: qlen <= L*C);
+// Work distribution.  Tasks are binned by their columns (ext_bin_of);
 // the binning pass writes one 48-byte descriptor per task in bin order.  Block
 // k of a bin's launch owns descriptors [k*T, k*T+T); its groups take them one
 // at a time through an LDS counter, so no device-scope atomic is on the task
@@ -46,7 +50,7 @@ namespace bsx {
 
 
 // waves per SIMD the register budget must allow (4 keeps VGPRs <= 128)
-constexpr int plain_min_waves(int C) { return C <= 6 ? 4 : C <= 8 ? 3 : C <= 16 ? 2 : 1; }
+constexpr int plain_min_waves(int C) { return C <= 6 ? 4 : 3; }
 
 template <int L, int C, bool E1>
 __global__ void __launch_bounds__(kExtBlock, plain_min_waves(C))
@@ -343,11 +347,17 @@ ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_
 
 // ---- binning: validate every task, group tasks by query length, write descriptors ----
 
-__device__ __forceinline__ int ext_bin_of(int qlen) {
+// Bin of a task by its query, or by its band where that is narrower (the wave
+// kernels' frame needs 2w + 1 + C columns).
+__device__ __forceinline__ int ext_bin_of(const ExtArgs& A, int64_t t, int qlen) {
 #pragma unroll
-  for (int b = 0; b < kQueryBins; ++b)
+  for (int b = 0; b <= kPairBins; ++b)
     if (qlen <= bin_limit(b)) return b;
-  return -1;
+  const int w = ext_clamped_w(A, t);
+#pragma unroll
+  for (int b = kPairBins; b < kQueryBins - 1; ++b)
+    if (qlen <= bin_limit(b) || 2 * (int64_t)w + 1 + kExtShape[b].cols <= bin_limit(b)) return b;
+  return kQueryBins - 1;
 }
 
 // Bin of a task the pair kernel does not take.
@@ -388,15 +398,14 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
       }
       continue;
     }
-    const int ql = A.qlen[t], tl = A.tlen[t], h0 = A.h0[t], w = A.w[t], eb = A.end_bonus[t];
-    int b = ext_bin_of(ql);
-    const bool ok = ql >= 1 && tl >= 0 && h0 >= 1 && w >= 0 && b >= 0 && eb > -kScoreLimit &&
-                    eb < kScoreLimit && (int64_t)h0 + (int64_t)ql * A.mat_max < kScoreLimit;
-    if (!ok) {
+    const int ql = A.qlen[t], tl = A.tlen[t], h0 = A.h0[t];
+    int b;
+    if (!ext_task_ok(A, t)) {
       b = 0xff;
       ++bad;
       first_bad = min(first_bad, (int)t);
     } else {
+      b = ext_bin_of(A, t, ql);
       if (b < kPairBins && !pair_takes(A, b, ql, tl, h0)) b = ext_group_bin_of(ql);
       if (mode == 0) {
         atomicAdd(&hist[b], 1u);
@@ -485,8 +494,7 @@ ext_unpack_kernel(ExtArgs A, ExtWork W, const int32_t* __restrict__ rec) {
 // surplus blocks exit at once (the host does not know the bin's count).  The
 // tuned tpb suits batches that fill the chip; below that a block takes only as
 // many tasks as leave every SIMD kBlocksPerSimd blocks, at least one per group:
-// with 32 per block, 4,001 flanks of 2 kb reads ran in 125 blocks (174 ms, now
-// 10.6) and 500 flanks of 150 bp reads in 16 (1.11 ms, now 0.24).
+// with 32 per block, 500 flanks of 150 bp reads ran in 16 (1.11 ms, so 0.24).
 template <int L, int C, bool E1>
 static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st) {
   constexpr int64_t kBlocksPerSimd = 4, kMaxBlocksPerCu = 128;
@@ -505,6 +513,8 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
   constexpr int L = kExtShape[B].lanes, C = kExtShape[B].cols;
   if constexpr (B < kPairBins) {
     if (pair) launch_pair_bin<C>(k, wk, B, n, st);
+  } else if constexpr (B < kQueryBins) {
+    launch_wave_bin<C>(k, wk, B, n, num_cu, st);
   } else if constexpr (B == kTunedBin[0] || B == kTunedBin[1]) {
     constexpr int V = B == kTunedBin[0] ? 0 : 1;
     if (wk.shape_var[V] == 1)
@@ -533,12 +543,16 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   a.pair = a.n >= kPairMinTasks && a.e_del <= kPairMaxGapExt && a.e_ins <= kPairMaxGapExt;
   hipLaunchKernelGGL(ext_reset_kernel, dim3(1), dim3(256), 0, st, wk, kExtCounterWords);
   if (a.n <= 0) return hipGetLastError();
+  const bool band = plan && plan->mode != kBandPlain;
+  if (a.n <= kDirectMaxTasks && !band && !wk.tev) {  // timed calls time the bins
+    launch_direct(a, wk, num_cu, st);
+    return hipGetLastError();
+  }
   int64_t blocks = (a.n + 255) / 256;  // unpack pass
   if (blocks > (int64_t)num_cu * 16) blocks = (int64_t)num_cu * 16;
   // count and scatter passes: each block ends with one global atomic per
   // non-empty bin and row bucket, so fewer, larger blocks
   const int64_t sblocks = blocks < (int64_t)num_cu * 4 ? blocks : (int64_t)num_cu * 4;
-  const bool band = plan && plan->mode != kBandPlain;
   ExtKArgs k{};
   k.query = a.query; k.target = a.target; k.rec = wk.rec;
   k.o_del = a.o_del; k.e_del = a.e_del; k.o_ins = a.o_ins; k.e_ins = a.e_ins; k.zdrop = a.zdrop;

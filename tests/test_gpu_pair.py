@@ -10,7 +10,7 @@ from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 FIELDS = ("score", "qle", "tle", "gtle", "gscore", "max_off", "cells")
-PAIR_MIN = 65536
+PAIR_MIN = 98305
 
 
 def make_tasks(seed, qlens, n, h0, w, eb=(0, 5, 30), tail=(0, 1, 40), sub=0.03, n_frac=0.0, tlen=None):
