@@ -2,6 +2,7 @@
 // host<->device staging, and dispatch to the extension / global kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <dlfcn.h>
 #include <cstdarg>
@@ -51,6 +52,28 @@ struct DevBuf {
   }
 };
 
+// Grow-only pinned host buffer; d is its address on the device.
+struct PinBuf {
+  void *p = nullptr, *d = nullptr;
+  size_t cap = 0;
+  hipError_t ensure(size_t bytes) {
+    if (bytes <= cap) return hipSuccess;
+    release();
+    const size_t want = bytes + bytes / 4 + 4096;
+    hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
+    if (e != hipSuccess) { p = nullptr; return e; }
+    e = hipHostGetDevicePointer(&d, p, 0);
+    if (e != hipSuccess) { release(); return e; }
+    cap = want;
+    return hipSuccess;
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = d = nullptr;
+    cap = 0;
+  }
+};
+
 }  // namespace
 
 // Device workspace of the batch entry points.  A context has its own; a
@@ -89,7 +112,8 @@ struct bsx_ctx {
   int kt_calls = 0, kt_used = 0;
   int64_t zslot = 1 << 16;     // bytes per slot: largest min(qlen,2w+1)*tlen accepted
   // staging for the host-memory entry points
-  DevBuf h_query, h_target, h_qoff, h_toff, h_i32, h_res;
+  DevBuf h_in, h_res;
+  PinBuf p_in, p_out;
   int32_t* err_host = nullptr;  // pinned: [0]=rejected count, [1]=first rejected index
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool pending_check = false;
@@ -288,7 +312,9 @@ void bsx_destroy(bsx_ctx* c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   c->wown.release();
-  for (DevBuf* b : {&c->h_query, &c->h_target, &c->h_qoff, &c->h_toff, &c->h_i32, &c->h_res, &c->stats, &c->model,
+  c->p_in.release();
+  c->p_out.release();
+  for (DevBuf* b : {&c->h_in, &c->h_res, &c->stats, &c->model,
                     &c->part, &c->grad})
     b->release();
   for (hipEvent_t e : c->kt_ev) (void)hipEventDestroy(e);
@@ -677,84 +703,123 @@ int bsx_band_train_device(bsx_ctx* c, const uint16_t* feats, const uint8_t* labe
   return BSX_OK;
 }
 
+// Host arrays of a batch call on their way to the device.
+struct HostIn {
+  const void* src;
+  size_t bytes;
+  void* dev;  // set by host_in
+};
+
+// Arrays of up to kStageEach bytes are gathered in pinned memory and copied at
+// once, as a copy costs 12-17 us of calls whatever its size; larger ones are
+// copied from where they lie, which the runtime does at the bus's rate.  A batch
+// that the kernel reads but once and that fits kInPlace is read over the bus.
+constexpr size_t kStageEach = 256 << 10, kInPlace = 32 << 10;
+
+static int host_in(bsx_ctx* c, HostIn* in, int k, bool once) {
+  size_t staged = 0, total = 0;
+  for (int x = 0; x < k; ++x)
+    if (in[x].bytes <= kStageEach) staged += align_up(in[x].bytes);
+    else total += align_up(in[x].bytes);
+  HIPCHK(c, c->p_in.ensure(staged), "hipHostMalloc(input)");
+  const bool in_place = once && total == 0 && staged <= kInPlace;
+  if (!in_place) HIPCHK(c, c->h_in.ensure(staged + total), "hipMalloc(input)");
+  char* base = in_place ? (char*)c->p_in.d : (char*)c->h_in.p;
+  size_t at = 0, big = staged;
+  for (int x = 0; x < k; ++x) {
+    if (in[x].bytes <= kStageEach) {
+      if (in[x].bytes) memcpy((char*)c->p_in.p + at, in[x].src, in[x].bytes);
+      in[x].dev = base + at;
+      at += align_up(in[x].bytes);
+    } else {
+      in[x].dev = base + big;
+      HIPCHK(c, hipMemcpyAsync(in[x].dev, in[x].src, in[x].bytes, hipMemcpyHostToDevice, c->stream), "H2D input");
+      big += align_up(in[x].bytes);
+    }
+  }
+  if (!in_place && staged)
+    HIPCHK(c, hipMemcpyAsync(base, c->p_in.p, staged, hipMemcpyHostToDevice, c->stream), "H2D input");
+  return BSX_OK;
+}
+
 int bsx_extend_batch(bsx_ctx* c, const bsx_scoring* sc, const bsx_ext_tasks* t, bsx_ext_results* r) {
   if (!c || !t || !r) return fail(c, BSX_EINVAL, "NULL argument");
-  int rc = check_scoring(c, sc);
+  ExtArgs a;
+  int rc = ext_args(c, sc, t, a);
   if (rc) return rc;
-  if (t->n < 0 || t->n > INT_MAX) return fail(c, BSX_EINVAL, "n must be in [0, 2^31-1]");
   const size_t n = (size_t)t->n;
   if (n == 0) return BSX_OK;
-  if (!t->query || !t->q_off || !t->qlen || !t->target || !t->t_off || !t->tlen || !t->h0 || !t->w ||
-      !t->end_bonus)
-    return fail(c, BSX_EINVAL, "task arrays must not be NULL");
   // extent of the sequence buffers actually referenced
   uint64_t qext = 0, text = 0;
+  int qmax = 0;
   for (size_t k = 0; k < n; ++k) {
     if (t->qlen[k] > 0 && t->q_off[k] + (uint64_t)t->qlen[k] > qext) qext = t->q_off[k] + t->qlen[k];
     if (t->tlen[k] > 0 && t->t_off[k] + (uint64_t)t->tlen[k] > text) text = t->t_off[k] + t->tlen[k];
+    qmax = t->qlen[k] > qmax ? t->qlen[k] : qmax;
   }
   (void)hipSetDevice(c->device);
-  HIPCHK(c, c->h_query.ensure(qext + 1), "hipMalloc(query)");
-  HIPCHK(c, c->h_target.ensure(text + 1), "hipMalloc(target)");
-  HIPCHK(c, c->h_qoff.ensure(8 * n), "hipMalloc(q_off)");
-  HIPCHK(c, c->h_toff.ensure(8 * n), "hipMalloc(t_off)");
-  HIPCHK(c, c->h_i32.ensure(5 * 4 * n), "hipMalloc(task ints)");
-  HIPCHK(c, c->h_res.ensure(8 * 4 * n + 8 * n), "hipMalloc(results)");
   hipStream_t st = c->stream;
-  uint8_t* dq = (uint8_t*)c->h_query.p;
-  uint8_t* dt = (uint8_t*)c->h_target.p;
-  int32_t* di = (int32_t*)c->h_i32.p;
-  if (qext) HIPCHK(c, hipMemcpyAsync(dq, t->query, qext, hipMemcpyHostToDevice, st), "H2D query");
-  if (text) HIPCHK(c, hipMemcpyAsync(dt, t->target, text, hipMemcpyHostToDevice, st), "H2D target");
-  HIPCHK(c, hipMemcpyAsync(c->h_qoff.p, t->q_off, 8 * n, hipMemcpyHostToDevice, st), "H2D q_off");
-  HIPCHK(c, hipMemcpyAsync(c->h_toff.p, t->t_off, 8 * n, hipMemcpyHostToDevice, st), "H2D t_off");
-  const int32_t* src[5] = {t->qlen, t->tlen, t->h0, t->w, t->end_bonus};
-  for (int k = 0; k < 5; ++k)
-    HIPCHK(c, hipMemcpyAsync(di + k * n, src[k], 4 * n, hipMemcpyHostToDevice, st), "H2D task ints");
-  bsx_ext_tasks dtk{(int64_t)n, dq, (const uint64_t*)c->h_qoff.p, di, dt, (const uint64_t*)c->h_toff.p,
-                    di + n, di + 2 * n, di + 3 * n, di + 4 * n};
-  int32_t* dr = (int32_t*)c->h_res.p;
-  int32_t* outs[6] = {r->score, r->qle, r->tle, r->gtle, r->gscore, r->max_off};
-  bsx_ext_results drs{};
-  int32_t** dslots[6] = {&drs.score, &drs.qle, &drs.tle, &drs.gtle, &drs.gscore, &drs.max_off};
-  for (int k = 0; k < 6; ++k) *dslots[k] = outs[k] ? dr + k * n : nullptr;
-  drs.cells = r->cells ? (int64_t*)(dr + 8 * n) : nullptr;
-  rc = bsx_extend_batch_device(c, sc, &dtk, &drs);
+  const bool direct = n <= (size_t)kDirectMaxTasks && c->band_policy == BSX_BAND_PLAIN && c->kt_used >= c->kt_calls;
+  HostIn in[9] = {{t->query, (size_t)qext, nullptr}, {t->target, (size_t)text, nullptr},
+                  {t->q_off, 8 * n, nullptr}, {t->t_off, 8 * n, nullptr}, {t->qlen, 4 * n, nullptr},
+                  {t->tlen, 4 * n, nullptr}, {t->h0, 4 * n, nullptr}, {t->w, 4 * n, nullptr},
+                  {t->end_bonus, 4 * n, nullptr}};
+  rc = host_in(c, in, 9, direct);
   if (rc) return rc;
+  a.query = (const uint8_t*)in[0].dev; a.target = (const uint8_t*)in[1].dev;
+  a.q_off = (const uint64_t*)in[2].dev; a.t_off = (const uint64_t*)in[3].dev;
+  a.qlen = (const int32_t*)in[4].dev; a.tlen = (const int32_t*)in[5].dev; a.h0 = (const int32_t*)in[6].dev;
+  a.w = (const int32_t*)in[7].dev; a.end_bonus = (const int32_t*)in[8].dev;
+  a.qmax = qmax;
+  constexpr size_t kChunk = 131072;  // records per copy to the host
+  HIPCHK(c, c->p_out.ensure(32 * (n < kChunk ? n : kChunk)), "hipHostMalloc(results)");
+  std::vector<uint8_t> bin;  // of a binned batch with rejected tasks
+  ExtWork wk = ext_work(c);
+  if (direct) {
+    a.rec_out = (int32_t*)c->p_out.d;
+    launch_direct(a, wk, c->num_cu, st);
+    HIPCHK(c, hipGetLastError(), "extension launch");
+    c->last_n = 0;
+  } else {
+    rc = ext_buffers(c, n);
+    if (rc) return rc;
+    if (c->band_policy == BSX_BAND_LEARNED) HIPCHK(c, c->ws->cls.ensure(n + 1), "hipMalloc(cls)");
+    wk = ext_work(c);
+    rc = extend_queue(c, a, wk, (uint8_t*)c->ws->cls.p);
+    if (rc) return rc;
+  }
   HIPCHK(c, hipStreamSynchronize(st), "hipStreamSynchronize");
   c->pending_check = false;
-  const int rejected = c->err_host[0];
-  std::vector<uint8_t> ok;
-  if (rejected > 0) {  // copy back only the tasks that ran; rejected slots stay untouched
-    ok.resize(n);
-    HIPCHK(c, hipMemcpy(ok.data(), c->ws->bin_of.p, n, hipMemcpyDeviceToHost), "D2H bin_of");
+  if (!direct && c->err_host[0] > 0) {  // rejected slots stay untouched
+    bin.resize(n);
+    HIPCHK(c, hipMemcpy(bin.data(), c->ws->bin_of.p, n, hipMemcpyDeviceToHost), "D2H bin_of");
   }
-  std::vector<int32_t> tmp;
-  std::vector<int64_t> tmp64;
-  for (int k = 0; k < 6; ++k) {
-    if (!outs[k]) continue;
-    if (rejected == 0) {
-      HIPCHK(c, hipMemcpy(outs[k], dr + k * n, 4 * n, hipMemcpyDeviceToHost), "D2H results");
-    } else {
-      tmp.resize(n);
-      HIPCHK(c, hipMemcpy(tmp.data(), dr + k * n, 4 * n, hipMemcpyDeviceToHost), "D2H results");
-      for (size_t q = 0; q < n; ++q)
-        if (ok[q] != 0xff) outs[k][q] = tmp[q];
+  size_t rejected = 0, first = 0;
+  for (size_t q0 = 0; q0 < n; q0 += kChunk) {
+    const size_t m = n - q0 < kChunk ? n - q0 : kChunk;
+    if (!direct) {
+      HIPCHK(c, hipMemcpyAsync(c->p_out.p, wk.rec + 8 * q0, 32 * m, hipMemcpyDeviceToHost, st), "D2H results");
+      HIPCHK(c, hipStreamSynchronize(st), "hipStreamSynchronize");
     }
-  }
-  if (r->cells) {
-    if (rejected == 0) {
-      HIPCHK(c, hipMemcpy(r->cells, drs.cells, 8 * n, hipMemcpyDeviceToHost), "D2H cells");
-    } else {
-      tmp64.resize(n);
-      HIPCHK(c, hipMemcpy(tmp64.data(), drs.cells, 8 * n, hipMemcpyDeviceToHost), "D2H cells");
-      for (size_t q = 0; q < n; ++q)
-        if (ok[q] != 0xff) r->cells[q] = tmp64[q];
+    const int32_t* rec = (const int32_t*)c->p_out.p;
+    for (size_t k = 0; k < m; ++k, rec += 8) {
+      const size_t q = q0 + k;
+      if (direct ? rec[7] == 0 : !bin.empty() && bin[q] == 0xff) {
+        if (!rejected++) first = q;
+        continue;
+      }
+      if (r->score) r->score[q] = rec[0];
+      if (r->qle) r->qle[q] = rec[1];
+      if (r->tle) r->tle[q] = rec[2];
+      if (r->gtle) r->gtle[q] = rec[3];
+      if (r->gscore) r->gscore[q] = rec[4];
+      if (r->max_off) r->max_off[q] = rec[5];
+      if (r->cells) r->cells[q] = (int64_t)(uint32_t)rec[6];
     }
   }
   if (rejected > 0)
-    return fail(c, BSX_EINVAL, "%d task(s) rejected (precondition violated); first is task %d", rejected,
-                c->err_host[1]);
+    return fail(c, BSX_EINVAL, "%d task(s) rejected (precondition violated); first is task %d", (int)rejected,
+                (int)first);
   return BSX_OK;
 }
 
@@ -931,28 +996,19 @@ int bsx_global_batch(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tasks* t, 
   }
   (void)hipSetDevice(c->device);
   const size_t slot = r->cigar ? (size_t)r->cigar_slot : 0;
-  HIPCHK(c, c->h_query.ensure(qext + 1), "hipMalloc(query)");
-  HIPCHK(c, c->h_target.ensure(text + 1), "hipMalloc(target)");
-  HIPCHK(c, c->h_qoff.ensure(8 * n), "hipMalloc(q_off)");
-  HIPCHK(c, c->h_toff.ensure(8 * n), "hipMalloc(t_off)");
-  HIPCHK(c, c->h_i32.ensure(3 * 4 * n), "hipMalloc(task ints)");
   HIPCHK(c, c->h_res.ensure(2 * 4 * n + 4 * n * slot), "hipMalloc(results)");
   hipStream_t st = c->stream;
-  uint8_t* dq = (uint8_t*)c->h_query.p;
-  uint8_t* dt = (uint8_t*)c->h_target.p;
-  int32_t* di = (int32_t*)c->h_i32.p;
-  if (qext) HIPCHK(c, hipMemcpyAsync(dq, t->query, qext, hipMemcpyHostToDevice, st), "H2D query");
-  if (text) HIPCHK(c, hipMemcpyAsync(dt, t->target, text, hipMemcpyHostToDevice, st), "H2D target");
-  HIPCHK(c, hipMemcpyAsync(c->h_qoff.p, t->q_off, 8 * n, hipMemcpyHostToDevice, st), "H2D q_off");
-  HIPCHK(c, hipMemcpyAsync(c->h_toff.p, t->t_off, 8 * n, hipMemcpyHostToDevice, st), "H2D t_off");
-  const int32_t* src[3] = {t->qlen, t->tlen, t->w};
-  for (int k = 0; k < 3; ++k)
-    HIPCHK(c, hipMemcpyAsync(di + k * n, src[k], 4 * n, hipMemcpyHostToDevice, st), "H2D task ints");
-  bsx_glb_tasks dtk{(int64_t)n, dq, (const uint64_t*)c->h_qoff.p, di, dt, (const uint64_t*)c->h_toff.p,
-                    di + n, di + 2 * n};
+  HostIn in[7] = {{t->query, (size_t)qext, nullptr}, {t->target, (size_t)text, nullptr}, {t->q_off, 8 * n, nullptr},
+                  {t->t_off, 8 * n, nullptr}, {t->qlen, 4 * n, nullptr}, {t->tlen, 4 * n, nullptr},
+                  {t->w, 4 * n, nullptr}};
+  rc = host_in(c, in, 7, false);
+  if (rc) return rc;
+  bsx_glb_tasks dtk{(int64_t)n, (const uint8_t*)in[0].dev, (const uint64_t*)in[2].dev, (const int32_t*)in[4].dev,
+                    (const uint8_t*)in[1].dev, (const uint64_t*)in[3].dev, (const int32_t*)in[5].dev,
+                    (const int32_t*)in[6].dev};
   int32_t* dr = (int32_t*)c->h_res.p;
-  bsx_glb_results drs{r->score ? dr : nullptr, r->n_cigar ? dr + n : nullptr,
-                      r->cigar ? (uint32_t*)(dr + 2 * n) : nullptr, r->cigar_slot};
+  bsx_glb_results drs{dr, r->n_cigar ? dr + n : nullptr, r->cigar ? (uint32_t*)(dr + 2 * n) : nullptr,
+                      r->cigar_slot};
   // The host sees every task's size, so the direction slot is sized for this
   // batch: raised (for this call only) to the largest min(qlen, 2w+1) * tlen,
   // within a scratch budget of kZslotHostMax bytes per slot.
@@ -969,22 +1025,44 @@ int bsx_global_batch(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tasks* t, 
   rc = bsx_global_batch_device(c, sc, &dtk, &drs);
   c->zslot = zslot0;
   if (rc) return rc;
-  HIPCHK(c, hipStreamSynchronize(st), "hipStreamSynchronize");
+  // The kernels leave every CIGAR in its slot, which is far larger than most (300
+  // words for 150 bp reads, of which 3 are used): another gathers the used words
+  // in pinned memory, in chunks of tasks that fit it.
+  constexpr size_t kChunk = 65536, kWords = 1 << 20;
+  const size_t most = n < kChunk ? n : kChunk;
+  const size_t room = std::min<size_t>(kWords, most * std::min<size_t>(slot, 16));
+  HIPCHK(c, c->p_out.ensure(16 * most + 4 * room), "hipHostMalloc(results)");
+  const int32_t* rec = (const int32_t*)c->p_out.p;
+  const uint32_t* words = (const uint32_t*)((const char*)c->p_out.p + 16 * most);
+  const uint8_t* bin_of = (const uint8_t*)c->ws->bin_of.p;
+  uint32_t* used = (uint32_t*)c->ws->small.p + kGlbGatherWord;
+  for (size_t q0 = 0; q0 < n; q0 += kChunk) {
+    const size_t m = n - q0 < kChunk ? n - q0 : kChunk;
+    HIPCHK(c, launch_glb_gather(drs.score + q0, drs.n_cigar ? drs.n_cigar + q0 : nullptr,
+                                drs.cigar ? drs.cigar + q0 * slot : nullptr, bin_of + q0, (int)m, (int64_t)slot,
+                                (int32_t*)c->p_out.d, (uint32_t*)((char*)c->p_out.d + 16 * most), (uint32_t)room, used,
+                                q0 > 0, st),
+           "gather launch");
+    HIPCHK(c, hipStreamSynchronize(st), "hipStreamSynchronize");
+    std::vector<uint32_t> slots;  // of a chunk with CIGARs that the room did not hold
+    bool all = true;
+    for (size_t k = 0; k < m; ++k) all = all && (rec[4 * k + 1] <= 0 || rec[4 * k + 2] >= 0);
+    if (!all && r->cigar) {
+      slots.resize(m * slot);
+      HIPCHK(c, hipMemcpy(slots.data(), drs.cigar + q0 * slot, 4 * m * slot, hipMemcpyDeviceToHost), "D2H cigar");
+    }
+    for (size_t k = 0; k < m; ++k) {
+      const size_t q = q0 + k;
+      const int32_t nc = rec[4 * k + 1], at = rec[4 * k + 2];
+      if (!rec[4 * k + 3]) continue;  // rejected: its slots stay untouched
+      if (r->score) r->score[q] = rec[4 * k];
+      if (r->n_cigar) r->n_cigar[q] = nc;
+      if (!r->cigar || nc <= 0) continue;
+      memcpy(r->cigar + q * slot, at >= 0 ? words + at : slots.data() + k * slot, 4 * (size_t)nc);
+    }
+  }
   c->pending_check = false;
   const int rejected = c->err_host[0], overflow = c->err_host[2];
-  std::vector<uint8_t> ok(n, 0);
-  if (rejected > 0) HIPCHK(c, hipMemcpy(ok.data(), c->ws->bin_of.p, n, hipMemcpyDeviceToHost), "D2H bin_of");
-  std::vector<int32_t> sco(n), ncg(n);
-  std::vector<uint32_t> cg(n * slot);
-  if (r->score) HIPCHK(c, hipMemcpy(sco.data(), drs.score, 4 * n, hipMemcpyDeviceToHost), "D2H score");
-  if (r->n_cigar) HIPCHK(c, hipMemcpy(ncg.data(), drs.n_cigar, 4 * n, hipMemcpyDeviceToHost), "D2H n_cigar");
-  if (r->cigar) HIPCHK(c, hipMemcpy(cg.data(), drs.cigar, 4 * n * slot, hipMemcpyDeviceToHost), "D2H cigar");
-  for (size_t q = 0; q < n; ++q) {
-    if (ok[q] == 0xff) continue;
-    if (r->score) r->score[q] = sco[q];
-    if (r->n_cigar) r->n_cigar[q] = ncg[q];
-    if (r->cigar && ncg[q] > 0) memcpy(r->cigar + q * slot, cg.data() + q * slot, 4 * (size_t)ncg[q]);
-  }
   if (rejected > 0)
     return fail(c, BSX_EINVAL, "%d task(s) rejected (precondition violated); first is task %d", rejected,
                 c->err_host[1]);

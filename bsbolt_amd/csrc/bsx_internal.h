@@ -151,6 +151,7 @@ struct ExtArgs {
   const int32_t* end_bonus;
   int32_t *score, *qle, *tle, *gtle, *gscore, *max_off;
   int64_t* cells;
+  int32_t* rec_out;  // unbinned batches: [n][8] results as in ExtWork::rec, word 7 = 1 (0: rejected), instead
 };
 
 // One task of a bin's work list (written by the binning pass, in bin order).
@@ -354,6 +355,13 @@ hipError_t launch_reg2aln_cigar(const Reg2alnArgs& a, int num_cu, hipStream_t st
 
 int64_t glb_groups(int num_cu, bool side);  // scratch slots, with or without the side-stream region
 void launch_glb_pair(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st);
+// Copies the results of n tasks into pinned memory: rec[n][4] = score, n_cigar,
+// first word of the CIGAR in `words` (-1: not there), 1 (0: rejected).  At most
+// 2^20 tasks a call.
+hipError_t launch_glb_gather(const int32_t* score, const int32_t* n_cigar, const uint32_t* cigar, const uint8_t* bin_of,
+                             int n, int64_t slot, int32_t* rec, uint32_t* words, uint32_t room, uint32_t* used,
+                             bool clear, hipStream_t st);
+constexpr int kGlbGatherWord = kCountSlots;  // its counter, cleared with the call's: cursor[0]
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st);
 // counters of a CIGAR call: counts, cursor, err[4], fetch, kcount, kcursor
 constexpr int kGlbCounterWords = 2 * kCountSlots + 4 + kFetchSlots + 2 * kGlbKeys;

@@ -78,8 +78,8 @@ struct ExtKArgs {
 // The eight result words of a task (ksw.c:473-478 plus the cell count), one
 // word per lane of the group (two per lane for L = 4).
 template <int L>
-__device__ __forceinline__ void write_rec(int32_t* rec, int task, int lig, int best, int qle, int tle, int gtle,
-                                          int gscore, int moff, uint32_t ncell) {
+__device__ __forceinline__ void write_rec(int32_t* rec, int64_t task, int lig, int best, int qle, int tle, int gtle,
+                                          int gscore, int moff, uint32_t ncell, int last = 0) {
   constexpr int S = L < 8 ? L : 8;
 #pragma unroll
   for (int r = 0; r < 8; r += S) {
@@ -92,8 +92,8 @@ __device__ __forceinline__ void write_rec(int32_t* rec, int task, int lig, int b
       v = f == 4 ? gscore : v;
       v = f == 5 ? moff : v;
       v = f == 6 ? (int)ncell : v;
-      v = f == 7 ? 0 : v;
-      rec[(int64_t)task * 8 + f] = v;
+      v = f == 7 ? last : v;
+      rec[task * 8 + f] = v;
     }
   }
 }

@@ -583,7 +583,9 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   if (a.e_del == 1 && a.e_ins == 1) launch_bins<true>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
   else launch_bins<false>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
   ss_join(wk.ss, st);
-  hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
+  if (a.score || a.qle || a.tle || a.gtle || a.gscore || a.max_off || a.cells)
+    hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk,
+                       (const int32_t*)wk.rec);
   return hipGetLastError();
 }
 

@@ -498,6 +498,42 @@ __global__ void __launch_bounds__(1024) glb_reset_kernel(GlbWork W) {
   if (threadIdx.x == 0) W.err[1] = 0x7fffffff;
 }
 
+__global__ void glb_clear_kernel(uint32_t* used) { *used = 0; }
+
+// A task per lane; a wave reserves the words of its tasks with one atomic.  CIGARs
+// of more than kGatherOps words stay in their slots, so the sum fits 32 bits.
+constexpr int kGatherOps = 4096;
+__global__ void __launch_bounds__(256)
+glb_gather_kernel(const int32_t* __restrict__ score, const int32_t* __restrict__ n_cigar,
+                  const uint32_t* __restrict__ cigar, const uint8_t* __restrict__ bin_of, int n, int64_t slot,
+                  int32_t* __restrict__ rec, uint32_t* __restrict__ words, uint32_t room, uint32_t* __restrict__ used) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+  const bool ok = k < n && bin_of[k] != 0xff;
+  const int nc = ok && n_cigar ? n_cigar[k] : 0;
+  const int have = cigar && nc > 0 && nc <= kGatherOps ? nc : 0;
+  int sum = have;  // inclusive sum over the wave
+  for (int d = 1; d < 64; d <<= 1) {
+    const int x = __shfl_up(sum, d);
+    sum += lane >= d ? x : 0;
+  }
+  uint32_t first = 0;
+  if (lane == 63 && sum > 0) first = atomicAdd(used, (uint32_t)sum);
+  first = (uint32_t)__shfl((int)first, 63) + (uint32_t)(sum - have);
+  const bool fits = have > 0 && first <= room && (uint32_t)have <= room - first;
+  if (k < n) *(int4*)(rec + 4 * (int64_t)k) = make_int4(ok ? score[k] : 0, nc, fits ? (int)first : -1, ok ? 1 : 0);
+  if (fits)
+    for (int x = 0; x < have; ++x) words[first + x] = cigar[(int64_t)k * slot + x];
+}
+
+hipError_t launch_glb_gather(const int32_t* score, const int32_t* n_cigar, const uint32_t* cigar, const uint8_t* bin_of,
+                             int n, int64_t slot, int32_t* rec, uint32_t* words, uint32_t room, uint32_t* used,
+                             bool clear, hipStream_t st) {
+  if (clear) hipLaunchKernelGGL(glb_clear_kernel, dim3(1), dim3(1), 0, st, used);
+  hipLaunchKernelGGL(glb_gather_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, score, n_cigar, cigar,
+                     bin_of, n, slot, rec, words, room, used);
+  return hipGetLastError();
+}
+
 // Direction-byte slots per CU, one slot a group.  A launch uses the part given
 // to its stream; launches that run one after another share kGlbSlotsOne.
 struct GlbPart { int first, slots; };

@@ -278,7 +278,7 @@ template void launch_wave_bin<32>(const ExtKArgs&, const ExtWork&, int, int64_t,
 
 
 // A batch without binning: block t runs task t, checked here, and writes its
-// results where the caller wants them.  Tasks of more than 256 columns need
+// results where the caller wants them, or as one record into pinned memory.  Tasks of more than 256 columns need
 // waves of more registers: PART 0 takes the others, PART 1 these, PART 2 all.
 template <int PART>
 __global__ void __launch_bounds__(64, wave_min_waves(PART == 0 ? 4 : 32))
@@ -286,7 +286,9 @@ ext_direct_kernel(ExtArgs A, ExtWork W) {
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x;
   const bool ok = ext_task_ok(A, t);
-  if (PART != 1 && lane == 0) {
+  if (PART != 1 && A.rec_out) {
+    if (!ok && lane < 8) A.rec_out[8 * t + lane] = 0;
+  } else if (PART != 1 && lane == 0) {
     W.bin_of[t] = ok ? 0 : 0xff;
     if (!ok) {
       atomicAdd(&W.err[0], 1);
@@ -306,7 +308,9 @@ ext_direct_kernel(ExtArgs A, ExtWork W) {
   else if (PART != 0 && fits(8)) R = wave_task<8>(A, q, tg, ql, tl, h0, w);
   else if (PART != 0 && fits(16)) R = wave_task<16>(A, q, tg, ql, tl, h0, w);
   else if (PART != 0) R = wave_task<32>(A, q, tg, ql, tl, h0, w);
-  if (lane == 0) {
+  if (A.rec_out) {
+    write_rec<64>(A.rec_out, t, lane, R.best, R.qle, R.tle, R.gtle, R.gscore, R.moff, R.ncell, 1);
+  } else if (lane == 0) {
     if (A.score) A.score[t] = R.best;
     if (A.qle) A.qle[t] = R.qle;
     if (A.tle) A.tle[t] = R.tle;
