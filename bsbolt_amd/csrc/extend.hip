@@ -496,8 +496,9 @@ ext_unpack_kernel(ExtArgs A, ExtWork W, const int32_t* __restrict__ rec) {
 // many tasks as leave every SIMD kBlocksPerSimd blocks, at least one per group:
 // with 32 per block, 500 flanks of 150 bp reads ran in 16 (1.11 ms, so 0.24).
 template <int L, int C, bool E1>
-static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st) {
-  constexpr int64_t kBlocksPerSimd = 4, kMaxBlocksPerCu = 128;
+static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st, bool pair) {
+  constexpr int64_t kBlocksPerSimd = 4;
+  const int64_t kMaxBlocksPerCu = pair ? 16 : 128;
   const int64_t fill = n / (num_cu * 4 * kBlocksPerSimd);
   k.tpb = (int)std::min<int64_t>(k.tpb, std::max<int64_t>(64 / L, fill));
   const int64_t blocks = std::min<int64_t>((n + k.tpb - 1) / k.tpb, (int64_t)num_cu * kMaxBlocksPerCu);
@@ -518,11 +519,11 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
   } else if constexpr (B == kTunedBin[0] || B == kTunedBin[1]) {
     constexpr int V = B == kTunedBin[0] ? 0 : 1;
     if (wk.shape_var[V] == 1)
-      launch_group<kAltShape[V][1].lanes, kAltShape[V][1].cols, E1>(k, wk, B, n, num_cu, st);
+      launch_group<kAltShape[V][1].lanes, kAltShape[V][1].cols, E1>(k, wk, B, n, num_cu, st, pair);
     else
-      launch_group<L, C, E1>(k, wk, B, n, num_cu, st);
+      launch_group<L, C, E1>(k, wk, B, n, num_cu, st, pair);
   } else {
-    launch_group<L, C, E1>(k, wk, B, n, num_cu, st);
+    launch_group<L, C, E1>(k, wk, B, n, num_cu, st, pair);
   }
 }
 

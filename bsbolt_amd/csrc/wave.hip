@@ -264,7 +264,8 @@ ext_wave_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
 
 template <int C>
 void launch_wave_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st) {
-  const int64_t blocks = std::min<int64_t>(n, (int64_t)num_cu * 128);
+  // as many as are resident: surplus blocks of an empty bin cost 9 us a launch
+  const int64_t blocks = std::min<int64_t>(n, (int64_t)num_cu * 4 * wave_min_waves(C));
   if (blocks < 1) return;
   time_begin(wk, time_slot_bin(bin), st);
   hipLaunchKernelGGL(ext_wave_kernel<C>, dim3((unsigned)blocks), dim3(64), 0, st, k, (const ExtDesc*)wk.desc,
