@@ -924,7 +924,7 @@ int bsx_reg2aln_cigar_device(bsx_ctx* c, const bsx_reg2aln_tasks* t, bsx_reg2aln
 
 static int glb_buffers(bsx_ctx* c, size_t n, bool cigar) {
   HIPCHK(c, c->ws->bin_of.ensure(n + 1), "hipMalloc(bin_of)");
-  HIPCHK(c, c->ws->list.ensure(4 * n + 4), "hipMalloc(list)");
+  HIPCHK(c, c->ws->list.ensure(4 * n * (n <= (size_t)kGlbDirectMaxTasks ? kGlbRest : 1) + 4), "hipMalloc(list)");
   HIPCHK(c, c->ws->small.ensure(kSmallBytes), "hipMalloc(work)");
   if (cigar) {
     HIPCHK(c, c->ws->zbuf.ensure((size_t)glb_groups(c->num_cu, c->ss_on) * (size_t)c->zslot), "hipMalloc(z)");

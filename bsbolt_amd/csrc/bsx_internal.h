@@ -316,6 +316,35 @@ struct GlbWork {
   const StreamSet* ss;  // side streams for the bins with few tasks per group (nullptr: one stream)
 };
 
+constexpr int kGlbMaxT = 1 << 16;
+__device__ __forceinline__ int glb_bin_of(int ncol) {
+#pragma unroll
+  for (int b = 0; b < kGlbBins; ++b)
+    if (ncol <= glb_bin_limit(b)) return b;
+  return -1;
+}
+// Whether task t may run: the reference's preconditions, and its directions fit
+// a slot.
+__device__ __forceinline__ bool glb_task_ok(const GlbArgs& A, const GlbWork& W, int64_t t) {
+  const int ql = A.qlen[t], tl = A.tlen[t], w = A.w[t];
+  const int diff = tl > ql ? tl - ql : ql - tl;
+  const int64_t ncol = ql < 2 * (int64_t)w + 1 ? ql : 2 * (int64_t)w + 1;
+  return ql >= 1 && ql <= kGlbMaxT && tl >= 1 && tl <= kGlbMaxT && w >= 0 && glb_bin_of((int)ncol) >= 0 && diff <= w &&
+         (A.cigar == nullptr || ncol * tl <= W.zslot);
+}
+// The bins that take what the unbinned kernel leaves, and the one of a band.
+constexpr int kGlbRest = 3;
+constexpr int kGlbRestBin[kGlbRest] = {5, 6, 7};
+__device__ __forceinline__ int glb_rest_of(int ncol) {
+  return ncol <= glb_bin_limit(kGlbRestBin[0]) ? 0 : ncol <= glb_bin_limit(kGlbRestBin[1]) ? 1 : 2;
+}
+// Largest batch that runs a wave per task without binning (gwave.hip).  us per
+// call, so / in bins beside each other: 100 bp reads 300 tasks 52 / 153, 8,000 127 /
+// 189, 16,000 202 / 223, 24,000 278 / 264; 150 bp 300 69 / 208, 16,000 289 / 341,
+// 24,000 398 / 365; 250 bp 300 111 / 308, 16,000 468 / 739, 24,000 653 / 628.
+constexpr int64_t kGlbDirectMaxTasks = 20480;
+void launch_glb_direct(const GlbArgs& a, const GlbWork& w, hipStream_t st);
+
 // NM / MD:Z / XB:Z of CIGARs (bwa_gen_cigar2's tail, bwa.c:250-343); fields as
 // bsx_md_tasks / bsx_md_results in include/bsx.h.
 struct MdArgs {

@@ -26,7 +26,6 @@
 namespace bsx {
 
 constexpr int kNegInf = -0x40000000;  // MINUS_INF, ksw.c:490
-constexpr int kGlbMaxT = 1 << 16;
 // dwords of a group's LDS window on its direction bytes (16 KB per block)
 template <int L>
 constexpr int zwin_dw() { return L < 16 ? 128 : 256; }
@@ -92,13 +91,16 @@ __device__ __forceinline__ int g_next(int x) {
 
 template <int L, int C>
 __global__ void __launch_bounds__(256)
-glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase) {
+glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase, int64_t first) {
   const int lane = threadIdx.x & 63;
   const int lig = lane & (L - 1);
   const int base = lig * C;
   const int group = (blockIdx.x * blockDim.x + threadIdx.x) / L;
-  uint32_t lbase = 0;
-  for (int b = 0; b < bin; ++b) lbase += W.counts[b];
+  int64_t lbase = first;  // of the bin's list; -1: it follows those before it
+  if (first < 0) {
+    lbase = 0;
+    for (int b = 0; b < bin; ++b) lbase += W.counts[b];
+  }
   const int32_t* __restrict__ list = W.list + lbase;
   const uint32_t nlist = W.counts[bin];
   uint8_t* __restrict__ z = W.z + (zbase + group) * W.zslot;  // zbase: this launch's slot region
@@ -394,13 +396,6 @@ glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase) {
   }
 }
 
-__device__ __forceinline__ int glb_bin_of(int ncol) {
-#pragma unroll
-  for (int b = 0; b < kGlbBins; ++b)
-    if (ncol <= glb_bin_limit(b)) return b;
-  return -1;
-}
-
 // Bin of the two-tasks-per-lane kernel for a valid task, or -1: the whole band
 // (not clipped to the query) fits, and every score fits its 16 bits.
 __device__ __forceinline__ int glb_pair_bin_of(const GlbArgs& A, int ql, int tl, int w) {
@@ -423,18 +418,15 @@ glb_bin_count_kernel(GlbArgs A, GlbWork W) {
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < A.n;
        t += (int64_t)gridDim.x * blockDim.x) {
     const int ql = A.qlen[t], tl = A.tlen[t], w = A.w[t];
-    const int diff = tl > ql ? tl - ql : ql - tl;
-    const int64_t ncol = ql < 2 * (int64_t)w + 1 ? ql : 2 * (int64_t)w + 1;
-    int b = glb_bin_of((int)ncol);  // by band width: a group holds n_col positions
-    const bool ok = ql >= 1 && ql <= kGlbMaxT && tl >= 1 && tl <= kGlbMaxT && w >= 0 && b >= 0 && diff <= w &&
-                    (A.cigar == nullptr || ncol * tl <= W.zslot);
+    int b;
+    const bool ok = glb_task_ok(A, W, t);
     if (!ok) {
       b = 0xff;
       atomicAdd(&W.err[0], 1);
       atomicMin(&W.err[1], (int)t);
     } else {
       const int pb = glb_pair_bin_of(A, ql, tl, w);
-      b = pb >= 0 ? pb : b;
+      b = pb >= 0 ? pb : glb_bin_of((int)min((int64_t)ql, 2 * (int64_t)w + 1));  // a group holds n_col positions
       atomicAdd(&hist[b], 1u);
       atomicAdd(&khist[glb_key(b, tl)], 1u);
     }
@@ -545,20 +537,21 @@ static_assert(StreamSet::kSide == 3, "slot parts");
 // latency of its rows, 115-145 us a bin whatever its share of the tasks, so the
 // four bins that are seldom empty run beside each other, and the wide ones follow
 // where they wait for nobody.  With all of them on one stream but (16,4) the
-// call took 2-3 times as long (us, before / now): 100 bp reads 4,000 tasks 480 /
-// 179, 64,000 685 / 426; 150 bp 4,000 815 / 245, 64,000 1143 / 646; 250 bp 4,000
-// 1187 / 392, 64,000 2156 / 1598.
+// call took longer (us, before / now): 100 bp reads 32,000 tasks 581 / 267, 64,000
+// 685 / 426; 150 bp 32,000 941 / 416, 64,000 1143 / 646; 250 bp 32,000 1848 / 963,
+// 64,000 2156 / 1598.
 constexpr int kGlbStream[kGlbBins] = {1, 0, 2, 3, 3, 3, 3, 3};
 
 int64_t glb_groups(int num_cu, bool side) { return (int64_t)num_cu * (side ? kGlbSlots : kGlbSlotsOne); }
 
 template <int B>
-static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st, GlbPart part) {
+static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st, GlbPart part,
+                           int64_t first = -1) {
   constexpr int L = kGlbShape[B].lanes, C = kGlbShape[B].cols;
   const int64_t room = std::min<int64_t>(part.slots / (256 / L), 7) * num_cu;
   const int64_t blocks = std::min<int64_t>(room, (a.n * L + 255) / 256);
   hipLaunchKernelGGL((glb_kernel<L, C>), dim3((unsigned)blocks), dim3(256), 0, st, a, w, B,
-                     (int64_t)part.first * num_cu);
+                     (int64_t)part.first * num_cu, first);
 }
 
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) {
@@ -566,6 +559,14 @@ hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) 
   a.pair = a.n >= kGlbPairMinTasks;
   hipLaunchKernelGGL(glb_reset_kernel, dim3(1), dim3(1024), 0, st, w);
   if (a.n <= 0) return hipGetLastError();
+  if (a.n <= std::min<int64_t>(kGlbDirectMaxTasks, (int64_t)num_cu * kGlbSlotsOne)) {
+    launch_glb_direct(a, w, st);
+    static_assert(kGlbRest == 3, "rest bins");
+    glb_launch_bin<kGlbRestBin[0]>(a, w, num_cu, st, kGlbAlone, 0);
+    glb_launch_bin<kGlbRestBin[1]>(a, w, num_cu, st, kGlbAlone, a.n);
+    glb_launch_bin<kGlbRestBin[2]>(a, w, num_cu, st, kGlbAlone, 2 * a.n);
+    return hipGetLastError();
+  }
   // each block ends with a global atomic per non-empty bucket
   const int64_t blocks = std::min<int64_t>((a.n + 255) / 256, (int64_t)num_cu * 4);
   hipLaunchKernelGGL(glb_bin_count_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, w);
