@@ -60,22 +60,8 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
     lo = qc == 3 ? A.prof_lo[3] : lo;
     return lo;
   };
-  // bytes first + 4*lane .. + 3 of a sequence (clamped addresses, always loaded)
-  struct Raw { uint32_t b[4]; };
-  auto load4 = [&](const uint8_t* p, int len, int first) -> Raw {
-    Raw r;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) r.b[k] = p[min(first + 4 * lane + k, len - 1)];
-    return r;
-  };
-  auto pack4 = [&](const Raw& r) -> uint32_t { return r.b[0] | r.b[1] << 8 | r.b[2] << 16 | r.b[3] << 24; };
-
   int G[C], E[C];
   uint32_t plo[C];
-  constexpr int QN = (C + 3) / 4;
-  uint32_t qpk[QN];  // query codes, 4 per register (for rows whose target base is N)
-#pragma unroll
-  for (int c = 0; c < QN; ++c) qpk[c] = 0;
   {
     uint32_t qb[C];
 #pragma unroll
@@ -85,17 +71,25 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
       const int j = base + c;
       const uint32_t qc = j < qlen ? min(qb[c], 4u) : 4u;
       plo[c] = prof(qc);
-      qpk[c / 4] |= qc << (8 * (c % 4));
       G[c] = ramp(j);
       E[c] = 0;
     }
   }
-  // 256-base windows of the target (row i) and of the query from column WF on
-  // (entering the frame), each with the next one already loading
-  uint32_t tch = pack4(load4(target, tlen, 0));
-  Raw tnx = load4(target, tlen, 256);
-  uint32_t qch = pack4(load4(query, qlen, WF));
-  Raw qnx = load4(query, qlen, WF + 256);
+  // The next 64 rows' bases by lane, as shifts into a profile word (32: not a base),
+  // and the profile words of the next 64 columns to enter the frame; the bytes of
+  // the 64 after them are already loading.  (Scalar instructions bound the row as
+  // much as vector ones: 80,000 flanks of 150 bp reads 595 us with bytes in the
+  // windows, 557 so.)
+  auto shift_of = [&](uint32_t b) -> uint32_t { return 8 * min(b, 4u); };
+  auto prof_at = [&](uint32_t b, int j) -> uint32_t { return prof(j < qlen ? min(b, 4u) : 4u); };
+  auto t_at = [&](int i) -> uint32_t { return target[min(i + lane, tlen - 1)]; };
+  auto q_at = [&](int j) -> uint32_t { return query[min(j + lane, qlen - 1)]; };
+  uint32_t tch = shift_of(t_at(0)), tnx = t_at(64);
+  uint32_t qch = 0, qnx = 0;
+  if (qlen > WF) {
+    qch = prof_at(q_at(WF), WF + lane);
+    qnx = q_at(WF + 64);
+  }
 
   int beg = 0, end = qlen, f0 = 0;
   int best = h0, best_i = -1, best_j = -1, gbest = -1, gbest_i = -1, moff = 0;
@@ -103,39 +97,26 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
   const int kE0 = base * e_ins;  // frame position k contributes k*e_ins
 
   for (int i = 0; i < tlen; ++i) {
-    if (i && (i & 255) == 0) {
-      tch = pack4(tnx);
-      tnx = load4(target, tlen, i + 256);
+    if (i && (i & 63) == 0) {
+      tch = shift_of(tnx);
+      tnx = t_at(i + 64);
     }
-    const int t = (int)((uint32_t)__builtin_amdgcn_readlane((int)tch, (i & 255) >> 2) >> (8 * (i & 3)) & 0xffu);
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)tch, i & 63);
 
     const int cap_beg = i - w;
     if (cap_beg - f0 >= C && f0 + WF < qlen) {
       // the frame moves one lane: lane 63 takes the next C columns
-      const int jn = f0 + WF;  // a multiple of C
-      const int jo = (jn - WF) & 255;
-      if (jn > WF && jo == 0) {
-        qch = pack4(qnx);
-        qnx = load4(query, qlen, jn + 256);
+      const int jn = f0 + WF, jo = f0 & 63;
+      if (f0 > 0 && jo == 0) {
+        qch = prof_at(qnx, jn + lane);
+        qnx = q_at(jn + 64);
       }
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)qch, (jo + c) >> 2);
-        const uint32_t qb = word >> (8 * ((jo + c) & 3)) & 0xffu;
-        const uint32_t qc = jn + c < qlen ? (qb > 4u ? 4u : qb) : 4u;
+        const int in = __builtin_amdgcn_readlane((int)qch, jo + c);
         G[c] = __builtin_amdgcn_update_dpp(ramp(jn + c), G[c], 0x130, 0xf, 0xf, false);  // wave_shl:1
         E[c] = __builtin_amdgcn_update_dpp(0, E[c], 0x130, 0xf, 0xf, false);
-        plo[c] = (uint32_t)__builtin_amdgcn_update_dpp((int)prof(qc), (int)plo[c], 0x130, 0xf, 0xf, false);
-        if (c % 4 == 0) {
-          uint32_t in = 0;
-#pragma unroll
-          for (int x = 0; x < 4 && c + x < C; ++x) {
-            const uint32_t wx = (uint32_t)__builtin_amdgcn_readlane((int)qch, (jo + c + x) >> 2);
-            const uint32_t bx = wx >> (8 * ((jo + c + x) & 3)) & 0xffu;
-            in |= (jn + c + x < qlen ? (bx > 4u ? 4u : bx) : 4u) << (8 * x);
-          }
-          qpk[c / 4] = (uint32_t)__builtin_amdgcn_update_dpp((int)in, (int)qpk[c / 4], 0x130, 0xf, 0xf, false);
-        }
+        plo[c] = (uint32_t)__builtin_amdgcn_update_dpp(in, (int)plo[c], 0x130, 0xf, 0xf, false);
       }
       f0 += C;
     }
@@ -151,10 +132,11 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
 
     const int d = end - f0 - base;  // live columns of this lane: c < d
     int M[C], ex[C];
-    if (__builtin_expect(t > 3, 0)) {
+    if (__builtin_expect(t == 32, 0)) {
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        const uint32_t qc = (qpk[c / 4] >> (8 * (c % 4))) & 0xffu;
+        const int j = f0 + base + c;
+        const uint32_t qb = query[min(j, qlen - 1)], qc = j < qlen ? qb : 4u;
         int s = A.prof_hi[4];
         s = qc == 0 ? A.prof_hi[0] : s;
         s = qc == 1 ? A.prof_hi[1] : s;
@@ -164,7 +146,7 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
       }
     } else {
 #pragma unroll
-      for (int c = 0; c < C; ++c) M[c] = __builtin_amdgcn_sbfe((int)plo[c], 8u * (uint32_t)t, 8u);
+      for (int c = 0; c < C; ++c) M[c] = __builtin_amdgcn_sbfe((int)plo[c], t, 8u);
     }
     int run = 0;
 #pragma unroll
