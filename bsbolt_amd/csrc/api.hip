@@ -777,7 +777,7 @@ int bsx_extend_batch(bsx_ctx* c, const bsx_scoring* sc, const bsx_ext_tasks* t, 
   ExtWork wk = ext_work(c);
   if (direct) {
     a.rec_out = (int32_t*)c->p_out.d;
-    launch_direct(a, wk, c->num_cu, st);
+    launch_direct(a, wk, c->num_cu, st, false);
     HIPCHK(c, hipGetLastError(), "extension launch");
     c->last_n = 0;
   } else {

@@ -96,6 +96,7 @@ __host__ __device__ inline int row_bucket(int tlen, int h0) {
 // frames of 24, 40, 80, 144 columns; class 4 is the plain kernel.  Count slots: plain bins
 // [0, kExtBins), narrow classes [kExtBins, kExtBins + kBandClasses - 1).
 constexpr int kBandClasses = 5;
+constexpr int kFrameWidth[kBandClasses - 1] = {24, 40, 80, 144};
 constexpr int kCountSlots = 16;
 static_assert(kExtBins + kBandClasses - 1 <= kCountSlots, "count slots for bins and narrow classes");
 constexpr int kNarrowQMax = 256;  // longest query the narrow kernels take
@@ -272,11 +273,13 @@ void launch_wave_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, i
 // 565; 150 bp 500 89 / 192, 32,000 278 / 573, 128,000 1044 / 1045; 250 bp 500 192 /
 // 330, 80,000 1521 / 2693, 128,000 2925 / 2741.
 constexpr int64_t kDirectMaxTasks = 98304;
-void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st);
+void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, bool cert);
 // lane-per-task frame kernel (frame of WF columns) of lane-frame class `cls`
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st);
 hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan);
+// routes a checked batch (nbin_of, need_plain)
+void launch_narrow_count(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan& plan);
 hipError_t launch_narrow(const ExtArgs& a, const ExtKArgs& k, const ExtWork& wk, int num_cu, hipStream_t st,
                          const BandPlan& plan);
 

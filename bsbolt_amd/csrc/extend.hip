@@ -540,13 +540,18 @@ static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num
 using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 11, 10, 9, 3, 2, 1, 0>;
 static_assert(kExtBins == 12, "launch order");
 
+static void launch_unpack(const ExtArgs& a, const ExtWork& wk, int64_t blocks, hipStream_t st) {
+  if (a.score || a.qle || a.tle || a.gtle || a.gscore || a.max_off || a.cells)
+    hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
+}
+
 hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan) {
   a.pair = a.n >= kPairMinTasks && a.e_del <= kPairMaxGapExt && a.e_ins <= kPairMaxGapExt;
   hipLaunchKernelGGL(ext_reset_kernel, dim3(1), dim3(256), 0, st, wk, kExtCounterWords);
   if (a.n <= 0) return hipGetLastError();
   const bool band = plan && plan->mode != kBandPlain;
   if (a.n <= kDirectMaxTasks && !band && !wk.tev) {  // timed calls time the bins
-    launch_direct(a, wk, num_cu, st);
+    launch_direct(a, wk, num_cu, st, false);
     return hipGetLastError();
   }
   int64_t blocks = (a.n + 255) / 256;  // unpack pass
@@ -570,6 +575,15 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
     k.trow_hi[t] = t < 4 ? (a.prof_lo[4] >> (8 * t)) & 0xffu : (uint32_t)a.prof_hi[4] & 0xffu;
   }
   hipLaunchKernelGGL(ext_bin_count_kernel, dim3((unsigned)sblocks), dim3(256), 0, st, a, wk, band ? 1 : 0);
+  if (band && a.n <= kDirectMaxTasks && !wk.tev && !plan->skip_plain) {
+    // Small batches run every task in full and test its frame on the way: us per
+    // call, so / the frames and then what they left, 150 bp reads in 24-column
+    // frames: 5,000 tasks 182 / 700, 30,000 336 / 958, 90,000 772 / 1467.
+    launch_narrow_count(a, wk, num_cu, st, *plan);
+    launch_direct(a, wk, num_cu, st, true);
+    launch_unpack(a, wk, blocks, st);
+    return hipGetLastError();
+  }
   if (band) {
     ExtKArgs kn = k;
     kn.tpb = wk.tpb_narrow;
@@ -584,9 +598,7 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   if (a.e_del == 1 && a.e_ins == 1) launch_bins<true>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
   else launch_bins<false>(k, wk, a.n, num_cu, st, a.pair, BinOrder{});
   ss_join(wk.ss, st);
-  if (a.score || a.qle || a.tle || a.gtle || a.gscore || a.max_off || a.cells)
-    hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk,
-                       (const int32_t*)wk.rec);
+  launch_unpack(a, wk, blocks, st);
   return hipGetLastError();
 }
 

@@ -26,6 +26,8 @@
 // cancels.  Raw query codes are staged per task in LDS; each row selects its
 // target base's score row (mat[t*5+q]) and extracts per-column scores with
 // v_perm_b32.
+#include <algorithm>
+
 #include "bsx_internal.h"
 #include "ext_common.h"
 
@@ -36,6 +38,8 @@ namespace bsx {
 __host__ __device__ constexpr int frame_lanes(int c) { return c <= 1 ? 8 : 16; }
 __host__ __device__ constexpr int frame_cols(int c) { return c == 0 ? 3 : c == 1 ? 5 : c == 2 ? 5 : 9; }
 __host__ __device__ constexpr int frame_of_class(int c) { return frame_lanes(c) * frame_cols(c); }
+static_assert(frame_of_class(0) == kFrameWidth[0] && frame_of_class(1) == kFrameWidth[1] &&
+              frame_of_class(2) == kFrameWidth[2] && frame_of_class(3) == kFrameWidth[3], "frame widths");
 
 // Measured cost of one DP row per task on MI355X (picoseconds of kernel time
 // per row over a 150 bp paired-end bisulfite batch, each kernel run alone):
@@ -545,12 +549,19 @@ static void launch_narrow_classes(const ExtKArgs& k, const ExtWork& wk, int64_t 
   launch_narrow_class<0, E1>(k, wk, n, num_cu, st);
 }
 
+// count and scatter: each block ends with global atomics per class and row bucket
+static int64_t narrow_blocks(const ExtArgs& a, int num_cu) {
+  return std::min<int64_t>((a.n + 255) / 256, (int64_t)num_cu * 4);
+}
+
+void launch_narrow_count(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan& plan) {
+  hipLaunchKernelGGL(ext_narrow_count_kernel, dim3((unsigned)narrow_blocks(a, num_cu)), dim3(256), 0, st, a, wk, plan);
+}
+
 hipError_t launch_narrow(const ExtArgs& a, const ExtKArgs& k, const ExtWork& wk, int num_cu, hipStream_t st,
                          const BandPlan& plan) {
-  // count and scatter: each block ends with global atomics per class and row bucket
-  int64_t blocks = (a.n + 255) / 256;
-  if (blocks > (int64_t)num_cu * 4) blocks = (int64_t)num_cu * 4;
-  hipLaunchKernelGGL(ext_narrow_count_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, plan);
+  const int64_t blocks = narrow_blocks(a, num_cu);
+  launch_narrow_count(a, wk, num_cu, st, plan);
   const int64_t per_block = (a.n + blocks - 1) / blocks;
   hipLaunchKernelGGL(ext_narrow_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, per_block);
   ss_fork(wk.ss, st);

@@ -34,21 +34,26 @@ namespace bsx {
 struct WaveRes {
   int best, qle, tle, gtle, gscore, moff;
   uint32_t ncell;
+  bool fail;  // a frame run would have stopped (wave_task's `fw`)
 };
 
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // A: the scoring fields (ExtArgs or ExtKArgs).  Every argument is uniform over
 // the wave; query and target hold qlen >= 1 and tlen >= 0 bases.
-template <int C, class Args>
+// fw (CERT): also tells whether the band-following run in a frame of fw columns
+// (narrow.hip) would have reached past it, by that run's own test on the same
+// values: the two are equal up to the row where it stops.
+template <int C, bool CERT, class Args>
 __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __restrict__ query,
-                                             const uint8_t* __restrict__ target, int qlen, int tlen, int h0, int w) {
+                                             const uint8_t* __restrict__ target, int qlen, int tlen, int h0, int w,
+                                             int fw = 0) {
   constexpr int WF = 64 * C;
   const int lane = threadIdx.x & 63;
   const int base = lane * C;
   const int e_del = A.e_del, e_ins = A.e_ins;
   const int oe_del = A.o_del + e_del, oe_ins = A.o_ins + e_ins;
-  WaveRes R{h0, 0, 0, 0, -1, 0, 0u};
+  WaveRes R{h0, 0, 0, 0, -1, 0, 0u, false};
   if (tlen <= 0) return R;  // ksw.c:473-478 with no row
 
   auto ramp = [&](int j) { const int g = j == 0 ? h0 : h0 - oe_ins - (j - 1) * e_ins; return g > 0 ? g : 0; };
@@ -91,7 +96,7 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
     qnx = q_at(WF + 64);
   }
 
-  int beg = 0, end = qlen, f0 = 0;
+  int beg = 0, end = qlen, f0 = 0, ff = 0;  // ff: first column of the narrow frame
   int best = h0, best_i = -1, best_j = -1, gbest = -1, gbest_i = -1, moff = 0;
   uint32_t ncell = 0;
   const int kE0 = base * e_ins;  // frame position k contributes k*e_ins
@@ -178,6 +183,14 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
       for (int c = 1; c < C; ++c) he = (ke & (C - 1)) == c ? h[c] : he;
       h1 = __builtin_amdgcn_readlane(he, ke / C);
     }
+    if (CERT && fw && end > ff + fw - 1) {  // the band reaches past the frame: its cells there must be 0
+      const int eF = ff + fw - 1, ce = eF - f0;
+      int he = h[0];
+#pragma unroll
+      for (int c = 1; c < C; ++c) he = (ce & (C - 1)) == c ? h[c] : he;
+      const int hF = ce >= 0 ? __builtin_amdgcn_readlane(he, ce / C) : 0;  // left of the wave's frame all is 0
+      R.fail = R.fail || hF != 0 || ramp(eF + 1) > 0;
+    }
     // G(j) = H(i, j-1) for j <= end; column 0 receives the first-column value
     const int hsh = __builtin_amdgcn_update_dpp(h1p, h[C - 1], 0x138, 0xf, 0xf, false);  // wave_shr:1
     uint32_t nzb = 0;  // bit c: column c holds a non-zero G or E after the row
@@ -217,6 +230,7 @@ __device__ __forceinline__ WaveRes wave_task(const Args& A, const uint8_t* __res
     if (h1 != 0) hz = end;
     beg = nb;
     end = min(hz >= 0 ? hz + 2 : nb + 1, qlen);
+    if (CERT) ff += min(beg - ff, 2);
   }
   R.best = best; R.qle = best_j + 1; R.tle = best_i + 1; R.gtle = gbest_i + 1; R.gscore = gbest;
   R.moff = moff; R.ncell = ncell;
@@ -239,7 +253,7 @@ ext_wave_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
     const int task = uni(a.x);
     const uint64_t qoff = (uint64_t)(uint32_t)uni(b.z) | (uint64_t)(uint32_t)uni(b.w) << 32;
     const uint64_t toff = (uint64_t)(uint32_t)uni(c.x) | (uint64_t)(uint32_t)uni(c.y) << 32;
-    const WaveRes R = wave_task<C>(A, A.query + qoff, A.target + toff, uni(a.y), uni(a.z), uni(a.w), uni(b.x));
+    const WaveRes R = wave_task<C, false>(A, A.query + qoff, A.target + toff, uni(a.y), uni(a.z), uni(a.w), uni(b.x));
     write_rec<64>(A.rec, task, threadIdx.x, R.best, R.qle, R.tle, R.gtle, R.gscore, R.moff, R.ncell);
   }
 }
@@ -263,19 +277,23 @@ template void launch_wave_bin<32>(const ExtKArgs&, const ExtWork&, int, int64_t,
 // A batch without binning: block t runs task t, checked here, and writes its
 // results where the caller wants them, or as one record into pinned memory.  Tasks of more than 256 columns need
 // waves of more registers: PART 0 takes the others, PART 1 these, PART 2 all.
-template <int PART>
+// CERT: a batch that was checked and routed (nbin_of); also marks the tasks whose
+// frame run fails (need_plain), and leaves every result in ExtWork::rec.
+template <int PART, bool CERT>
 __global__ void __launch_bounds__(64, wave_min_waves(PART == 0 ? 4 : 32))
 ext_direct_kernel(ExtArgs A, ExtWork W) {
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x;
-  const bool ok = ext_task_ok(A, t);
-  if (PART != 1 && A.rec_out) {
-    if (!ok && lane < 8) A.rec_out[8 * t + lane] = 0;
-  } else if (PART != 1 && lane == 0) {
-    W.bin_of[t] = ok ? 0 : 0xff;
-    if (!ok) {
-      atomicAdd(&W.err[0], 1);
-      atomicMin(&W.err[1], (int)t);
+  const bool ok = CERT ? W.bin_of[t] != 0xff : ext_task_ok(A, t);
+  if (!CERT && PART != 1) {
+    if (A.rec_out) {
+      if (!ok && lane < 8) A.rec_out[8 * t + lane] = 0;
+    } else if (lane == 0) {
+      W.bin_of[t] = ok ? 0 : 0xff;
+      if (!ok) {
+        atomicAdd(&W.err[0], 1);
+        atomicMin(&W.err[1], (int)t);
+      }
     }
   }
   if (!ok) return;
@@ -284,15 +302,22 @@ ext_direct_kernel(ExtArgs A, ExtWork W) {
   const auto fits = [&](int C) { return ql <= 64 * C || 2 * (int64_t)w + 1 + C <= 64 * C; };
   if (PART != 2 && fits(4) != (PART == 0)) return;
   const uint8_t *q = A.query + A.q_off[t], *tg = A.target + A.t_off[t];
+  int fw = 0;
+  if (CERT) {
+    const int nb = W.nbin_of[t];
+    fw = nb == 0 ? kFrameWidth[0] : nb == 1 ? kFrameWidth[1] : nb == 2 ? kFrameWidth[2] : nb == 3 ? kFrameWidth[3] : 0;
+  }
   WaveRes R{};
-  if (PART != 1 && fits(1)) R = wave_task<1>(A, q, tg, ql, tl, h0, w);
-  else if (PART != 1 && fits(2)) R = wave_task<2>(A, q, tg, ql, tl, h0, w);
-  else if (PART != 1 && fits(4)) R = wave_task<4>(A, q, tg, ql, tl, h0, w);
-  else if (PART != 0 && fits(8)) R = wave_task<8>(A, q, tg, ql, tl, h0, w);
-  else if (PART != 0 && fits(16)) R = wave_task<16>(A, q, tg, ql, tl, h0, w);
-  else if (PART != 0) R = wave_task<32>(A, q, tg, ql, tl, h0, w);
-  if (A.rec_out) {
-    write_rec<64>(A.rec_out, t, lane, R.best, R.qle, R.tle, R.gtle, R.gscore, R.moff, R.ncell, 1);
+  if (PART != 1 && fits(1)) R = wave_task<1, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  else if (PART != 1 && fits(2)) R = wave_task<2, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  else if (PART != 1 && fits(4)) R = wave_task<4, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  else if (PART != 0 && fits(8)) R = wave_task<8, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  else if (PART != 0 && fits(16)) R = wave_task<16, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  else if (PART != 0) R = wave_task<32, CERT>(A, q, tg, ql, tl, h0, w, fw);
+  if (CERT && R.fail && lane == 0) W.need_plain[t] = 1;
+  int32_t* rec = CERT ? W.rec : A.rec_out;
+  if (rec) {
+    write_rec<64>(rec, t, lane, R.best, R.qle, R.tle, R.gtle, R.gscore, R.moff, R.ncell, CERT ? 0 : 1);
   } else if (lane == 0) {
     if (A.score) A.score[t] = R.best;
     if (A.qle) A.qle[t] = R.qle;
@@ -309,18 +334,24 @@ ext_direct_kernel(ExtArgs A, ExtWork W) {
 // the others: a long one takes milliseconds (4,000 flanks of 2 kb reads: 3.68 ms
 // after them, 2.26 beside), though the fork costs every other batch 20-27 us
 // (2,000 flanks of 100 bp reads: 69 without, 95 with).
-void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st) {
+template <bool CERT>
+static void direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st) {
   const dim3 grid((unsigned)a.n), block(64);
   if (a.qmax <= 256) {
-    hipLaunchKernelGGL(ext_direct_kernel<0>, grid, block, 0, st, a, wk);
+    hipLaunchKernelGGL((ext_direct_kernel<0, CERT>), grid, block, 0, st, a, wk);
   } else if (a.n <= (int64_t)num_cu * 4 * wave_min_waves(32)) {
-    hipLaunchKernelGGL(ext_direct_kernel<2>, grid, block, 0, st, a, wk);
+    hipLaunchKernelGGL((ext_direct_kernel<2, CERT>), grid, block, 0, st, a, wk);
   } else {
     ss_fork(wk.ss, st);
-    hipLaunchKernelGGL(ext_direct_kernel<0>, grid, block, 0, st, a, wk);
-    hipLaunchKernelGGL(ext_direct_kernel<1>, grid, block, 0, pick_stream(wk.ss, st, 1), a, wk);
+    hipLaunchKernelGGL((ext_direct_kernel<0, CERT>), grid, block, 0, st, a, wk);
+    hipLaunchKernelGGL((ext_direct_kernel<1, CERT>), grid, block, 0, pick_stream(wk.ss, st, 1), a, wk);
     ss_join(wk.ss, st);
   }
+}
+
+void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, bool cert) {
+  if (cert) direct<true>(a, wk, num_cu, st);
+  else direct<false>(a, wk, num_cu, st);
 }
 
 }  // namespace bsx

@@ -63,3 +63,33 @@ def test_unbinned_batches_reject_like_the_bins(engine, n):
     good[bad] = False
     for k in FIELDS[:6]:
         assert (out[k][bad] == -12345).all() and np.array_equal(out[k][good], want[k][good]), k
+
+
+@pytest.mark.parametrize("cls", (0, 1, 2, 3))
+@pytest.mark.parametrize("scoring", ("asym", "bsbolt", "gap25"))
+def test_frames_of_small_batches_fail_as_the_frame_kernels_do(cls, scoring):
+    """The same results and the same count of failed frames as the frame kernels,
+    which a timed call still runs."""
+    from bsbolt_amd import bsx
+    from bsbolt_amd.bsx import Scoring
+    sc = Scoring.make(**SCORINGS[scoring])
+    parts = [make_tasks(31, (5, 24, 25, 40, 41, 80, 81, 100, 144, 145, 150, 224), 1800, lambda r, q: r.integers(1, 150),
+                        (0, 3, 10, 12, 20, 40, 100), sub=0.05),
+             make_tasks(32, (30, 60, 120, 250), 400, lambda r, q: r.integers(100, 900), (5, 30, 100), sub=0.1),
+             make_tasks(33, (30, 90, 200, 500), 200, lambda r, q: r.integers(1, 200), (100,), n_frac=0.02)]
+    e = bsx.Engine(0)
+    try:
+        e.set_band_policy(bsx.BAND_FIXED, cls)
+        for t in parts:
+            want, _ = O.extend2_batch(t, nthreads=8, scoring=sc.as_dict())
+            seen = []
+            for n, timed in ((len(t), 0), (len(t), 1), (5000, 0), (5000, 1)):
+                b, idx = repeat(t, n)
+                e.set_kernel_timing(timed)
+                got = e.extend(b, sc)
+                for k in FIELDS:
+                    assert np.array_equal(got[k], want[k][idx]), (k, n, timed)
+                seen.append(np.asarray(e.band_stats()).tolist())
+            assert seen[0] == seen[1] and seen[2] == seen[3], cls
+    finally:
+        e.close()
