@@ -566,7 +566,7 @@ def main():
     per_launch = kms[:len(limits)] / max(kcalls, 1)
     dom = int(np.argmax(per_launch))
     lanes, cols = bsx.EXT_SHAPES[dom]
-    dom_name = f"ext_pair_kernel<{cols}, true>" if lanes == 1 else f"ext_plain_kernel<{lanes}, {cols}, true>"
+    dom_name = f"ext_pair_kernel<{cols}, true>" if lanes == 1 else f"ext_wave_kernel<{cols}>"
     dom_cells = int(cells[bin_of == dom].sum())
     dom_ms = float(per_launch[dom])
     dom_tops = dom_cells * OPS_PER_CELL / (dom_ms / 1e3) / 1e12

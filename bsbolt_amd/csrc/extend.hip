@@ -541,8 +541,7 @@ using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 11, 10, 9, 3, 2, 1, 0
 static_assert(kExtBins == 12, "launch order");
 
 static void launch_unpack(const ExtArgs& a, const ExtWork& wk, int64_t blocks, hipStream_t st) {
-  if (a.score || a.qle || a.tle || a.gtle || a.gscore || a.max_off || a.cells)
-    hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
+  hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);
 }
 
 hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t st, const BandPlan* plan) {
@@ -578,7 +577,7 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   if (band && a.n <= kDirectMaxTasks && !wk.tev && !plan->skip_plain) {
     // Small batches run every task in full and test its frame on the way: us per
     // call, so / the frames and then what they left, 150 bp reads in 24-column
-    // frames: 5,000 tasks 182 / 700, 30,000 336 / 958, 90,000 772 / 1467.
+    // frames: 30,000 tasks 336 / 958, 90,000 772 / 1467; learned: 5,000 188 / 933.
     launch_narrow_count(a, wk, num_cu, st, *plan);
     launch_direct(a, wk, num_cu, st, true);
     launch_unpack(a, wk, blocks, st);

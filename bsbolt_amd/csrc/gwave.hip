@@ -284,7 +284,8 @@ __global__ void __launch_bounds__(64, 4) glb_direct_kernel(GlbArgs A, GlbWork W)
   const bool want = A.cigar != nullptr;
   const int64_t range = (int64_t)(ql + tl) * (A.pen_max + max(A.e_del, A.e_ins) + A.mat_max) + A.o_del + A.o_ins;
   const auto fits = [&](int C) {
-    return range < kGRange && (ql <= 64 * C || 2 * w + C <= 64 * C) && (!want || (int64_t)((tl - 1) >> 6) * 2048 * C <= W.zslot);
+    return range < kGRange && (ql <= 64 * C || 2 * w + C <= 64 * C) &&
+           (!want || (int64_t)((tl - 1) >> 6) * 2048 * C <= W.zslot);
   };
   const int C = fits(1) ? 1 : fits(2) ? 2 : fits(4) ? 4 : 0;
   if (C == 0) {

@@ -1,29 +1,25 @@
-// Lane-per-task form of the bit-exact ksw_extend2 (bsbolt/External/BWA/ksw.c:380-479)
-// for short queries.
+// Lane-per-task form of the band-following frame run (narrow.hip) for short
+// queries.
 //
-// Each lane of a wave owns one whole task: the DP state of its query columns
-// 0..Q-1 lives in that lane's VGPRs (G[c] = eh[c].h = H(i-1, c-1), E[c] =
-// eh[c].e) and a row is the reference's column loop run sequentially inside the
-// lane -- the same recurrences in the same order, so F needs no scan and no
-// value crosses lanes.  The cost of a row is ~22 VALU instructions per column
-// for 64 tasks at once, against the group kernels' fixed per-row cost of prefix
-// scans and group reductions paid per 4 tasks.
+// Each lane of a wave owns one whole task: the DP state of its frame's columns
+// lives in that lane's VGPRs and a row is the reference's column loop run
+// sequentially inside the lane, so F needs no scan and no value crosses lanes.
 //
 // Band.  Columns < beg are dead: beg never decreases and the kernel keeps them
-// at G = E = 0 (zeroing them when the cap i-w moves beg past non-zero columns),
-// so running them is harmless -- their M, E, F and H are 0, which leaves F(beg)
-// = 0, H(i, beg-1) = 0 and the row maximum unchanged.  Columns >= end keep
-// their stale state (the reference reads it again when the band regrows): the
-// per-column masks c < end and c <= end select the writes.
+// at G = E = 0 (zeroing them when the band cap i-w moves beg past non-zero
+// columns), so running them is harmless.  Columns >= end keep their stale state
+// (the reference reads it again when the band regrows): the per-column masks c <
+// end and c <= end select the writes.
 //
-// Work distribution.  Waves are persistent: a bin's work list is split into
+// Work distribution.  Waves are persistent: a class's work list is split into
 // eight slices, each with a fetch counter; a wave starts on slice blockIdx % 8
 // and moves on when its slice runs dry.  Every K rows the wave stops at a sync
 // point where lanes without a task install their prefetched next task, lanes
 // without a next task move the prefetched descriptor into place and issue the
 // query/target loads, free descriptor slots are refilled with one atomic per
 // wave.  All loads a sync point consumes were issued K rows earlier, so the
-// rows themselves never wait on memory.  Target bases come in 16-base windows, the next one prefetched.
+// rows themselves never wait on memory.  Target bases come in 16-base windows,
+// the next one prefetched.
 #include <algorithm>
 
 #include "bsx_internal.h"
@@ -334,7 +330,8 @@ ext_lane_frame_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const ui
           nz[c >> 5] |= (uint32_t)min(G[c] | E[c], 1) << (c & 31);
           if (c == WF - 1) hlast = h;
           le = lt;
-          asm volatile("" ::"v"(G[c]), "v"(E[c]), "v"(h1), "v"(f), "v"(mk));  // as in the lane kernel
+          // the column ends here: nothing of it sinks, nothing of the next is hoisted
+          asm volatile("" ::"v"(G[c]), "v"(E[c]), "v"(h1), "v"(f), "v"(mk));
           __builtin_amdgcn_sched_barrier(0);
         }
         fail = fail || (spill && hlast != 0);  // a non-zero cell past the frame

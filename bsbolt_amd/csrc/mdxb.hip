@@ -254,8 +254,9 @@ __device__ __forceinline__ MdRes md_words_walk(const MdArgs& a, const MdTask& T,
     const int64_t p = T.k0 + y;
     uint32_t d[4];
     __builtin_memcpy(d, opac32 + (p >> 4), 16);
+    // base i of a dword's 16: bits 2i (high) and 2i + 1 (low)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) d[q] = __builtin_bitreverse32(__builtin_bswap32(d[q]));  // base i of 16: bits 2i (high), 2i + 1
+    for (int q = 0; q < 4; ++q) d[q] = __builtin_bitreverse32(__builtin_bswap32(d[q]));
     const uint32_t sh = 2u * (uint32_t)(p & 15);
     const uint32_t s0 = unshuffle(__builtin_amdgcn_alignbit(d[1], d[0], sh) ^ flip);
     const uint32_t s1 = unshuffle(__builtin_amdgcn_alignbit(d[2], d[1], sh) ^ flip);

@@ -447,7 +447,7 @@ ext_narrow_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block) {
   // the others at the back (back cursor, counting down from the end); the
   // other classes fill their lists from the front.  The front is the lane
   // frame kernel's list: longest run first, in row buckets, each rank placed
-  // in its fetch slice as in the lane-kernel bins.
+  // in its fetch slice, so that each slice is longest first.
   constexpr int NF = kLaneFrameClasses * kRowBuckets;
   __shared__ uint32_t off[kBandClasses], hist[kBandClasses], cur[kBandClasses];
   __shared__ uint32_t boff[kLaneFrameClasses], bhist[kLaneFrameClasses], bcur[kLaneFrameClasses];
@@ -518,8 +518,7 @@ static void launch_narrow_class(const ExtKArgs& k, const ExtWork& wk, int64_t n,
   if (blocks < 1) return;
   // Classes on separate streams, and the largest class's two kernels beside each
   // other (975,231 flanks of 150 bp reads in 24-column frames: 2.29 ms one after the
-  // other, 2.19 so); a timed
-  // class keeps to one stream.
+  // other, 2.19 so); a timed class keeps to one stream.
   const hipStream_t sl = pick_stream(wk.ss, st, CL == 3 ? 0 : CL + 1);
   const hipStream_t sg = CL == 0 && !wk.tev ? st : sl;
   time_begin(wk, time_slot_class(CL), sl);

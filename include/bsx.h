@@ -320,7 +320,8 @@ void bsx_graph_destroy(bsx_graph *graph);
  * bsx_kernel_times: waits, then writes the summed milliseconds per slot over
  * the recorded calls (slots 0..bins-1 = plain kernels by query-length bin,
  * then the 4 narrow classes, slot 15 = band predictor), the number of calls
- * in *calls, and starts a new recording.  bsx_ext_bin_limits writes the
+ * in *calls, and starts a new recording.  A timed call is binned whatever its
+ * size (untimed ones of up to 98304 tasks are not).  bsx_ext_bin_limits writes the
  * largest query length of each plain bin and returns the number of bins. */
 int bsx_set_kernel_timing(bsx_ctx *ctx, int max_calls);
 int bsx_kernel_times(bsx_ctx *ctx, float *ms, int n_slots, int *calls);
