@@ -178,14 +178,16 @@ constexpr int kBinStream[2][kExtBins] = {{0, 0, 0, 0, 0, 3, 2, 1, 0, 0, 1, 2}, {
 inline hipStream_t pick_stream(const StreamSet* ss, hipStream_t main, int k) {
   return (ss && k > 0 && ss->side[k - 1]) ? ss->side[k - 1] : main;
 }
-inline void ss_fork(const StreamSet* ss, hipStream_t main) {
+// side streams 1..n wait for the call's stream, and it for them (each costs the
+// device a few us of event handling)
+inline void ss_fork(const StreamSet* ss, hipStream_t main, int n = StreamSet::kSide) {
   if (!ss || !ss->fork) return;
   (void)hipEventRecord(ss->fork, main);
-  for (int k = 0; k < StreamSet::kSide; ++k) (void)hipStreamWaitEvent(ss->side[k], ss->fork, 0);
+  for (int k = 0; k < n; ++k) (void)hipStreamWaitEvent(ss->side[k], ss->fork, 0);
 }
-inline void ss_join(const StreamSet* ss, hipStream_t main) {
+inline void ss_join(const StreamSet* ss, hipStream_t main, int n = StreamSet::kSide) {
   if (!ss || !ss->fork) return;
-  for (int k = 0; k < StreamSet::kSide; ++k) {
+  for (int k = 0; k < n; ++k) {
     (void)hipEventRecord(ss->join[k], ss->side[k]);
     (void)hipStreamWaitEvent(main, ss->join[k], 0);
   }

@@ -332,8 +332,9 @@ ext_direct_kernel(ExtArgs A, ExtWork W) {
 // One launch with the registers of the widest task while the batch has at most
 // as many tasks as the chip holds such waves.  Beyond, the wide tasks run beside
 // the others: a long one takes milliseconds (4,000 flanks of 2 kb reads: 3.68 ms
-// after them, 2.26 beside), though the fork costs every other batch 20-27 us
-// (2,000 flanks of 100 bp reads: 69 without, 95 with).
+// after them, 2.26 beside), though the fork costs every other batch some 9 us
+// (2,000 flanks of 100 bp reads: 69 without, 78 with; 97 with a fork of all
+// three side streams).
 template <bool CERT>
 static void direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st) {
   const dim3 grid((unsigned)a.n), block(64);
@@ -342,10 +343,10 @@ static void direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t 
   } else if (a.n <= (int64_t)num_cu * 4 * wave_min_waves(32)) {
     hipLaunchKernelGGL((ext_direct_kernel<2, CERT>), grid, block, 0, st, a, wk);
   } else {
-    ss_fork(wk.ss, st);
+    ss_fork(wk.ss, st, 1);
     hipLaunchKernelGGL((ext_direct_kernel<0, CERT>), grid, block, 0, st, a, wk);
     hipLaunchKernelGGL((ext_direct_kernel<1, CERT>), grid, block, 0, pick_stream(wk.ss, st, 1), a, wk);
-    ss_join(wk.ss, st);
+    ss_join(wk.ss, st, 1);
   }
 }
 
