@@ -448,6 +448,23 @@ def host_buffer_leg(eng, batch, reps):
             "note": "host buffers in and out (bsx_extend_batch), plain form"}
 
 
+def plain_bins(batch, limits):
+    """Plain bin of every task under the default scoring (slots of
+    bsx.ext_bin_limits): by query length, past 256 bases by the columns of the
+    band where those are fewer, and apart where the pair kernels' 16-bit scores
+    or targets do not hold the task."""
+    from bsbolt_amd import bsx
+    Q = bsx.EXT_QUERY_BINS
+    ql, h0, w = (getattr(batch, k).astype(np.int64) for k in ("qlen", "h0", "w"))
+    w = np.minimum(w, np.maximum(ql + batch.end_bonus - 6 + 1, 1))  # ksw.c:399-407 with a = 1, o = 6, e = 1
+    pairs = sum(lanes == 1 for lanes, _ in bsx.EXT_SHAPES[:Q])
+    need = np.searchsorted(limits[:Q], ql)
+    for b in range(Q - 1, pairs - 1, -1):
+        need = np.where((need > b) & (2 * w + 1 + bsx.EXT_SHAPES[b][1] <= limits[b]), b, need)
+    out = (need < pairs) & ((batch.tlen > 640) | (h0 + ql > np.where(need < pairs - 1, 511, 255)))
+    return np.where(out, np.where(ql <= limits[Q], Q, np.where(ql <= limits[Q + 1], Q + 1, pairs)), need)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -562,11 +579,13 @@ def main():
     # dominant kernel: the plain bin with the most time; its algorithmic work is
     # the cells of the tasks in that bin
     limits = bsx.ext_bin_limits()
-    bin_of = np.searchsorted(limits, batch.qlen)
+    bin_of = plain_bins(batch, limits)
     per_launch = kms[:len(limits)] / max(kcalls, 1)
     dom = int(np.argmax(per_launch))
     lanes, cols = bsx.EXT_SHAPES[dom]
-    dom_name = f"ext_pair_kernel<{cols}, true>" if lanes == 1 else f"ext_wave_kernel<{cols}>"
+    dom_name = (f"ext_plain_kernel (queries of up to {limits[dom]} bases outside the pair kernels' range)"
+                if dom >= bsx.EXT_QUERY_BINS else
+                f"ext_pair_kernel<{cols}, true>" if lanes == 1 else f"ext_wave_kernel<{cols}>")
     dom_cells = int(cells[bin_of == dom].sum())
     dom_ms = float(per_launch[dom])
     dom_tops = dom_cells * OPS_PER_CELL / (dom_ms / 1e3) / 1e12
@@ -633,7 +652,8 @@ def main():
                      "ms_per_launch": dom_ms, "share_of_step_in_order": dom_ms / ms_in_order,
                      "ms_per_step_launches_in_order": ms_in_order,
                      "algorithmic_bytes_per_launch": dom_bytes,
-                     "kernel_ms_per_step": {f"bin<={int(l)}": float(t) for l, t in zip(limits, per_launch) if t > 0}},
+                     "kernel_ms_per_step": {f"{'bin' if b < bsx.EXT_QUERY_BINS else 'outside the pair range'}<={int(l)}":
+                                            float(t) for b, (l, t) in enumerate(zip(limits, per_launch)) if t > 0}},
         "roofline_step": {"bound": "valu", "achieved": tops, "peak": PEAK_PK16_TOPS, "unit": "TOP/s",
                           "frac": tops / PEAK_PK16_TOPS, "frac_int32": tops / PEAK_INT32_TOPS},
         "roofline_hbm": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",

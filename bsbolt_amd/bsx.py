@@ -41,9 +41,11 @@ EXPORTS = ("bsx_create", "bsx_destroy", "bsx_last_error", "bsx_set_stream", "bsx
            "bsx_extend_batch_device_noalloc", "bsx_ksw_global2", "bsx_reg2aln_cigar_device",
            "bsx_set_tuning", "bsx_get_tuning")
 TIMED_SLOTS = 16
-# lanes per task and columns per lane of the plain form's query-length bins (bsx_internal.h
-# kExtShape); one lane per task is the two-tasks-per-lane kernel
-EXT_SHAPES = ((1, 32), (1, 64), (1, 96), (1, 128), (1, 224), (64, 4), (64, 8), (64, 16), (64, 32))
+# lanes per task and columns per lane of the plain form's timed bins (include/bsx.h,
+# bsx_ext_bin_limits): nine by query length, where one lane per task is the
+# two-tasks-per-lane kernel, and the widest shapes of the two for tasks outside its range
+EXT_QUERY_BINS = 9
+EXT_SHAPES = ((1, 32), (1, 64), (1, 96), (1, 128), (1, 224), (64, 4), (64, 8), (64, 16), (64, 32), (16, 6), (32, 6))
 
 # learned-band form (include/bsx.h)
 BAND_PLAIN, BAND_LEARNED, BAND_FIXED = 0, 1, 2

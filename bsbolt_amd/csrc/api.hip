@@ -108,8 +108,8 @@ struct bsx_ctx {
   int adam_step = 0;
   int64_t last_n = 0;  // tasks of the last extension call (for bsx_band_stats)
   // per-kernel timing of the extension calls (bsx_set_kernel_timing)
-  std::vector<hipEvent_t> kt_ev;   // [calls][2 * kTimedSlots]
-  std::vector<uint32_t> kt_mask;   // [calls] slots recorded
+  std::vector<hipEvent_t> kt_ev;   // [calls][2 * kTimedLaunches]
+  std::vector<uint32_t> kt_mask;   // [calls] launches recorded
   int kt_calls = 0, kt_used = 0;
   int64_t zslot = 1 << 16;     // bytes per slot: largest min(qlen,2w+1)*tlen accepted
   // staging for the host-memory entry points
@@ -446,7 +446,7 @@ static int ext_buffers(bsx_ctx* c, size_t n) {
 static int extend_queue(bsx_ctx* c, const ExtArgs& a, ExtWork wk, uint8_t* cls) {
   const size_t n = (size_t)a.n;
   if (c->kt_used < c->kt_calls) {  // per-kernel timing of this call
-    wk.tev = &c->kt_ev[(size_t)c->kt_used * 2 * kTimedSlots];
+    wk.tev = &c->kt_ev[(size_t)c->kt_used * 2 * kTimedLaunches];
     wk.tmask = &c->kt_mask[c->kt_used];
     *wk.tmask = 0;
     ++c->kt_used;
@@ -454,9 +454,9 @@ static int extend_queue(bsx_ctx* c, const ExtArgs& a, ExtWork wk, uint8_t* cls) 
   BandPlan plan{kBandPlain, 0, nullptr, false, false};
   if (c->band_policy == BSX_BAND_LEARNED) {
     if (!c->model_ready) return fail(c, BSX_EINVAL, "learned band policy without a band model (bsx_band_model_set)");
-    time_begin(wk, kTimedSlots - 1, c->stream);
+    time_begin(wk, kTimePredict, c->stream);
     HIPCHK(c, mlp_launch_predict_tasks(a, model_view(c), cls, c->num_cu, c->stream), "band predict");
-    time_end(wk, kTimedSlots - 1, c->stream);
+    time_end(wk, kTimePredict, c->stream);
     plan = BandPlan{kBandLearned, 0, cls, false, false};
   } else if (c->band_policy == BSX_BAND_FIXED) {
     plan = BandPlan{kBandFixed, c->band_class, nullptr, true, false};
@@ -523,7 +523,7 @@ int bsx_set_kernel_timing(bsx_ctx* c, int max_calls) {
   if (!c || max_calls < 0 || max_calls > 4096) return fail(c, BSX_EINVAL, "max_calls must be in [0, 4096]");
   (void)hipSetDevice(c->device);
   HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-  const size_t need = (size_t)max_calls * 2 * kTimedSlots;
+  const size_t need = (size_t)max_calls * 2 * kTimedLaunches;
   while (c->kt_ev.size() < need) {
     hipEvent_t e;
     HIPCHK(c, hipEventCreate(&e), "hipEventCreate");
@@ -541,12 +541,12 @@ int bsx_kernel_times(bsx_ctx* c, float* ms, int n_slots, int* calls) {
   HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
   for (int s = 0; s < n_slots; ++s) ms[s] = 0.f;
   for (int k = 0; k < c->kt_used; ++k)
-    for (int s = 0; s < kTimedSlots && s < n_slots; ++s) {
-      if (!(c->kt_mask[k] >> s & 1u)) continue;
+    for (int x = 0; x < kTimedLaunches; ++x) {
+      if (!(c->kt_mask[k] >> x & 1u) || time_slot(x) >= n_slots) continue;
       float t = 0.f;
-      const hipEvent_t* e = &c->kt_ev[(size_t)k * 2 * kTimedSlots + 2 * s];
+      const hipEvent_t* e = &c->kt_ev[(size_t)k * 2 * kTimedLaunches + 2 * x];
       HIPCHK(c, hipEventElapsedTime(&t, e[0], e[1]), "hipEventElapsedTime");
-      ms[s] += t;
+      ms[time_slot(x)] += t;
     }
   if (calls) *calls = c->kt_used;
   c->kt_used = 0;
@@ -554,9 +554,9 @@ int bsx_kernel_times(bsx_ctx* c, float* ms, int n_slots, int* calls) {
 }
 
 int bsx_ext_bin_limits(int32_t* limits, int n) {
-  if (!limits) return kQueryBins;
-  for (int b = 0; b < kQueryBins && b < n; ++b) limits[b] = bin_limit(b);
-  return kQueryBins;
+  if (!limits) return kTimedBins;
+  for (int b = 0; b < kTimedBins && b < n; ++b) limits[b] = timed_bin_limit(b);
+  return kTimedBins;
 }
 
 int bsx_set_band_policy(bsx_ctx* c, int policy, int band_class) {

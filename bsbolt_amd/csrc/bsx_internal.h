@@ -209,9 +209,9 @@ struct ExtWork {
   uint32_t* bcursor;   // [kExtBins * kRowBuckets] scatter cursors of the same
   uint32_t* fcount;    // [kLaneFrameClasses * kRowBuckets] front tasks per lane-frame class and row bucket
   uint32_t* fcursor;   // [kLaneFrameClasses * kRowBuckets] scatter cursors of the same
-  // optional per-kernel timing: events [2*slot], [2*slot+1] around each kernel
-  // launch (slots: plain bins, then narrow classes, then the predictor); *tmask
-  // gets bit `slot` set for every pair recorded
+  // optional per-kernel timing: events [2*x], [2*x+1] around timed launch x
+  // (time_of_bin, time_of_class, kTimePredict); *tmask gets bit x set for every
+  // pair recorded
   hipEvent_t* tev = nullptr;
   uint32_t* tmask = nullptr;
   const StreamSet* ss = nullptr;  // side streams (nullable: everything on the call's stream)
@@ -246,19 +246,32 @@ static_assert(kExtShape[kTunedBin[0]].lanes == kAltShape[0][0].lanes &&
               kExtShape[kTunedBin[1]].cols == kAltShape[1][0].cols &&
               kAltShape[0][1].lanes * kAltShape[0][1].cols == bin_limit(kTunedBin[0]) &&
               kAltShape[1][1].lanes * kAltShape[1][1].cols == bin_limit(kTunedBin[1]), "alternative shapes");
-// timing slots: the plain bins (the last one is not timed), the narrow classes,
-// and the predictor last
-constexpr int kTimedSlots = 16;
-constexpr int time_slot_bin(int b) { return b < 11 ? b : -1; }
-constexpr int time_slot_class(int c) { return 11 + c; }
-static_assert(11 + kBandClasses <= kTimedSlots, "timing slots");
-inline void time_begin(const ExtWork& wk, int slot, hipStream_t st) {
-  if (wk.tev && slot >= 0) (void)hipEventRecord(wk.tev[2 * slot], st);
+// Timed launches: the plain bins, the narrow classes, the predictor.
+constexpr int kTimedLaunches = kExtBins + kBandClasses;
+constexpr int time_of_bin(int b) { return b; }
+constexpr int time_of_class(int c) { return kExtBins + c; }
+constexpr int kTimePredict = kTimedLaunches - 1;
+static_assert(kTimedLaunches <= 32, "one mask bit per timed launch");
+// Slots of bsx_kernel_times, several bins to one where a caller need not tell
+// them apart: the query bins, the bins of tasks outside the pair kernel's range
+// (those of short queries, then the others), the narrow classes, the predictor.
+constexpr int kTimedSlots = 16, kTimedBins = kQueryBins + 2, kOutsideShort = 96;
+static_assert(kTimedBins + kBandClasses == kTimedSlots, "timing slots");
+constexpr int time_slot(int launch) {
+  return launch < kQueryBins ? launch
+         : launch < kExtBins ? kQueryBins + (bin_limit(launch) > kOutsideShort ? 1 : 0)
+                             : kTimedBins + launch - kExtBins;
 }
-inline void time_end(const ExtWork& wk, int slot, hipStream_t st) {
-  if (wk.tev && slot >= 0) {
-    (void)hipEventRecord(wk.tev[2 * slot + 1], st);
-    *wk.tmask |= 1u << slot;
+constexpr int timed_bin_limit(int s) {
+  return s < kQueryBins ? bin_limit(s) : s == kQueryBins ? kOutsideShort : bin_limit(kExtBins - 1);
+}
+inline void time_begin(const ExtWork& wk, int launch, hipStream_t st) {
+  if (wk.tev) (void)hipEventRecord(wk.tev[2 * launch], st);
+}
+inline void time_end(const ExtWork& wk, int launch, hipStream_t st) {
+  if (wk.tev) {
+    (void)hipEventRecord(wk.tev[2 * launch + 1], st);
+    *wk.tmask |= 1u << launch;
   }
 }
 

@@ -503,10 +503,10 @@ static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int nu
   k.tpb = (int)std::min<int64_t>(k.tpb, std::max<int64_t>(64 / L, fill));
   const int64_t blocks = std::min<int64_t>((n + k.tpb - 1) / k.tpb, (int64_t)num_cu * kMaxBlocksPerCu);
   if (blocks < 1) return;
-  time_begin(wk, time_slot_bin(B), st);
+  time_begin(wk, time_of_bin(B), st);
   hipLaunchKernelGGL((ext_plain_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, st, k,
                      (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B);
-  time_end(wk, time_slot_bin(B), st);
+  time_end(wk, time_of_bin(B), st);
 }
 
 template <int B, bool E1>

@@ -521,12 +521,12 @@ static void launch_narrow_class(const ExtKArgs& k, const ExtWork& wk, int64_t n,
   // other, 2.19 so); a timed class keeps to one stream.
   const hipStream_t sl = pick_stream(wk.ss, st, CL == 3 ? 0 : CL + 1);
   const hipStream_t sg = CL == 0 && !wk.tev ? st : sl;
-  time_begin(wk, time_slot_class(CL), sl);
+  time_begin(wk, time_of_class(CL), sl);
   if constexpr (CL < kLaneFrameClasses) launch_lane_frame<frame_of_class(CL), E1>(k, wk, CL, num_cu, sl);
   hipLaunchKernelGGL((ext_narrow_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, sg, k,
                      (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, (const uint32_t*)wk.split, CL,
                      wk.need_plain);
-  time_end(wk, time_slot_class(CL), sg);
+  time_end(wk, time_of_class(CL), sg);
 }
 
 template <bool E1>

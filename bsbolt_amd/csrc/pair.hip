@@ -369,11 +369,11 @@ template <int Q>
 void launch_pair_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, hipStream_t st) {
   const int64_t blocks = (n + 127) / 128;  // surplus blocks exit at once
   if (blocks < 1) return;
-  time_begin(wk, time_slot_bin(bin), st);
+  time_begin(wk, time_of_bin(bin), st);
   const bool same = k.o_del + k.e_del == k.o_ins + k.e_ins;  // one gap-open value serves E and F
   hipLaunchKernelGGL((same ? ext_pair_kernel<Q, true> : ext_pair_kernel<Q, false>), dim3((unsigned)blocks), dim3(64),
                      0, st, k, (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, bin);
-  time_end(wk, time_slot_bin(bin), st);
+  time_end(wk, time_of_bin(bin), st);
 }
 template void launch_pair_bin<32>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);
 template void launch_pair_bin<64>(const ExtKArgs&, const ExtWork&, int, int64_t, hipStream_t);

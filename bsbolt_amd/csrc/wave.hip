@@ -263,10 +263,10 @@ void launch_wave_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, i
   // as many as are resident: surplus blocks of an empty bin cost 9 us a launch
   const int64_t blocks = std::min<int64_t>(n, (int64_t)num_cu * 4 * wave_min_waves(C));
   if (blocks < 1) return;
-  time_begin(wk, time_slot_bin(bin), st);
+  time_begin(wk, time_of_bin(bin), st);
   hipLaunchKernelGGL(ext_wave_kernel<C>, dim3((unsigned)blocks), dim3(64), 0, st, k, (const ExtDesc*)wk.desc,
                      (const uint32_t*)wk.counts, bin);
-  time_end(wk, time_slot_bin(bin), st);
+  time_end(wk, time_of_bin(bin), st);
 }
 template void launch_wave_bin<4>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);
 template void launch_wave_bin<8>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);

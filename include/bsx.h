@@ -318,11 +318,16 @@ void bsx_graph_destroy(bsx_graph *graph);
  * bsx_set_kernel_timing(ctx, k): the next k extension calls on the context
  * record HIP events around each kernel launch (0 switches it off).
  * bsx_kernel_times: waits, then writes the summed milliseconds per slot over
- * the recorded calls (slots 0..bins-1 = plain kernels by query-length bin,
- * then the 4 narrow classes, slot 15 = band predictor), the number of calls
- * in *calls, and starts a new recording.  A timed call is binned whatever its
- * size (untimed ones of up to 98304 tasks are not).  bsx_ext_bin_limits writes the
- * largest query length of each plain bin and returns the number of bins. */
+ * the recorded calls (slots 0..bins-1 = plain kernels, bins being what
+ * bsx_ext_bin_limits returns; then the 4 narrow classes; slot 15 = band
+ * predictor), the number of calls in *calls, and starts a new recording.  A
+ * timed call is binned whatever its size (untimed ones of up to 98304 tasks are
+ * not).  bsx_ext_bin_limits writes the largest query length of each plain bin and
+ * returns the number of bins, 11: nine by query length (past 256 bases by the
+ * columns of the band, where those are fewer), then two for the queries of up to
+ * 96 and of up to 192 bases that the two-tasks-per-lane kernels do not take (a
+ * batch below 65536 tasks, or scores, targets or gap costs outside their 16-bit
+ * range). */
 int bsx_set_kernel_timing(bsx_ctx *ctx, int max_calls);
 int bsx_kernel_times(bsx_ctx *ctx, float *ms, int n_slots, int *calls);
 int bsx_ext_bin_limits(int32_t *limits, int n);
