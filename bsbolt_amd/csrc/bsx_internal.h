@@ -8,17 +8,19 @@ namespace bsx {
 // Extension work is split into bins by query length; each bin runs a kernel
 // instantiation.  Index = bin id.  Shape (1, Q) is the two-tasks-per-lane
 // kernel (pair.hip, queries of at most Q bases); shape (64, C) the wave kernel
-// (wave.hip, queries or bands of at most 64*C columns); other shapes (L, C) a group
-// kernel with L lanes per task and C query columns per lane (qlen <= L*C).  The bins
-// from kQueryBins on take the queries of the pair bins where the pair kernel
-// does not run them: batches below kPairMinTasks and tasks outside its range
-// (pair_takes).
-constexpr int kExtBins = 12;
+// (wave.hip, queries or bands of at most 64*C columns).  The bins from
+// kQueryBins on take the queries of the pair bins where the pair kernel does not
+// run them: batches below kPairMinTasks and tasks outside its range (pair_takes).
+// Their shape (1, Q) is the task-per-lane kernel (lane.hip), other shapes (L, C) a
+// group kernel with L lanes per task and C query columns per lane (qlen <= L*C).
+constexpr int kExtBins = 14;
 constexpr int kPairBins = 5;
-constexpr int kQueryBins = 9;  // bins told apart by query length alone
+constexpr int kQueryBins = 9;  // bins of the pair and the wave kernels
+constexpr int kLaneBins = 2;   // bins of the task-per-lane kernel, after them
 struct BinShape { int lanes, cols; };
-constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}, {1, 224}, {64, 4},
-                                          {64, 8}, {64, 16}, {64, 32}, {16, 6},  {16, 8},  {32, 6}};
+constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}, {1, 224}, {64, 4}, {64, 8},
+                                          {64, 16}, {64, 32}, {1, 32},  {1, 64},  {16, 6},  {16, 8}, {32, 6}};
+constexpr bool is_lane_bin(int b) { return b >= kQueryBins && b < kQueryBins + kLaneBins; }
 constexpr int kExtBlock = 64;             // threads per extension block: one wave, so a block
                                           // never holds wave slots idle while a sibling finishes
 constexpr int kExtTasksPerBlock = 32;     // task descriptors owned by one plain-kernel block
@@ -32,7 +34,7 @@ constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; 
 constexpr int kGlbBins = 8;
 constexpr BinShape kGlbShape[kGlbBins] = {
     {8, 2}, {8, 3}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
-constexpr int kExtSlices = 8;  // fetch-counter slots per bin (CIGAR bins, lane frame classes)
+constexpr int kExtSlices = 8;  // fetch-counter slots per lane bin and lane frame class (a CIGAR bin uses one)
 // Bins of the two-tasks-per-lane CIGAR kernel (gpair.hip), after the others:
 // band widths 2w+1 up to kGlbPairCols, each from glb_pair_top + 1 on.
 constexpr int kGlbPairBins = 5;
@@ -82,7 +84,7 @@ __host__ __device__ inline uint32_t slice_begin(uint32_t n, int s) {
 // bucketed in steps of 8 rows up to 192 and of 32 beyond, bucket 0 = longest.
 // Steps of 32 throughout cost the pair kernels a quarter to a third more rows
 // (the waves of a bucket all run as long as its longest run); steps of 4
-// changed nothing.  The lane frame kernel's lists place rank r of that order at
+// changed nothing.  The lists of the lane kernels place rank r of that order at
 // slot r / kExtSlices of fetch slice r % kExtSlices, so that every slice is
 // itself longest first.  The order changes no result.
 constexpr int kRowBuckets = 32;
@@ -97,7 +99,7 @@ __host__ __device__ inline int row_bucket(int tlen, int h0) {
 // [0, kExtBins), narrow classes [kExtBins, kExtBins + kBandClasses - 1).
 constexpr int kBandClasses = 5;
 constexpr int kFrameWidth[kBandClasses - 1] = {24, 40, 80, 144};
-constexpr int kCountSlots = 16;
+constexpr int kCountSlots = 20;
 static_assert(kExtBins + kBandClasses - 1 <= kCountSlots, "count slots for bins and narrow classes");
 constexpr int kNarrowQMax = 256;  // longest query the narrow kernels take
 // Frame classes run by the lane-per-task frame kernel (one task per lane) for
@@ -174,7 +176,8 @@ struct StreamSet {
 };
 // streams of the plain bins' launches, without and with the pair kernels: 0 =
 // the call's stream, k > 0 = side[k-1]
-constexpr int kBinStream[2][kExtBins] = {{0, 0, 0, 0, 0, 3, 2, 1, 0, 0, 1, 2}, {0, 3, 2, 1, 0, 3, 2, 1, 3, 3, 1, 2}};
+constexpr int kBinStream[2][kExtBins] = {{0, 0, 0, 0, 0, 3, 2, 1, 0, 3, 1, 0, 2, 3},
+                                         {0, 3, 2, 1, 0, 3, 2, 1, 3, 2, 1, 3, 1, 2}};
 inline hipStream_t pick_stream(const StreamSet* ss, hipStream_t main, int k) {
   return (ss && k > 0 && ss->side[k - 1]) ? ss->side[k - 1] : main;
 }
@@ -238,7 +241,7 @@ inline void ext_counters(ExtWork& wk, uint32_t* p) {
 // Bins with alternative group shapes (same columns per task, so the binning is
 // unchanged; the tuner picks one per device): index 0 = queries of at most 96
 // bases, 1 = queries of 97-128.  Variant 0 is kExtShape's shape.
-constexpr int kTunedBin[2] = {9, 10};
+constexpr int kTunedBin[2] = {11, 12};
 constexpr BinShape kAltShape[2][2] = {{{16, 6}, {32, 3}}, {{16, 8}, {32, 4}}};
 static_assert(kExtShape[kTunedBin[0]].lanes == kAltShape[0][0].lanes &&
               kExtShape[kTunedBin[0]].cols == kAltShape[0][0].cols &&
@@ -289,6 +292,9 @@ void launch_wave_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, i
 // 330, 80,000 1521 / 2693, 128,000 2925 / 2741.
 constexpr int64_t kDirectMaxTasks = 98304;
 void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, bool cert);
+// task-per-lane kernel of bin `bin` (queries of at most Q bases)
+template <int Q, bool E1>
+void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st);
 // lane-per-task frame kernel (frame of WF columns) of lane-frame class `cls`
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st);

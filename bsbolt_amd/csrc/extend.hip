@@ -1,8 +1,9 @@
 // Bit-exact batched ksw_extend2 (bsbolt/External/BWA/ksw.c:380-479) for gfx950.
 //
-// This file holds the group kernel, for queries of up to 192 bases in batches or
-// tasks that the pair kernel (pair.hip) does not take; the wave kernel (wave.hip)
-// takes longer ones and small batches.
+// This file holds the group kernel, for queries of 65-192 bases in batches or
+// tasks that the pair kernel (pair.hip) does not take; the task-per-lane kernel
+// (lane.hip) takes shorter ones of these, the wave kernel (wave.hip) longer ones
+// and small batches.
 //
 // Layout.  A task is owned by a group of L lanes (L = 16 or 32; 64/L tasks
 // per wave64); lane g holds query columns [g*C, g*C+C) of the DP state in VGPRs:
@@ -428,11 +429,11 @@ ext_bin_count_kernel(ExtArgs A, ExtWork W, int mode) {
 // row bucket in LDS, reserves one range per (bin, bucket) with a single global
 // atomic, and writes the descriptors of its tasks into those ranges.  A task's
 // rank in its bin's longest-first order is its bucket's base plus its place in
-// the bucket.
+// the bucket; lane bins spread the ranks over the fetch slices.
 __global__ void __launch_bounds__(256)
 ext_bin_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block, const uint8_t* __restrict__ need) {
   constexpr int NB = kExtBins * kRowBuckets;
-  __shared__ uint32_t off[NB], hist[NB], cur[NB], lbase[kExtBins];
+  __shared__ uint32_t off[NB], hist[NB], cur[NB], lbase[kExtBins], lsize[kExtBins];
   const int64_t t0 = (int64_t)blockIdx.x * per_block;
   const int64_t t1 = min(A.n, t0 + per_block);
   for (int k = threadIdx.x; k < NB; k += blockDim.x) { hist[k] = 0; cur[k] = 0; }
@@ -454,6 +455,7 @@ ext_bin_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block, const uint8_t* _
     uint32_t s = 0;
     for (int b = 0; b < (int)threadIdx.x; ++b) s += W.counts[b];
     lbase[threadIdx.x] = s;
+    lsize[threadIdx.x] = W.counts[threadIdx.x];
   }
   __syncthreads();
   for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
@@ -461,7 +463,8 @@ ext_bin_scatter_kernel(ExtArgs A, ExtWork W, int64_t per_block, const uint8_t* _
     if (b == 0xff || (need && !need[t])) continue;
     const int kb = b * kRowBuckets + row_bucket(A.tlen[t], A.h0[t]);
     const uint32_t r = off[kb] + atomicAdd(&cur[kb], 1u);
-    write_desc(A, t, W.desc + lbase[b] + r);
+    const uint32_t p = is_lane_bin(b) ? slice_begin(lsize[b], (int)(r % kExtSlices)) + r / kExtSlices : r;
+    write_desc(A, t, W.desc + lbase[b] + p);
   }
 }
 
@@ -516,6 +519,8 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
     if (pair) launch_pair_bin<C>(k, wk, B, n, st);
   } else if constexpr (B < kQueryBins) {
     launch_wave_bin<C>(k, wk, B, n, num_cu, st);
+  } else if constexpr (is_lane_bin(B)) {
+    launch_lane_bin<C, E1>(k, wk, B, n, num_cu, st);
   } else if constexpr (B == kTunedBin[0] || B == kTunedBin[1]) {
     constexpr int V = B == kTunedBin[0] ? 0 : 1;
     if (wk.shape_var[V] == 1)
@@ -534,11 +539,12 @@ static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num
 }
 // The 224-column kernel first, on the call's own stream: its waves need a SIMD
 // to themselves and wait for long once smaller ones are spread over all of them.
-// Then the group bins, nearly empty in a batch with pair bins: behind a pair
-// kernel even an empty launch waits until the chip has room for its blocks (0.5
-// ms for one of 250 bp reads).
-using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 11, 10, 9, 3, 2, 1, 0>;
-static_assert(kExtBins == 12, "launch order");
+// Then the bins of tasks outside the pair kernels' range, mostly empty under
+// BSBolt's scoring with reads of up to 250 bases: behind a pair kernel even an
+// empty launch waits until the chip has room for its blocks (0.5 ms for one of
+// 250 bp reads).
+using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 13, 12, 11, 10, 9, 3, 2, 1, 0>;
+static_assert(kExtBins == 14, "launch order");
 
 static void launch_unpack(const ExtArgs& a, const ExtWork& wk, int64_t blocks, hipStream_t st) {
   hipLaunchKernelGGL(ext_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, wk, (const int32_t*)wk.rec);

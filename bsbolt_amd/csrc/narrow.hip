@@ -43,16 +43,15 @@ static_assert(frame_of_class(0) == kFrameWidth[0] && frame_of_class(1) == kFrame
 
 // Measured cost of one DP row per task on MI355X (picoseconds of kernel time
 // per row over a 150 bp paired-end bisulfite batch, each kernel run alone):
-// the plain form's bins (the pair kernels, the wave kernels, then the group
-// kernels) and the
-// frame classes (lane-per-task frames of 24 and
+// the plain form's bins (the pair, the wave, the task-per-lane, then the group
+// kernels) and the frame classes (lane-per-task frames of 24 and
 // 40 columns -- upper bounds, from the rows of the runs that completed --
 // and group frames of 80 and 144 columns).  A task goes to its predicted frame
 // class only where that class is at least 20% cheaper per row than the plain
 // bin of its query length.
-constexpr int kPlainRowPs[kExtBins] = {15, 22, 32, 55, 240, 255, 465, 830, 1500, 109, 158, 600};
+constexpr int kPlainRowPs[kExtBins] = {15, 22, 32, 55, 240, 255, 465, 830, 1500, 43, 59, 109, 158, 600};
 constexpr int kFrameRowPs[kBandClasses - 1] = {29, 75, 152, 239};
-static_assert(kExtBins == 12 && kBandClasses == 5, "row cost tables");
+static_assert(kExtBins == 14 && kBandClasses == 5, "row cost tables");
 __host__ __device__ constexpr bool narrow_pays(int c, int b) {
   return 10 * kFrameRowPs[c] < 8 * kPlainRowPs[b];
 }
