@@ -23,7 +23,7 @@ constexpr BinShape kExtShape[kExtBins] = {{1, 32},  {1, 64},  {1, 96},  {1, 128}
 constexpr bool is_lane_bin(int b) { return b >= kQueryBins && b < kQueryBins + kLaneBins; }
 constexpr int kExtBlock = 64;             // threads per extension block: one wave, so a block
                                           // never holds wave slots idle while a sibling finishes
-constexpr int kExtTasksPerBlock = 32;     // task descriptors owned by one plain-kernel block
+constexpr int kExtTasksPerBlock = 32;     // four times the task descriptors a plain-kernel block fetches at a time
 constexpr int kNarrowTasksPerBlock = 16;  // ... by one narrow-kernel block
 constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; }
 
@@ -218,8 +218,8 @@ struct ExtWork {
   hipEvent_t* tev = nullptr;
   uint32_t* tmask = nullptr;
   const StreamSet* ss = nullptr;  // side streams (nullable: everything on the call's stream)
-  // tuning: descriptors per block of the plain group kernels and of the frame
-  // group kernels, and the shape variant of the bins with alternatives
+  // tuning: four times the chunk of the plain group kernels, descriptors per block
+  // of the frame group kernels, and the shape variant of the bins with alternatives
   int tpb_plain = kExtTasksPerBlock, tpb_narrow = kNarrowTasksPerBlock;
   int shape_var[2] = {0, 0};
 };
@@ -294,7 +294,7 @@ constexpr int64_t kDirectMaxTasks = 98304;
 void launch_direct(const ExtArgs& a, const ExtWork& wk, int num_cu, hipStream_t st, bool cert);
 // task-per-lane kernel of bin `bin` (queries of at most Q bases)
 template <int Q, bool E1>
-void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st);
+void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st, bool pair);
 // lane-per-task frame kernel (frame of WF columns) of lane-frame class `cls`
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st);

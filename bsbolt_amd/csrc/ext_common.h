@@ -71,7 +71,8 @@ struct ExtKArgs {
   int32_t prof_hi[5];   // by query code q: mat[20+q]
   uint32_t trow_lo[5];  // by target code t: bytes q = 0..3 hold mat[t*5+q]
   uint32_t trow_hi[5];  // by target code t: byte 0 holds mat[t*5+4]
-  int tpb;              // task descriptors owned by one block
+  int tpb;              // frame group kernels: task descriptors owned by one block
+  int chunk;            // plain group kernels: task descriptors a block fetches at a time
   int mat_max;          // largest substitution score, at least 0
 };
 

@@ -31,15 +31,14 @@
 // H(i, -1) = the first-column value of ksw.c:421-424.
 //
 // Work distribution.  Tasks are binned by their columns (ext_bin_of);
-// the binning pass writes one 48-byte descriptor per task in bin order.  Block
-// k of a bin's launch owns descriptors [k*T, k*T+T); its groups take them one
-// at a time through an LDS counter, so no device-scope atomic is on the task
-// path (same-address device atomics serialise at a few per microsecond) and the
-// hardware dispatcher balances the blocks.  The next task's descriptor, query
-// bases and first target word are loaded one task ahead, so a task starts
-// without a memory round trip.  Groups run a flattened loop (start-task-or-row
-// per iteration) so the groups of a wave never wait for one another between
-// tasks.
+// the binning pass writes one 48-byte descriptor per task in bin order.  A block
+// (one wave) takes them in chunks of a few; its groups take a chunk's one at a
+// time through an LDS counter, so only one device-scope atomic a chunk is on the
+// task path (same-address device atomics serialise at a few per microsecond).  The
+// next task's descriptor, query bases and first target word are loaded one task
+// ahead, so a task starts without a memory round trip.  Groups run a flattened
+// loop (start-task-or-row per iteration) so the groups of a wave never wait for
+// one another between tasks.
 #include <algorithm>
 #include <utility>
 
@@ -48,30 +47,35 @@
 
 namespace bsx {
 
-
-
 // waves per SIMD the register budget must allow (4 keeps VGPRs <= 128)
 constexpr int plain_min_waves(int C) { return C <= 6 ? 4 : 3; }
 
 template <int L, int C, bool E1>
 __global__ void __launch_bounds__(kExtBlock, plain_min_waves(C))
-ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t* __restrict__ counts,
-                 int bin) {
-  __shared__ uint32_t lds_next;
+ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t* __restrict__ counts, int bin,
+                 uint32_t* __restrict__ fetch) {
+  __shared__ uint32_t lds_next;      // descriptors of the block's chunks handed out
+  __shared__ uint32_t lds_first[4];  // chunk c of the block starts at lds_first[c & 3]
   const int lane = threadIdx.x & 63;
   const int lig = lane & (L - 1);
   const int base = lig * C;
   uint32_t lbase = 0;
   for (int b = 0; b < bin; ++b) lbase += counts[b];
   const uint32_t nlist = counts[bin];
-  // The grid is capped (most bins of a large batch are small, and a launch's
-  // surplus blocks are not free: 122,000 empty ones took 27-54 us a bin), so a
-  // block owns more than one chunk of tpb descriptors where the bin is large.
-  const uint32_t tpb = max((uint32_t)A.tpb, (nlist + gridDim.x - 1) / gridDim.x);
-  const uint32_t blk0 = blockIdx.x * tpb;
-  if (blk0 >= nlist) return;  // uniform over the block
-  const uint32_t blk1 = min(blk0 + tpb, nlist);
-  if (threadIdx.x == 0) lds_next = blk0;
+  // The grid is as large as the chip (launch_group).  A list that gives each block
+  // no more than a chunk is shared out evenly; of a longer one block k takes chunk
+  // k and fetches the others, longest first like the list.  With fixed shares of a
+  // long list the chip waits for the blocks of its front: 1,000,000 flanks of
+  // 129-144 bases outside the pair range 62.7 ms, so 49.4; with 32 descriptors at a
+  // time 53.0, 16 50.0, 8 49.2.
+  const uint32_t chunk = (uint32_t)A.chunk;
+  const bool more = nlist > gridDim.x * chunk;
+  const uint32_t take = more ? chunk : max(64u / L, (nlist + gridDim.x - 1) / gridDim.x);
+  if (blockIdx.x * take >= nlist) return;  // uniform over the block
+  if (threadIdx.x == 0) {
+    lds_next = 0;
+    lds_first[0] = blockIdx.x * take;
+  }
   __syncthreads();
   const ExtDesc* __restrict__ desc = desc_all + lbase;
   // E1: both gap extensions are 1 (BSBolt's -E 1,1), so the per-column
@@ -79,15 +83,23 @@ ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_
   const int e_del = E1 ? 1 : A.e_del, e_ins = E1 ? 1 : A.e_ins;
   const int oe_del = A.o_del + e_del, oe_ins = A.o_ins + e_ins;
 
-  // next descriptor position for this group; blk1 once the block's range is taken
+  // next descriptor position for this group; nlist once the block's are taken
   auto next_pos = [&]() -> uint32_t {
     // Branch-free fetch: every lane issues the atomic and only lane 0 of the
     // group adds 1.  No lane-divergent region may precede the broadcast: with
     // `if (lig == 0)` around the atomic the compiler can give the other lanes a
     // loop of their own that reaches the broadcast without lane 0's new value.
     const uint32_t mine = atomicAdd(&lds_next, lig == 0 ? 1u : 0u);
-    const uint32_t p = __shfl(mine, 0, L);
-    return p < blk1 ? p : blk1;
+    const uint32_t x = (uint32_t)__shfl((int)mine, 0, L), c = x / take, r = x - c * take;
+    // The first task of a chunk fetches the next one.  At most 64 / L <= chunk tasks
+    // are handed out at once, so a chunk is known before its first task is.
+    // (Branch-free over the group's lanes, like the count above.)
+    if (more && r == 0) {
+      const uint32_t got = atomicAdd(fetch, lig == 0 ? 1u : 0u);
+      lds_first[(c + 1) & 3] = (gridDim.x + (uint32_t)__shfl((int)got, 0, L)) * chunk;
+    }
+    const uint32_t p = more || c == 0 ? lds_first[c & 3] + r : nlist;
+    return min(p, nlist);
   };
 
   // ---- two-stage prefetch ----
@@ -99,8 +111,8 @@ ext_plain_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_
   int4 d2a = make_int4(0, 0, 0, 0), d2b = d2a, d2c = d2a;
   auto load_desc = [&]() {
     const uint32_t p = next_pos();
-    d2_ok = p < blk1;
-    const int4* d = (const int4*)(desc + (d2_ok ? p : blk0));
+    d2_ok = p < nlist;
+    const int4* d = (const int4*)(desc + (d2_ok ? p : blockIdx.x));
     d2a = d[0]; d2b = d[1]; d2c = d[2];
   };
   bool nx_ok = false;
@@ -493,22 +505,18 @@ ext_unpack_kernel(ExtArgs A, ExtWork W, const int32_t* __restrict__ rec) {
   }
 }
 
-// One block per tpb descriptors of bin B; the grid covers the whole batch and
-// surplus blocks exit at once (the host does not know the bin's count).  The
-// tuned tpb suits batches that fill the chip; below that a block takes only as
-// many tasks as leave every SIMD kBlocksPerSimd blocks, at least one per group:
-// with 32 per block, 500 flanks of 150 bp reads ran in 16 (1.11 ms, so 0.24).
+// As many blocks as the chip holds, or as give every group of the batch one task:
+// most bins of a large batch are nearly empty, and a launch's surplus blocks are
+// not free (1,000,000 flanks of 150 bp reads 1.38 ms with 16 blocks a CU, 1.58 with
+// 24 or more; 122,000 empty ones took 27-54 us a bin).
 template <int L, int C, bool E1>
-static void launch_group(ExtKArgs k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st, bool pair) {
-  constexpr int64_t kBlocksPerSimd = 4;
-  const int64_t kMaxBlocksPerCu = pair ? 16 : 128;
-  const int64_t fill = n / (num_cu * 4 * kBlocksPerSimd);
-  k.tpb = (int)std::min<int64_t>(k.tpb, std::max<int64_t>(64 / L, fill));
-  const int64_t blocks = std::min<int64_t>((n + k.tpb - 1) / k.tpb, (int64_t)num_cu * kMaxBlocksPerCu);
+static void launch_group(const ExtKArgs& k, const ExtWork& wk, int B, int64_t n, int num_cu, hipStream_t st) {
+  constexpr int64_t kBlocksPerCu = 16;
+  const int64_t blocks = std::min<int64_t>((n + 64 / L - 1) / (64 / L), num_cu * kBlocksPerCu);
   if (blocks < 1) return;
   time_begin(wk, time_of_bin(B), st);
   hipLaunchKernelGGL((ext_plain_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, st, k,
-                     (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B);
+                     (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B, wk.fetch + B * kExtSlices);
   time_end(wk, time_of_bin(B), st);
 }
 
@@ -520,15 +528,15 @@ static void launch_bin(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num_
   } else if constexpr (B < kQueryBins) {
     launch_wave_bin<C>(k, wk, B, n, num_cu, st);
   } else if constexpr (is_lane_bin(B)) {
-    launch_lane_bin<C, E1>(k, wk, B, n, num_cu, st);
+    launch_lane_bin<C, E1>(k, wk, B, n, num_cu, st, pair);
   } else if constexpr (B == kTunedBin[0] || B == kTunedBin[1]) {
     constexpr int V = B == kTunedBin[0] ? 0 : 1;
     if (wk.shape_var[V] == 1)
-      launch_group<kAltShape[V][1].lanes, kAltShape[V][1].cols, E1>(k, wk, B, n, num_cu, st, pair);
+      launch_group<kAltShape[V][1].lanes, kAltShape[V][1].cols, E1>(k, wk, B, n, num_cu, st);
     else
-      launch_group<L, C, E1>(k, wk, B, n, num_cu, st, pair);
+      launch_group<L, C, E1>(k, wk, B, n, num_cu, st);
   } else {
-    launch_group<L, C, E1>(k, wk, B, n, num_cu, st, pair);
+    launch_group<L, C, E1>(k, wk, B, n, num_cu, st);
   }
 }
 
@@ -542,8 +550,10 @@ static void launch_bins(const ExtKArgs& k, const ExtWork& wk, int64_t n, int num
 // Then the bins of tasks outside the pair kernels' range, mostly empty under
 // BSBolt's scoring with reads of up to 250 bases: behind a pair kernel even an
 // empty launch waits until the chip has room for its blocks (0.5 ms for one of
-// 250 bp reads).
-using BinOrder = std::integer_sequence<int, 4, 8, 7, 6, 5, 13, 12, 11, 10, 9, 3, 2, 1, 0>;
+// 250 bp reads).  The 64-base lane kernel goes ahead of the group kernels, whose
+// waves would leave no SIMD the registers for its own (100,000 flanks of 150 bp
+// reads with 600 added to their scores 2.08 ms behind them, 1.45 ahead).
+using BinOrder = std::integer_sequence<int, 4, 10, 8, 7, 6, 5, 13, 12, 11, 9, 3, 2, 1, 0>;
 static_assert(kExtBins == 14, "launch order");
 
 static void launch_unpack(const ExtArgs& a, const ExtWork& wk, int64_t blocks, hipStream_t st) {
@@ -567,7 +577,7 @@ hipError_t launch_extend(ExtArgs a, const ExtWork& wk, int num_cu, hipStream_t s
   ExtKArgs k{};
   k.query = a.query; k.target = a.target; k.rec = wk.rec;
   k.o_del = a.o_del; k.e_del = a.e_del; k.o_ins = a.o_ins; k.e_ins = a.e_ins; k.zdrop = a.zdrop;
-  k.tpb = wk.tpb_plain;
+  k.chunk = std::max(4, wk.tpb_plain / 4);
   k.mat_max = a.mat_max;
   for (int q = 0; q < 5; ++q) { k.prof_lo[q] = a.prof_lo[q]; k.prof_hi[q] = a.prof_hi[q]; }
   for (int t = 0; t < 5; ++t) {  // the same matrix by target code

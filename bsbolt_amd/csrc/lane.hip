@@ -738,8 +738,14 @@ ext_lane_frame_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const ui
   }
 }
 
+// A batch without pair kernels shares the chip between these and the group kernels
+// from the start: up to half a million tasks, one wave a SIMD leaves those half of
+// its registers (gap extensions of 26, 100 bp reads, 131,072 / 262,144 tasks: 673 /
+// 917 us with two, 413 / 729 with one; 1,000,000 of 33-64 bases alone 1.80 ms with two,
+// 2.49 with one).
+constexpr int64_t kLaneShareTasks = 524288;
 template <int Q, bool E1>
-void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st) {
+void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, int num_cu, hipStream_t st, bool pair) {
   static int per_cu = 0;
   if (per_cu == 0) {
     int nb = 0;
@@ -747,17 +753,18 @@ void launch_lane_bin(const ExtKArgs& k, const ExtWork& wk, int bin, int64_t n, i
       nb = 4;
     per_cu = nb;
   }
-  const int64_t blocks = std::min<int64_t>((int64_t)per_cu * num_cu, (n + 63) / 64);
+  const int waves = !pair && n < kLaneShareTasks ? std::min(per_cu, 4) : per_cu;
+  const int64_t blocks = std::min<int64_t>((int64_t)waves * num_cu, (n + 63) / 64);
   if (blocks < 1) return;
   time_begin(wk, time_of_bin(bin), st);
   hipLaunchKernelGGL((ext_lane_kernel<Q, E1>), dim3((unsigned)blocks), dim3(64), 0, st, k, (const ExtDesc*)wk.desc,
                      (const uint32_t*)wk.counts, bin, wk.fetch);
   time_end(wk, time_of_bin(bin), st);
 }
-template void launch_lane_bin<32, true>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);
-template void launch_lane_bin<32, false>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);
-template void launch_lane_bin<64, true>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);
-template void launch_lane_bin<64, false>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t);
+template void launch_lane_bin<32, true>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t, bool);
+template void launch_lane_bin<32, false>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t, bool);
+template void launch_lane_bin<64, true>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t, bool);
+template void launch_lane_bin<64, false>(const ExtKArgs&, const ExtWork&, int, int64_t, int, hipStream_t, bool);
 
 template <int WF, bool E1>
 void launch_lane_frame(const ExtKArgs& k, const ExtWork& wk, int cls, int num_cu, hipStream_t st) {

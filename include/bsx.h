@@ -341,8 +341,9 @@ int bsx_ext_bin_limits(int32_t *limits, int n);
 int bsx_set_side_streams(bsx_ctx *ctx, int enable);
 
 /* ---- tuning table (no counterpart in the reference) ----
- * table[0] descriptors per block of the plain group kernels, table[1] of the
- * frame group kernels (both 16..4096), table[2] / table[3] the group shape of
+ * table[0] four times the task descriptors that a block of the plain group
+ * kernels fetches at a time, table[1] those that a block of the frame group
+ * kernels owns (both 16..4096), table[2] / table[3] the group shape of
  * the bins of queries 65-96 / 97-128 bases (0: 16 lanes x 6 / 8 columns,
  * 1: 32 lanes x 3 / 4 columns).  Every table gives the same results.
  * bsx_create loads the autotuner's cache entry for the device (key
