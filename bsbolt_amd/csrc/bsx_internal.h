@@ -28,12 +28,9 @@ constexpr int kNarrowTasksPerBlock = 16;  // ... by one narrow-kernel block
 constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; }
 
 // The CIGAR (ksw_global2) kernel bins tasks the same way with its own shapes.
-// A bin of its own for bands of 25-32 ((8,4)) lost: it is one launch more in a
-// chain of two on its stream (9,319 tasks of 150 bp reads: 417 us of kernels with
-// it, 307 without), and only 7% of the tasks have such a band.
-constexpr int kGlbBins = 8;
+constexpr int kGlbBins = 9;
 constexpr BinShape kGlbShape[kGlbBins] = {
-    {8, 2}, {8, 3}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
+    {8, 2}, {8, 3}, {8, 4}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
 constexpr int kExtSlices = 8;  // fetch-counter slots per lane bin and lane frame class (a CIGAR bin uses one)
 // Bins of the two-tasks-per-lane CIGAR kernel (gpair.hip), after the others:
 // band widths 2w+1 up to kGlbPairCols, each from glb_pair_top + 1 on.
@@ -64,9 +61,11 @@ __host__ __device__ constexpr int glb_key(int bin, int tlen) {
 __host__ __device__ constexpr int glb_pair_rows(int tlen) { return (tlen + 3) / 4 * 4; }
 // Smallest batch whose narrow bands run the pair kernel: below it the batch
 // takes the latency of its waves, and the group kernels finish sooner.  us per
-// call, pair / group kernels: 100 bp reads 128,000 tasks 1026 / 721, 192,000 1068 /
-// 1030, 256,000 1088 / 1326; 150 bp 128,000 1329 / 1141, 192,000 1346 / 1621; 250
-// bp 128,000 2526 / 2757, 192,000 2553 / 3858.
+// call, pair / group kernels: 100 bp reads 128,000 tasks 984 / 740, 192,000 1066 /
+// 1007, 256,000 1065 / 1291; 150 bp 128,000 1296 / 1097, 160,000 1325 / 1293,
+// 192,000 1314 / 1545; 250 bp 100,000 2520 / 1928, 128,000 2478 / 2249, 160,000 2500 /
+// 2774.  Tasks of one kind fill the waves sooner: 131,072 of 150 bp reads of half
+// band 7 / 15 410 / 721 and 564 / 1096.
 constexpr int64_t kGlbPairMinTasks = 131072;
 constexpr int glb_bin_limit(int b) { return kGlbShape[b].lanes * kGlbShape[b].cols; }
 // First entry of fetch slice s of a list of n entries: a balanced partition,
@@ -358,14 +357,14 @@ __device__ __forceinline__ bool glb_task_ok(const GlbArgs& A, const GlbWork& W, 
 }
 // The bins that take what the unbinned kernel leaves, and the one of a band.
 constexpr int kGlbRest = 3;
-constexpr int kGlbRestBin[kGlbRest] = {5, 6, 7};
+constexpr int kGlbRestBin[kGlbRest] = {6, 7, 8};
 __device__ __forceinline__ int glb_rest_of(int ncol) {
   return ncol <= glb_bin_limit(kGlbRestBin[0]) ? 0 : ncol <= glb_bin_limit(kGlbRestBin[1]) ? 1 : 2;
 }
 // Largest batch that runs a wave per task without binning (gwave.hip).  us per
-// call, so / in bins beside each other: 100 bp reads 300 tasks 52 / 153, 8,000 127 /
-// 189, 16,000 202 / 223, 24,000 278 / 264; 150 bp 300 69 / 208, 16,000 289 / 341,
-// 24,000 398 / 365; 250 bp 300 111 / 308, 16,000 468 / 739, 24,000 653 / 628.
+// call, so / in bins beside each other: 100 bp reads 300 tasks 55 / 148, 8,000 134 /
+// 187, 20,000 252 / 251, 24,000 290 / 266; 150 bp 300 73 / 208, 16,000 298 / 313, 20,000
+// 361 / 360, 24,000 416 / 365; 250 bp 300 118 / 308, 16,000 472 / 727, 30,000 794 / 830.
 constexpr int64_t kGlbDirectMaxTasks = 20480;
 void launch_glb_direct(const GlbArgs& a, const GlbWork& w, hipStream_t st);
 

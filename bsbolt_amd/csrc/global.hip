@@ -89,36 +89,97 @@ __device__ __forceinline__ int g_next(int x) {
                  : __builtin_amdgcn_update_dpp(0, x, 0x130, 0xf, 0xf, true);  // wave_shl:1
 }
 
+// Direction-byte slots per CU, one slot a group.  Launches that run one after
+// another share kGlbSlotsOne of them; launches beside each other divide kGlbSlots
+// (glb_part).
+constexpr int kGlbSlotsOne = 128, kGlbSlots = 192;
+// A batch without pair kernels takes the latency of its rows, 115-145 us a bin
+// whatever its share of the tasks, so the bins that are seldom empty run beside each
+// other, each as a part of its own, and the wide ones follow one another as another
+// part.  With all of them on one stream but (16,4) the call took longer (us, so /
+// now): 100 bp reads 32,000 tasks 581 / 280, 64,000 685 / 432; 150 bp 32,000 941 / 404,
+// 64,000 1143 / 640; 250 bp 32,000 1848 / 874, 64,000 2156 / 1262.
+constexpr int kGlbPart[kGlbBins] = {1, 0, 4, 2, 3, 3, 3, 3, 3};
+constexpr int kGlbParts = 5;
+constexpr int kGlbPartSlots[kGlbParts] = {56, 56, 32, 32, 16};  // slots a part has in any case
+// slots per CU that a bin's launch can use
+constexpr int glb_most_slots(int b) {
+  const int s = 7 * (256 / kGlbShape[b].lanes);
+  return s < kGlbSlots ? s : kGlbSlots;
+}
+constexpr int glb_part_slots() {
+  int n = 0;
+  for (int k = 0; k < kGlbParts; ++k) n += kGlbPartSlots[k];
+  return n;
+}
+static_assert(glb_part_slots() == kGlbSlots, "slot parts");
+
+// The slots of part k, for launches beside each other: what its largest list can use
+// of its own share, and of what the other parts leave of theirs.  Every launch finds
+// the same division from the counts.  With fixed shares a batch of one kind ran on a
+// third of the slots (131,000 tasks of 150 bp reads, all of half band 7 / 11: 1043 /
+// 1217 us, so 721 / 843).
+struct GlbSlots { int64_t first, count; };
+__device__ __forceinline__ GlbSlots glb_part(const uint32_t* __restrict__ counts, int k, int num_cu) {
+  int64_t use[kGlbParts] = {}, part[kGlbParts];
+#pragma unroll
+  for (int b = 0; b < kGlbBins; ++b) {  // in steps of 32: whole blocks of any bin
+    const int64_t n = ((int64_t)counts[b] + 31) / 32 * 32, most = (int64_t)glb_most_slots(b) * num_cu / 32 * 32;
+    use[kGlbPart[b]] = max(use[kGlbPart[b]], min(n, most));
+  }
+  int64_t left = (int64_t)kGlbSlots * num_cu / 32 * 32;
+#pragma unroll
+  for (int s = 0; s < kGlbParts; ++s) {
+    part[s] = min(use[s], (int64_t)kGlbPartSlots[s] * num_cu / 32 * 32);
+    left -= part[s];
+  }
+  GlbSlots p{0, 0};
+#pragma unroll
+  for (int s = 0; s < kGlbParts; ++s) {
+    const int64_t more = min(use[s] - part[s], left);
+    left -= more;
+    part[s] += more;
+    p.first += s < k ? part[s] : 0;
+    p.count = s == k ? part[s] : p.count;
+  }
+  return p;
+}
+
+constexpr int kGlbWinDwords = 4096;  // LDS windows of a block
+
+// Block `block` of `blocks` on a bin's list.  first: of the list, or -1 (it follows
+// the lists before it); slot0: the blocks' first direction slot.
 template <int L, int C>
-__global__ void __launch_bounds__(256)
-glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase, int64_t first) {
+__device__ __forceinline__ void glb_run(const GlbArgs& A, const GlbWork& W, int bin, uint32_t block, uint32_t blocks,
+                                        int64_t slot0, int64_t first, uint32_t* __restrict__ zwin_all,
+                                        uint2* __restrict__ s_prof) {
+  if (block >= blocks) return;  // uniform over the block
   const int lane = threadIdx.x & 63;
   const int lig = lane & (L - 1);
   const int base = lig * C;
-  const int group = (blockIdx.x * blockDim.x + threadIdx.x) / L;
-  int64_t lbase = first;  // of the bin's list; -1: it follows those before it
+  const int group = (int)block * (256 / L) + threadIdx.x / L;
+  int64_t lbase = first;
   if (first < 0) {
     lbase = 0;
     for (int b = 0; b < bin; ++b) lbase += W.counts[b];
   }
   const int32_t* __restrict__ list = W.list + lbase;
   const uint32_t nlist = W.counts[bin];
-  uint8_t* __restrict__ z = W.z + (zbase + group) * W.zslot;  // zbase: this launch's slot region
+  uint8_t* __restrict__ z = W.z + (slot0 + group) * W.zslot;
   constexpr int ZW = zwin_dw<L>();
-  __shared__ uint32_t zwin_all[256 / L][ZW];
-  uint32_t* __restrict__ zwin = zwin_all[threadIdx.x / L];
+  static_assert(256 / L * ZW <= kGlbWinDwords, "LDS windows");
+  uint32_t* __restrict__ zwin = zwin_all + threadIdx.x / L * ZW;
   const int oe_del = A.o_del + A.e_del, oe_ins = A.o_ins + A.e_ins;
   const int e_del = A.e_del, e_ins = A.e_ins;
 
   // profile words by query code (code 4 for N and positions past the query),
   // for the position entering the band on each row
-  __shared__ uint2 s_prof[5];
   if (threadIdx.x < 5) s_prof[threadIdx.x] = make_uint2(A.prof_lo[threadIdx.x], (uint32_t)A.prof_hi[threadIdx.x]);
   __syncthreads();
   // Every group's first task is its own number; only when the list is longer
   // than the grid do groups fetch more (each wave's fetch is a device atomic on
   // one address, ~10 ns apiece serialised, so an empty or short list has none).
-  const uint32_t groups = gridDim.x * (256 / L);
+  const uint32_t groups = blocks * (256 / L);
   uint32_t idx = (uint32_t)group;
   while (idx < nlist) {
     const int task = list[idx];
@@ -396,6 +457,32 @@ glb_kernel(GlbArgs A, GlbWork W, int bin, int64_t zbase, int64_t first) {
   }
 }
 
+// part: the launch's among those beside each other, or -1 (it has kGlbSlotsOne
+// slots per CU)
+template <int B>
+__global__ void __launch_bounds__(256) glb_kernel(GlbArgs A, GlbWork W, int part, int num_cu, int64_t first) {
+  constexpr int L = kGlbShape[B].lanes, C = kGlbShape[B].cols;
+  __shared__ uint32_t zwin[kGlbWinDwords];
+  __shared__ uint2 s_prof[5];
+  const GlbSlots p = part < 0 ? GlbSlots{0, (int64_t)kGlbSlotsOne * num_cu} : glb_part(W.counts, part, num_cu);
+  glb_run<L, C>(A, W, B, blockIdx.x, min((uint32_t)(p.count / (256 / L)), gridDim.x), p.first, first, zwin, s_prof);
+}
+
+// Two bins in one launch, beside each other: bands of 25-32 are few in a read set's
+// batch, and a launch of their own in front of another adds its latency to the call
+// (32,000 tasks of 100 bp reads: 312 us on the stream of (8,3), 280 so).
+template <int B1, int B2>
+__global__ void __launch_bounds__(256) glb_two_kernel(GlbArgs A, GlbWork W, int num_cu) {
+  constexpr int L1 = kGlbShape[B1].lanes, C1 = kGlbShape[B1].cols, L2 = kGlbShape[B2].lanes, C2 = kGlbShape[B2].cols;
+  __shared__ uint32_t zwin[kGlbWinDwords];
+  __shared__ uint2 s_prof[5];
+  const GlbSlots p = glb_part(W.counts, kGlbPart[B1], num_cu), q = glb_part(W.counts, kGlbPart[B2], num_cu);
+  const uint32_t np = min((uint32_t)(p.count / (256 / L1)), gridDim.x);
+  const uint32_t nq = min((uint32_t)(q.count / (256 / L2)), gridDim.x - np);
+  if (blockIdx.x < np) glb_run<L1, C1>(A, W, B1, blockIdx.x, np, p.first, -1, zwin, s_prof);
+  else glb_run<L2, C2>(A, W, B2, blockIdx.x - np, nq, q.first, -1, zwin, s_prof);
+}
+
 // Bin of the two-tasks-per-lane kernel for a valid task, or -1: the whole band
 // (not clipped to the query) fits, and every score fits its 16 bits.
 __device__ __forceinline__ int glb_pair_bin_of(const GlbArgs& A, int ql, int tl, int w) {
@@ -526,32 +613,19 @@ hipError_t launch_glb_gather(const int32_t* score, const int32_t* n_cigar, const
   return hipGetLastError();
 }
 
-// Direction-byte slots per CU, one slot a group.  A launch uses the part given
-// to its stream; launches that run one after another share kGlbSlotsOne.
-struct GlbPart { int first, slots; };
-constexpr int kGlbSlotsOne = 128, kGlbSlots = 192;
-constexpr GlbPart kGlbAlone = {0, kGlbSlotsOne};
-constexpr GlbPart kGlbStreamPart[1 + StreamSet::kSide] = {{0, 64}, {64, 64}, {128, 32}, {160, 32}};
-static_assert(StreamSet::kSide == 3, "slot parts");
-// Streams of the bins in a batch without pair kernels.  Such a batch takes the
-// latency of its rows, 115-145 us a bin whatever its share of the tasks, so the
-// four bins that are seldom empty run beside each other, and the wide ones follow
-// where they wait for nobody.  With all of them on one stream but (16,4) the
-// call took longer (us, before / now): 100 bp reads 32,000 tasks 581 / 267, 64,000
-// 685 / 426; 150 bp 32,000 941 / 416, 64,000 1143 / 646; 250 bp 32,000 1848 / 963,
-// 64,000 2156 / 1598.
-constexpr int kGlbStream[kGlbBins] = {1, 0, 2, 3, 3, 3, 3, 3};
-
 int64_t glb_groups(int num_cu, bool side) { return (int64_t)num_cu * (side ? kGlbSlots : kGlbSlotsOne); }
 
 template <int B>
-static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st, GlbPart part,
+static int64_t glb_blocks(const GlbArgs& a, int num_cu, int most) {
+  constexpr int L = kGlbShape[B].lanes;
+  return std::min<int64_t>((int64_t)std::min(glb_most_slots(B), most) * num_cu / (256 / L), (a.n * L + 255) / 256);
+}
+
+template <int B>
+static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipStream_t st, int part = -1,
                            int64_t first = -1) {
-  constexpr int L = kGlbShape[B].lanes, C = kGlbShape[B].cols;
-  const int64_t room = std::min<int64_t>(part.slots / (256 / L), 7) * num_cu;
-  const int64_t blocks = std::min<int64_t>(room, (a.n * L + 255) / 256);
-  hipLaunchKernelGGL((glb_kernel<L, C>), dim3((unsigned)blocks), dim3(256), 0, st, a, w, B,
-                     (int64_t)part.first * num_cu, first);
+  const int64_t blocks = glb_blocks<B>(a, num_cu, part < 0 ? kGlbSlotsOne : kGlbSlots);
+  hipLaunchKernelGGL(glb_kernel<B>, dim3((unsigned)blocks), dim3(256), 0, st, a, w, part, num_cu, first);
 }
 
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) {
@@ -562,9 +636,9 @@ hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) 
   if (a.n <= std::min<int64_t>(kGlbDirectMaxTasks, (int64_t)num_cu * kGlbSlotsOne)) {
     launch_glb_direct(a, w, st);
     static_assert(kGlbRest == 3, "rest bins");
-    glb_launch_bin<kGlbRestBin[0]>(a, w, num_cu, st, kGlbAlone, 0);
-    glb_launch_bin<kGlbRestBin[1]>(a, w, num_cu, st, kGlbAlone, a.n);
-    glb_launch_bin<kGlbRestBin[2]>(a, w, num_cu, st, kGlbAlone, 2 * a.n);
+    glb_launch_bin<kGlbRestBin[0]>(a, w, num_cu, st, -1, 0);
+    glb_launch_bin<kGlbRestBin[1]>(a, w, num_cu, st, -1, a.n);
+    glb_launch_bin<kGlbRestBin[2]>(a, w, num_cu, st, -1, 2 * a.n);
     return hipGetLastError();
   }
   // each block ends with a global atomic per non-empty bucket
@@ -573,34 +647,44 @@ hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) 
   hipLaunchKernelGGL(glb_bin_offset_kernel, dim3(1), dim3(1024), 0, st, w);
   hipLaunchKernelGGL(glb_bin_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, w, (a.n + blocks - 1) / blocks);
   if (a.pair) {
-    // Only bin 3 (bands of 65-128) is likely to hold tasks beside the pair
+    // Only bin 4 (bands of 65-128) is likely to hold tasks beside the pair
     // bins.  The others go ahead of everything, 5 us each while the chip is
     // empty: behind a pair kernel, or beside one, even an empty launch waits
     // until there is room for its blocks (0.5-1.3 ms measured).
-    glb_launch_bin<7>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<6>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<5>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<4>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<2>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<1>(a, w, num_cu, st, kGlbAlone);
-    glb_launch_bin<0>(a, w, num_cu, st, kGlbAlone);
+    glb_launch_bin<8>(a, w, num_cu, st);
+    glb_launch_bin<7>(a, w, num_cu, st);
+    glb_launch_bin<6>(a, w, num_cu, st);
+    glb_launch_bin<5>(a, w, num_cu, st);
+    glb_launch_bin<3>(a, w, num_cu, st);
+    glb_launch_bin<2>(a, w, num_cu, st);
+    glb_launch_bin<1>(a, w, num_cu, st);
+    glb_launch_bin<0>(a, w, num_cu, st);
     ss_fork(w.ss, st);
-    glb_launch_bin<3>(a, w, num_cu, pick_stream(w.ss, st, 3), kGlbAlone);
+    glb_launch_bin<4>(a, w, num_cu, pick_stream(w.ss, st, 3));
     launch_glb_pair(a, w, num_cu, st);
-  } else {
+  } else if (w.ss) {
     ss_fork(w.ss, st);  // side streams start after the scatter
-    const auto beside = [&](auto bin) {
-      constexpr int B = decltype(bin)::value, k = kGlbStream[B];
-      glb_launch_bin<B>(a, w, num_cu, pick_stream(w.ss, st, k), w.ss ? kGlbStreamPart[k] : kGlbAlone);
-    };
-    beside(std::integral_constant<int, 1>());
-    beside(std::integral_constant<int, 2>());
-    beside(std::integral_constant<int, 0>());
-    beside(std::integral_constant<int, 3>());
-    beside(std::integral_constant<int, 7>());
-    beside(std::integral_constant<int, 6>());
-    beside(std::integral_constant<int, 5>());
-    beside(std::integral_constant<int, 4>());
+    glb_launch_bin<1>(a, w, num_cu, st, kGlbPart[1]);
+    hipLaunchKernelGGL((glb_two_kernel<2, 3>),
+                       dim3((unsigned)(glb_blocks<2>(a, num_cu, kGlbSlots) + glb_blocks<3>(a, num_cu, kGlbSlots))),
+                       dim3(256), 0, pick_stream(w.ss, st, 2), a, w, num_cu);
+    glb_launch_bin<0>(a, w, num_cu, pick_stream(w.ss, st, 1), kGlbPart[0]);
+    const hipStream_t s3 = pick_stream(w.ss, st, 3);
+    glb_launch_bin<4>(a, w, num_cu, s3, kGlbPart[4]);
+    glb_launch_bin<8>(a, w, num_cu, s3, kGlbPart[8]);
+    glb_launch_bin<7>(a, w, num_cu, s3, kGlbPart[7]);
+    glb_launch_bin<6>(a, w, num_cu, s3, kGlbPart[6]);
+    glb_launch_bin<5>(a, w, num_cu, s3, kGlbPart[5]);
+  } else {
+    glb_launch_bin<1>(a, w, num_cu, st);
+    glb_launch_bin<2>(a, w, num_cu, st);
+    glb_launch_bin<3>(a, w, num_cu, st);
+    glb_launch_bin<0>(a, w, num_cu, st);
+    glb_launch_bin<4>(a, w, num_cu, st);
+    glb_launch_bin<8>(a, w, num_cu, st);
+    glb_launch_bin<7>(a, w, num_cu, st);
+    glb_launch_bin<6>(a, w, num_cu, st);
+    glb_launch_bin<5>(a, w, num_cu, st);
   }
   ss_join(w.ss, st);  // the call's stream waits for the side streams
   return hipGetLastError();
