@@ -85,6 +85,7 @@ struct Work {
   DevBuf nbin_of, need_plain, cls;        // learned-band form
   DevBuf zbuf;                            // direction-byte slots of the global kernel
   DevBuf zpair;                           // direction scratch of its two-tasks-per-lane form
+  bool zpair_failed = false;              // there was no memory for it
   void release() {
     for (DevBuf* b : {&bin_of, &list, &desc, &rec, &small, &nbin_of, &need_plain, &cls, &zbuf, &zpair}) b->release();
   }
@@ -949,7 +950,13 @@ static int glb_buffers(bsx_ctx* c, size_t n, bool cigar) {
   HIPCHK(c, c->ws->small.ensure(kSmallBytes), "hipMalloc(work)");
   if (cigar) {
     HIPCHK(c, c->ws->zbuf.ensure((size_t)glb_groups(c->num_cu, c->ss_on) * (size_t)c->zslot), "hipMalloc(z)");
-    if (n >= (size_t)kGlbPairMinTasks) HIPCHK(c, c->ws->zpair.ensure((size_t)glb_pair_bytes(c->num_cu)), "hipMalloc(zpair)");
+    // Without memory for this one the group kernels take every task.  (A graph's
+    // workspace is sized ahead of its capture, in which nothing may be allocated.)
+    Work& w = *c->ws;
+    if (n >= (size_t)kGlbPairMinTasks && (&w == &c->wown || !w.zpair_failed)) {
+      w.zpair_failed = w.zpair.ensure((size_t)glb_pair_bytes(c->num_cu)) != hipSuccess;
+      if (w.zpair_failed) (void)hipGetLastError();
+    }
   }
   return BSX_OK;
 }

@@ -334,7 +334,7 @@ struct GlbWork {
   uint32_t* kcursor;  // [kGlbKeys] scatter cursors of the same
   uint8_t* z;    // per-group direction-byte slots
   int64_t zslot; // bytes per slot
-  uint8_t* zpair;      // direction scratch of the pair kernel (glb_pair_bytes), nullptr without CIGARs
+  uint8_t* zpair;      // direction scratch of the pair kernel (glb_pair_bytes), nullptr without CIGARs or memory
   int64_t pair_bytes;  // this bin's share of it
   const StreamSet* ss;  // side streams for the bins with few tasks per group (nullptr: one stream)
 };

@@ -630,7 +630,7 @@ static void glb_launch_bin(const GlbArgs& a, const GlbWork& w, int num_cu, hipSt
 
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st) {
   w.pair_bytes = glb_pair_bytes(num_cu);
-  a.pair = a.n >= kGlbPairMinTasks;
+  a.pair = a.n >= kGlbPairMinTasks && (!a.cigar || w.zpair);
   hipLaunchKernelGGL(glb_reset_kernel, dim3(1), dim3(1024), 0, st, w);
   if (a.n <= 0) return hipGetLastError();
   if (a.n <= std::min<int64_t>(kGlbDirectMaxTasks, (int64_t)num_cu * kGlbSlotsOne)) {

@@ -152,7 +152,8 @@ int bsx_global_batch_device(bsx_ctx *ctx, const bsx_scoring *sc,
  * needs min(qlen, 2w+1) * tlen bytes; larger ones are rejected (BSX_EINVAL).
  * The context holds #CU * 192 such slots of device memory (#CU * 128 with
  * side streams off, bsx_set_side_streams), and 10 MiB per CU more once a batch
- * of 98,304 tasks or more has asked for CIGARs.  The host-memory call
+ * of 131,072 tasks or more has asked for CIGARs (where that much is not free, the
+ * call runs without); a captured graph holds its own of both.  The host-memory call
  * bsx_global_batch (and so bsx_ksw_global2) raises the slot for its own call
  * to the batch's largest need, up to 256 KiB; the device-memory call cannot see
  * the sizes and uses the slot as set. */
