@@ -203,6 +203,9 @@ __device__ __forceinline__ uint32_t plane_of(const uint32_t (&v)[8], uint32_t ma
   return r;
 }
 
+// bases between the start of the reference's first dword and its first byte
+__device__ __forceinline__ int md_lead(const MdArgs& a) { return 4 * (int)((uintptr_t)a.opac & 3); }
+
 // The walk by words; st is 1 where only md_walk can tell (a slot overflows or a
 // number has four digits).  The caller has checked that the walk stays in its
 // window, that three dwords past the window's last lie in the reference, and
@@ -210,7 +213,9 @@ __device__ __forceinline__ uint32_t plane_of(const uint32_t (&v)[8], uint32_t ma
 __device__ __forceinline__ MdRes md_words_walk(const MdArgs& a, const MdTask& T, const uint32_t* __restrict__ num,
                                                bool md_words, bool xb_words) {
   MdRes R{};
-  const uint32_t* __restrict__ opac32 = (const uint32_t*)a.opac;
+  // the reference from its first byte's dword on
+  const uint32_t* __restrict__ opac32 = (const uint32_t*)((uintptr_t)a.opac & ~(uintptr_t)3);
+  const int lead = md_lead(a);
   const uint32_t flip = T.fwd ? 0u : ~0u;
   const uint32_t i2b = T.fwd ? 0x54474341u : 0x41434754u;  // "ACGT", "TGCA"
   const uint32_t md_cap = (uint32_t)(a.md_slot < (1 << 28) ? a.md_slot : 1 << 28) * 8;
@@ -251,7 +256,7 @@ __device__ __forceinline__ MdRes md_words_walk(const MdArgs& a, const MdTask& T,
     }
     const int nb = min(rem, 32);
     // ---- window bases [y, y + 36) as planes (H: high bits of the codes, L: low) ----
-    const int64_t p = T.k0 + y;
+    const int64_t p = T.k0 + y + lead;
     uint32_t d[4];
     __builtin_memcpy(d, opac32 + (p >> 4), 16);
     // base i of a dword's 16: bits 2i (high) and 2i + 1 (low)
@@ -387,8 +392,9 @@ __global__ void __launch_bounds__(kMdBlock) md_kernel(MdArgs a) {
       T.o1 = !reverse ? (!T.is_crick ? 2 : 1) : (!T.is_crick ? 2 : 3);
       T.o2 = !reverse ? (!T.is_crick ? 3 : 2) : (!T.is_crick ? 1 : 2);
       T.o3 = !reverse ? (!T.is_crick ? 4 : 3) : (!T.is_crick ? 0 : 1);
-      const bool words = ysum + 4 <= T.clen && T.l_query >= 32 && ((uintptr_t)a.opac & 3) == 0 &&
-                         ((T.k0 + T.clen) >> 4) + 3 <= (l_pac - 1) >> 4;
+      const int lead = md_lead(a);
+      const bool words = ysum + 4 <= T.clen && T.l_query >= 32 &&
+                         ((T.k0 + T.clen + lead) >> 4) + 3 <= (l_pac - 1 + lead) >> 4;
       R.st = 1;
       if (words) R = md_words_walk(a, T, num, md_words, xb_words);
       if (R.st != 0) R = md_walk(a, T, md_words, xb_words);
