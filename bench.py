@@ -636,7 +636,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "int32",
+        "dtype": "int16/int32",  # scores in packed 16 bits where a per-task range check holds them exactly
         "data": "synthetic (seeded genome + bisulfite read simulation; no external data)",
         "config": {"workload": f"{args.workload}: {cfg.genome_len // 1_000_000} Mb genome, {wl.n_reads} reads "
                                f"x {cfg.read_len} bp{' PE' if cfg.paired else ' SE'}, all mem_chain2aln "

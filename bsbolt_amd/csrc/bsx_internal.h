@@ -123,13 +123,14 @@ constexpr int kScoreLimit = 1 << 20;
 constexpr int pair_score_max(int Q) { return Q <= 128 ? 511 : 255; }
 constexpr int kPairMaxTlen = 640;   // with kPairMaxGapExt: the gap cost of a z-drop test,
 constexpr int kPairMaxGapExt = 25;  // e * (tlen + Q), and the z-drop itself fit 15 bits
-// Smallest batch whose short queries run the pair kernel.  A lane runs its two
-// tasks serially, so a batch takes at least its longest run (0.4 ms for 100 bp
+// Smallest binned batch whose short queries run the pair kernel.  A lane runs its
+// two tasks serially, so a batch takes at least its longest run (0.4 ms for 100 bp
 // reads, 0.8 ms for 150 bp); below this the group kernels, which spread a task
 // over 16 lanes, finish sooner.  us per call, pair / group kernels: 100 bp
 // 32,000 tasks 429 / 276, 64,000 451 / 431, 128,000 529 / 763; 150 bp 32,000
-// 810 / 555, 64,000 874 / 968, 128,000 1406 / 1869.  (Only the learned-band form
-// bins a batch of fewer than kDirectMaxTasks.)
+// 810 / 555, 64,000 874 / 968, 128,000 1406 / 1869.  It decides for timed calls
+// only, as others of up to kDirectMaxTasks are not binned; their routing to frame
+// classes, which bsx_band_stats counts, goes by these bins too.
 constexpr int64_t kPairMinTasks = 65536;
 
 // Kernel-side view of an extension batch (all pointers are device memory).

@@ -31,10 +31,12 @@
 //
 // 24 packed instructions per cell of two tasks (11 of them the recurrences, 12
 // the directions) against ~250 per row of 16-24 cells for 8 tasks in the group
-// kernels; VALU-bound over a call (570M wave instructions, 1.0 of its 1.7 ms of
-// kernels for 596,416 tasks of 150 bp reads), and the direction bytes move at
-// 3.3 TB/s.  That CIGAR pass: 4.80 -> 1.89 ms.  Register budgets are set so that
-// nothing spills: a spilled load in the row loop waits for the stores before it.
+// kernels.  596,416 tasks of 150 bp reads: 511M wave instructions, 0.9 ms of issue,
+// of the call's 2.00 ms (4.81 with the group kernels); in order the five kernels
+// take 3.1 ms, each mostly the latency of a wave or two per SIMD.  Register budgets
+// are set so that no vector register spills (a spilled load in the row loop waits
+// for the stores before it); uniform values of the walk do, 39 (NC = 15) to 231 (63),
+// into vector registers.
 #include <algorithm>
 
 #include "bsx_internal.h"

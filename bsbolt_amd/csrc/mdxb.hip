@@ -11,8 +11,8 @@
 //
 // A walk of every base by every lane was bound by instructions: some lane of the
 // wave always had a call or a mismatch, so each of 150 steps ran the whole body.
-// 400,009 regions of 150 bp reads: 871 us then, 156 now, of which the vector
-// instructions (5,300 a wave) take 58; the rest is the addresses of 139 loads and
+// 400,009 regions of 150 bp reads: 871 us then, 158 now, of which the vector
+// instructions (5,400 a wave) take 59; the rest is the addresses of 139 loads and
 // stores a wave, each of whose lanes touches lines of its own.
 #include "bsx_internal.h"
 

@@ -48,7 +48,8 @@ static_assert(frame_of_class(0) == kFrameWidth[0] && frame_of_class(1) == kFrame
 // 40 columns -- upper bounds, from the rows of the runs that completed --
 // and group frames of 80 and 144 columns).  A task goes to its predicted frame
 // class only where that class is at least 20% cheaper per row than the plain
-// bin of its query length.
+// bin it would run in: beside the pair kernels no frame is for queries of up to 96
+// bases.
 constexpr int kPlainRowPs[kExtBins] = {15, 22, 32, 55, 240, 255, 465, 830, 1500, 43, 59, 109, 158, 600};
 constexpr int kFrameRowPs[kBandClasses - 1] = {29, 75, 152, 239};
 static_assert(kExtBins == 14 && kBandClasses == 5, "row cost tables");

@@ -39,12 +39,13 @@
 // VALU-bound: 20 packed instructions per column (162 per block) and ~175 per
 // row, for 128 tasks at once; the kernels it replaced took 31 per column for 64
 // tasks (lane per task) and ~300 per row for 2-4 tasks (16-64 lanes per task).
-// Widths 32 to 96 hold the state in the 256 VGPRs of two (three) waves per SIMD
-// and issue VALU on 79-90% of the cycles.  Widths 128 and 224 take all 512
-// registers of a SIMD for one wave: the compiler keeps the columns past ~96 in
-// accumulation registers, two to four moves per eight columns, and a lone wave
-// issues on half the cycles; that still is 3 (128) to 6 (224) times the group
-// kernels' rate.  Kernel alone, queries of <= 32 / 33-64 / 65-96 / 97-128 /
+// Widths 32 and 64 hold the state in the 256 VGPRs of two (three) waves per SIMD
+// and issue VALU on 87-90% of the cycles.  Width 96 fills them and spills 28 (100
+// bytes of scratch a lane, most of the 194 MB that a launch over 3.9M flanks
+// writes): 79%.  Widths 128 and 224 take all 512 registers of a SIMD for one wave:
+// the compiler keeps the columns past ~96 in accumulation registers, two to four
+// moves per eight columns, 224 spills 44 (180 bytes), and a lone wave issues on
+// half the cycles; that still is 3 (128) to 6 (224) times the group kernels' rate.  Kernel alone, queries of <= 32 / 33-64 / 65-96 / 97-128 /
 // 129-224 bases: 3.9M flanks of 2x150 bp reads 0.42 / 1.42 / 1.47 / 0.85 / 0.14
 // ms (was 1.16 / 3.5 / 5.0 / 2.5 / 0.33); 351,491 flanks of 250 bp reads 0.18 /
 // 0.49 / 0.86 / 1.19 / 2.39 ms (97 and longer: was 2.3 / 9.2).  Whole calls: 4.2

@@ -22,8 +22,9 @@
 //
 // The row is bound by instruction issue (about 130 vector and 60 scalar
 // instructions for C = 4); a lone wave takes 0.6 us a row, as each waits for the one
-// before.  4,001 flanks of 2 kb reads, most of band 100: 2.24 ms, where rows of all
-// 2,048 columns took 8.1.
+// before.  4,001 flanks of 2 kb reads, most of band 100: 2.06 ms, where rows of all
+// 2,048 columns took 8.1.  C = 32 spills 34 of its 256 registers where a whole bin
+// is its own (140 bytes of scratch a lane).
 #include <algorithm>
 
 #include "bsx_internal.h"
@@ -275,8 +276,8 @@ template void launch_wave_bin<32>(const ExtKArgs&, const ExtWork&, int, int64_t,
 
 
 // A batch without binning: block t runs task t, checked here, and writes its
-// results where the caller wants them, or as one record into pinned memory.  Tasks of more than 256 columns need
-// waves of more registers: PART 0 takes the others, PART 1 these, PART 2 all.
+// results where the caller wants them, or as one record into pinned memory.  Tasks of
+// more than 256 columns need waves of more registers: PART 0 takes the others, PART 1 these, PART 2 all.
 // CERT: a batch that was checked and routed (nbin_of); also marks the tasks whose
 // frame run fails (need_plain), and leaves every result in ExtWork::rec.
 template <int PART, bool CERT>

@@ -254,11 +254,13 @@ int   bsx_timer_stop(bsx_ctx *ctx, float *ms);
  * adaptive band).  Under BSX_BAND_LEARNED the extension entry points first
  * predict a frame class per task with the band model (band-following frames of
  * 24, 40, 80 or 144 columns, or plain), run the frame kernel for the tasks whose
- * class is a frame, and keep a frame result only when the run's band never left
- * the frame with a non-zero cell (checked exactly, per row); every other task
- * runs the plain kernel.  Results are identical to BSX_BAND_PLAIN in every case.
- * BSX_BAND_FIXED runs every task whose query is <= 256 bases through frame class
- * `band_class` first (tests, labels). */
+ * class is a frame that costs less than their plain kernel, and keep a frame
+ * result only when the run's band never left the frame with a non-zero cell
+ * (checked exactly, per row); every other task runs the plain kernel.  Results are
+ * identical to BSX_BAND_PLAIN in every case.  BSX_BAND_FIXED runs every task whose
+ * query is <= 256 bases through frame class `band_class` first (tests, labels).
+ * Under both, an untimed call of up to 98304 tasks runs no frame kernel: every task
+ * runs in full, and its frame is only tested on the way. */
 #define BSX_BAND_PLAIN   0
 #define BSX_BAND_LEARNED 1
 #define BSX_BAND_FIXED   2
@@ -268,7 +270,10 @@ int   bsx_timer_stop(bsx_ctx *ctx, float *ms);
 #define BSX_BAND_PARAMS 6085    /* MLP 24-64-64-5: W1,b1,W2,b2,W3,b3 (row = out) */
 int bsx_set_band_policy(bsx_ctx *ctx, int policy, int band_class);
 /* Per class c of the last learned/fixed extension call: out[2c] tasks routed to
- * class c (c = 4: plain only), out[2c+1] of those whose frame run fell back. */
+ * class c (c = 4: plain only), out[2c+1] of those whose frame run fell back (or,
+ * where the frames were only tested, would have).  What a learned call routes to a
+ * frame depends on the plain kernels of its batch size: past 65536 tasks, no query
+ * of up to 96 bases that the two-tasks-per-lane kernels take. */
 int bsx_band_stats(bsx_ctx *ctx, int64_t out[2 * BSX_BAND_CLASSES]);
 /* FP32 master parameters of the band model (set resets the Adam state). */
 int bsx_band_model_set(bsx_ctx *ctx, const float *params, int64_t n_params);
