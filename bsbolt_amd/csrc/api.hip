@@ -991,7 +991,7 @@ int bsx_global_batch_device(bsx_ctx* c, const bsx_scoring* sc, const bsx_glb_tas
   wk.cursor = wk.counts + kCountSlots;
   wk.err = (int32_t*)(wk.cursor + kCountSlots);
   wk.fetch = (uint32_t*)(wk.err + 4);
-  wk.kcount = wk.fetch + kFetchSlots;
+  wk.kcount = wk.fetch + kCountSlots;
   wk.kcursor = wk.kcount + kGlbKeys;
   wk.zslot = c->zslot;
   wk.ss = c->ss_on ? &c->ss : nullptr;

@@ -31,7 +31,7 @@ constexpr int bin_limit(int b) { return kExtShape[b].lanes * kExtShape[b].cols; 
 constexpr int kGlbBins = 9;
 constexpr BinShape kGlbShape[kGlbBins] = {
     {8, 2}, {8, 3}, {8, 4}, {16, 4}, {32, 4}, {64, 4}, {64, 8}, {64, 16}, {64, 32}};
-constexpr int kExtSlices = 8;  // fetch-counter slots per lane bin and lane frame class (a CIGAR bin uses one)
+constexpr int kExtSlices = 8;  // slices of a lane kernel's list, each with a fetch counter
 // Bins of the two-tasks-per-lane CIGAR kernel (gpair.hip), after the others:
 // band widths 2w+1 up to kGlbPairCols, each from glb_pair_top + 1 on.
 constexpr int kGlbPairBins = 5;
@@ -106,7 +106,18 @@ constexpr int kNarrowQMax = 256;  // longest query the narrow kernels take
 // the group frame kernel.  Both compute the same frame run.
 constexpr int kLaneFrameClasses = 2;
 constexpr int kLaneFrameQMax = 128;
-constexpr int kFetchSlots = kCountSlots * kExtSlices;
+// Fetch counters of an extension call: one for each slice of the lists that the
+// task-per-lane kernels take (bins, then frame classes) and one for each group bin,
+// each in a line of its own.  A wave of a lane kernel asks every slice of its list
+// before it ends, and those atomics on one line wait for one another.  RRBS reads in
+// 40-column frames, us per call with a list's counters side by side / so, two runs:
+// 98,305 tasks 924, 925 / 887, 924; 300,000 1192, 1204 / 1141, 1176; 1,000,000 1763,
+// 1747 / 1710, 1706.  32 words apart measured the same.
+constexpr int kFetchPad = 16;  // words from one to the next
+constexpr int kLaneLists = kLaneBins + kLaneFrameClasses;
+constexpr int lane_fetch(int list) { return list * kExtSlices * kFetchPad; }
+constexpr int group_fetch(int bin) { return (kLaneLists * kExtSlices + bin - kQueryBins - kLaneBins) * kFetchPad; }
+constexpr int kExtFetchWords = group_fetch(kExtBins);
 enum BandMode { kBandPlain = 0, kBandLearned = 1, kBandFixed = 2 };
 struct BandPlan {
   int mode;            // BandMode
@@ -202,7 +213,7 @@ struct ExtWork {
   int32_t* rec;        // [n][8] packed per-task results
   uint32_t* counts;    // [kCountSlots] tasks per bin / narrow class
   uint32_t* cursor;    // [kCountSlots] scatter cursors
-  uint32_t* fetch;     // [kFetchSlots] persistent-kernel fetch counters, kExtSlices per count slot
+  uint32_t* fetch;     // [kExtFetchWords] fetch counters (lane_fetch, group_fetch)
   uint32_t* split;     // [2 * kLaneFrameClasses]: per lane-frame class, tasks at the front of its
                        // list (query <= kLaneFrameQMax) and the back-of-list cursor
   int32_t* err;        // [0] rejected count, [1] lowest rejected index
@@ -225,14 +236,14 @@ struct ExtWork {
 };
 // The counters of a workspace lie in one array: counts, cursor, err[4], fetch,
 // split, bcount, bcursor, fcount, fcursor.
-constexpr int kExtCounterWords = 2 * kCountSlots + 4 + kFetchSlots + 2 * kLaneFrameClasses +
+constexpr int kExtCounterWords = 2 * kCountSlots + 4 + kExtFetchWords + 2 * kLaneFrameClasses +
                                  2 * kExtBins * kRowBuckets + 2 * kLaneFrameClasses * kRowBuckets;
 inline void ext_counters(ExtWork& wk, uint32_t* p) {
   wk.counts = p;
   wk.cursor = wk.counts + kCountSlots;
   wk.err = (int32_t*)(wk.cursor + kCountSlots);
   wk.fetch = (uint32_t*)(wk.err + 4);
-  wk.split = wk.fetch + kFetchSlots;
+  wk.split = wk.fetch + kExtFetchWords;
   wk.bcount = wk.split + 2 * kLaneFrameClasses;
   wk.bcursor = wk.bcount + kExtBins * kRowBuckets;
   wk.fcount = wk.bcursor + kExtBins * kRowBuckets;
@@ -416,7 +427,7 @@ hipError_t launch_glb_gather(const int32_t* score, const int32_t* n_cigar, const
                              bool clear, hipStream_t st);
 constexpr int kGlbGatherWord = kCountSlots;  // its counter, cleared with the call's: cursor[0]
 hipError_t launch_global_impl(GlbArgs a, GlbWork w, int num_cu, hipStream_t st);
-// counters of a CIGAR call: counts, cursor, err[4], fetch, kcount, kcursor
-constexpr int kGlbCounterWords = 2 * kCountSlots + 4 + kFetchSlots + 2 * kGlbKeys;
+// counters of a CIGAR call: counts, cursor, err[4], fetch (one a bin), kcount, kcursor
+constexpr int kGlbCounterWords = 3 * kCountSlots + 4 + 2 * kGlbKeys;
 
 }  // namespace bsx

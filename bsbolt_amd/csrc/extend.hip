@@ -516,7 +516,7 @@ static void launch_group(const ExtKArgs& k, const ExtWork& wk, int B, int64_t n,
   if (blocks < 1) return;
   time_begin(wk, time_of_bin(B), st);
   hipLaunchKernelGGL((ext_plain_kernel<L, C, E1>), dim3((unsigned)blocks), dim3(kExtBlock), 0, st, k,
-                     (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B, wk.fetch + B * kExtSlices);
+                     (const ExtDesc*)wk.desc, (const uint32_t*)wk.counts, B, wk.fetch + group_fetch(B));
   time_end(wk, time_of_bin(B), st);
 }
 

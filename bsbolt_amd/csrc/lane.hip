@@ -66,7 +66,7 @@ ext_lane_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
   for (int b = 0; b < bin; ++b) lbase += counts[b];
   const uint32_t nlist = counts[bin];
   const ExtDesc* __restrict__ desc = desc_all + lbase;
-  uint32_t* __restrict__ fslot = fetch + bin * kExtSlices;
+  uint32_t* __restrict__ fslot = fetch + lane_fetch(bin - kQueryBins);
   const int cs0 = (int)(blockIdx.x % kExtSlices);
   int cs = cs0;
   bool exhausted = nlist == 0;
@@ -241,7 +241,7 @@ ext_lane_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const uint32_t
       }
       if (plo == phi && nlo < nhi) { plo = nlo; phi = nhi; nlo = nhi = 0; }
       if (!apend && !exhausted && nlo == nhi && phi - plo < CH / 2) {
-        aret = atomicAdd(&fslot[cs], lane == 0 ? (uint32_t)CH : 0u);  // branch-free; lane 0's value is read
+        aret = atomicAdd(&fslot[cs * kFetchPad], lane == 0 ? (uint32_t)CH : 0u);  // branch-free; lane 0's value is read
         apend = true;
         acs = cs;
       }
@@ -400,7 +400,7 @@ ext_lane_frame_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const ui
   for (int b = 0; b < cls; ++b) lbase += counts[kExtBins + b];
   const uint32_t nlist = split[cls];  // the class's short-query tasks lead its list
   const ExtDesc* __restrict__ desc = desc_all + lbase;
-  uint32_t* __restrict__ fslot = fetch + (kExtBins + cls) * kExtSlices;
+  uint32_t* __restrict__ fslot = fetch + lane_fetch(kLaneBins + cls);
   const int cs0 = (int)(blockIdx.x % kExtSlices);
   int cs = cs0;
   bool exhausted = nlist == 0;
@@ -581,7 +581,7 @@ ext_lane_frame_kernel(ExtKArgs A, const ExtDesc* __restrict__ desc_all, const ui
       }
       if (plo == phi && nlo < nhi) { plo = nlo; phi = nhi; nlo = nhi = 0; }
       if (!apend && !exhausted && nlo == nhi && phi - plo < CH / 2) {
-        aret = atomicAdd(&fslot[cs], lane == 0 ? (uint32_t)CH : 0u);
+        aret = atomicAdd(&fslot[cs * kFetchPad], lane == 0 ? (uint32_t)CH : 0u);
         apend = true;
         acs = cs;
       }
